@@ -425,6 +425,33 @@ int svbrdf_conv3x3_input_grad(const float *grad_y, const float *y, int activatio
                               int width, const float *packed_t, int cin, float *grad_x, void *workspace,
                               size_t workspace_bytes, void *stream);
 
+/* The same convolutions (same epilogues, gate, results to fp32 rounding) on
+ * the bf16 matrix cores: every fp32 input and weight enters as the exact sum of
+ * three bf16 values and a product as its six leading bf16 products, accumulated
+ * in fp32; the error against 64 bits is below the fp32 matrix instruction's,
+ * and infinities and NaN spread as in svbrdf_conv3x3.  The weights are laid out
+ * once in the matrix core's order: a 16-byte aligned buffer of
+ * svbrdf_conv3x3_split_weights_bytes(cin, cout) bytes (cin and cout exchanged
+ * for the input gradient's), written by svbrdf_conv3x3_pack_split (arguments
+ * as svbrdf_conv3x3_pack) or, from svbrdf_conv3x3_pack's output, by
+ * svbrdf_conv3x3_split_packed (cin, cout: of the convolution that reads it).
+ * svbrdf_conv3x3_split_preferred: whether this path is the faster one for a
+ * shape (more than 8 output channels, at least 32 input channels, 2 GFLOP); it
+ * takes any shape of at least 16 input channels.  Workspace:
+ * svbrdf_conv3x3_split_workspace_bytes, as svbrdf_conv3x3_workspace_bytes. */
+int svbrdf_conv3x3_split_preferred(int n, int cin, int height, int width, int cout);
+size_t svbrdf_conv3x3_split_weights_bytes(int cin, int cout);
+int svbrdf_conv3x3_pack_split(const float *weight, int cout, int cin, const float *style, float scale, int demodulate,
+                              int transpose, void *split, void *stream);
+int svbrdf_conv3x3_split_packed(const float *packed, int cin, int cout, void *split, void *stream);
+size_t svbrdf_conv3x3_split_workspace_bytes(int n, int cin, int height, int width, int cout);
+int svbrdf_conv3x3_split(const float *x, int n, int cin, int height, int width, const void *split, int cout,
+                         const float *bias, const float *noise, float noise_strength, int activation, float *y,
+                         void *workspace, size_t workspace_bytes, void *stream);
+int svbrdf_conv3x3_input_grad_split(const float *grad_y, const float *y, int activation, int n, int cout, int height,
+                                    int width, const void *split_t, int cin, float *grad_x, void *workspace,
+                                    size_t workspace_bytes, void *stream);
+
 /* dL/dw [cout, cin, 3, 3] of a 3x3 convolution (stride 1, zero padding 1)
  * from its input x [n, cin, height, width] and grad_z [n, cout, height,
  * width], the gradient of the loss with respect to the convolution's output

@@ -30,25 +30,65 @@ def _check(t, name):
         raise ValueError(f"{name} must be a float32 CUDA tensor (there is no CPU path), got {t.dtype} on {t.device}")
 
 
-def pack3x3(weight, style=None, scale=1.0, demodulate=False, transpose=False):
-    """[Cout, Cin, 3, 3] -> the kernel's layout ([9, Cin, Cout], or the input-
-    gradient layout [9, Cout, Cin] with flipped taps when transpose), times
-    scale * style[ci] and demodulated per output channel when asked."""
+def _pack_inputs(weight, style):
     w = weight.detach().contiguous()
     _check(w, "weight")
-    cout, cin = int(w.shape[0]), int(w.shape[1])
     if tuple(w.shape[2:]) != (3, 3):
         raise ValueError(f"weight must be [Cout, Cin, 3, 3], got {tuple(w.shape)}")
     st = None
     if style is not None:
         st = style.detach().reshape(-1).contiguous()
         _check(st, "style")
-        if st.numel() != cin:
-            raise ValueError(f"style must have {cin} values, got {st.numel()}")
+        if st.numel() != int(w.shape[1]):
+            raise ValueError(f"style must have {int(w.shape[1])} values, got {st.numel()}")
+    return w, st
+
+
+def pack3x3(weight, style=None, scale=1.0, demodulate=False, transpose=False):
+    """[Cout, Cin, 3, 3] -> the kernel's layout ([9, Cin, Cout], or the input-
+    gradient layout [9, Cout, Cin] with flipped taps when transpose), times
+    scale * style[ci] and demodulated per output channel when asked."""
+    w, st = _pack_inputs(weight, style)
+    cout, cin = int(w.shape[0]), int(w.shape[1])
     out = torch.empty((9, cout, cin) if transpose else (9, cin, cout), dtype=torch.float32, device=w.device)
     _lib.call("svbrdf_conv3x3_pack", _lib.ptr(w), cout, cin, _lib.ptr(st), float(scale), int(bool(demodulate)),
               int(bool(transpose)), _lib.ptr(out), _lib.stream_handle(w.device))
     return out
+
+
+def _takes_split(n, cin, h, w, cout):
+    """Whether a shape runs on the bf16 matrix cores with split operands
+    (fp32 results; csrc/conv_split.hip)."""
+    return bool(_lib.query("svbrdf_conv3x3_split_preferred", n, cin, h, w, cout))
+
+
+def _split_buffer(cin, cout, device):
+    return torch.empty(int(_lib.query("svbrdf_conv3x3_split_weights_bytes", cin, cout)) // 4, dtype=torch.float32,
+                       device=device)
+
+
+def _split_packed(packed, out=None):
+    """Split weights of a convolution from its packed ones ([9, Cin, Cout])."""
+    _, cin, cout = (int(s) for s in packed.shape)
+    packed = packed.contiguous()
+    out = _split_buffer(cin, cout, packed.device) if out is None else out
+    _lib.call("svbrdf_conv3x3_split_packed", _lib.ptr(packed), cin, cout, _lib.ptr(out),
+              _lib.stream_handle(packed.device))
+    return out
+
+
+def _pack_for(n, h, w, weight, style=None, scale=1.0, demodulate=False, transpose=False):
+    """(packed, split) weights for a convolution of n images of h x w: the
+    layout that its path reads, the other None."""
+    cout, cin = int(weight.shape[0]), int(weight.shape[1])
+    k, m = (cout, cin) if transpose else (cin, cout)
+    if not _takes_split(n, k, h, w, m):
+        return pack3x3(weight, style, scale, demodulate, transpose), None
+    wt, st = _pack_inputs(weight, style)
+    out = _split_buffer(k, m, wt.device)
+    _lib.call("svbrdf_conv3x3_pack_split", _lib.ptr(wt), cout, cin, _lib.ptr(st), float(scale), int(bool(demodulate)),
+              int(bool(transpose)), _lib.ptr(out), _lib.stream_handle(wt.device))
+    return None, out
 
 
 def conv3x3_packed(x, packed, cout, bias=None, noise=None, noise_strength=0.0, act="none"):
@@ -58,6 +98,18 @@ def conv3x3_packed(x, packed, cout, bias=None, noise=None, noise_strength=0.0, a
     n, cin, h, w = (int(s) for s in x.shape)
     if tuple(packed.shape) != (9, cin, cout):
         raise ValueError(f"packed weights {tuple(packed.shape)} do not match Cin={cin}, Cout={cout}")
+    split = _split_packed(packed) if _takes_split(n, cin, h, w, cout) else None
+    return _conv3x3(x, packed, split, cin, cout, bias, noise, noise_strength, act)
+
+
+def _conv3x3(x, packed, split, cin, cout, bias=None, noise=None, noise_strength=0.0, act="none"):
+    """conv3x3_packed on the split weights, or on the packed ones where those
+    are None; cin, cout: the weights'."""
+    x = x.contiguous()
+    _check(x, "x")
+    n, channels, h, w = (int(s) for s in x.shape)
+    if channels != cin:
+        raise ValueError(f"x has {channels} channels, the weights Cin={cin}")
     if bias is not None:
         bias = bias.detach().reshape(-1).contiguous()
         _check(bias, "bias")
@@ -69,10 +121,12 @@ def conv3x3_packed(x, packed, cout, bias=None, noise=None, noise_strength=0.0, a
     y = torch.empty((n, cout, h, w), dtype=torch.float32, device=x.device)
     # K-split partial sums of small images (torch's caching allocator makes
     # this a free-list lookup after the first call)
-    ws_bytes = int(_lib.query("svbrdf_conv3x3_workspace_bytes", n, cin, h, w, cout))
+    kind = "svbrdf_conv3x3" if split is None else "svbrdf_conv3x3_split"
+    ws_bytes = int(_lib.query(f"{kind}_workspace_bytes", n, cin, h, w, cout))
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
-    _lib.call("svbrdf_conv3x3", _lib.ptr(x), n, cin, h, w, _lib.ptr(packed), cout, _lib.ptr(bias), _lib.ptr(noise),
-              float(noise_strength), ACT[act], _lib.ptr(y), _lib.ptr(ws), ws_bytes, _lib.stream_handle(x.device))
+    _lib.call(kind, _lib.ptr(x), n, cin, h, w, _lib.ptr(packed if split is None else split), cout, _lib.ptr(bias),
+              _lib.ptr(noise), float(noise_strength), ACT[act], _lib.ptr(y), _lib.ptr(ws), ws_bytes,
+              _lib.stream_handle(x.device))
     return y
 
 
@@ -89,11 +143,23 @@ def conv3x3_input_grad(grad_y, y, packed_t, cin, act):
         raise ValueError(f"y {tuple(y.shape)} and grad_y {tuple(g.shape)} differ")
     if tuple(packed_t.shape) != (9, cout, cin):
         raise ValueError(f"packed weights {tuple(packed_t.shape)} do not match Cout={cout}, Cin={cin}")
+    split_t = _split_packed(packed_t) if _takes_split(n, cout, h, w, cin) else None
+    return _input_grad(g, y, packed_t, split_t, cin, act)
+
+
+def _input_grad(grad_y, y, packed_t, split_t, cin, act):
+    """conv3x3_input_grad on the split weights, or on the packed ones where those are None."""
+    g, y = grad_y.contiguous(), y.contiguous()
+    _check(g, "grad_y")
+    _check(y, "y")
+    n, cout, h, w = (int(s) for s in g.shape)
     gx = torch.empty((n, cin, h, w), dtype=torch.float32, device=g.device)
-    ws_bytes = int(_lib.query("svbrdf_conv3x3_workspace_bytes", n, cout, h, w, cin))
+    kind = "" if split_t is None else "_split"
+    ws_bytes = int(_lib.query(f"svbrdf_conv3x3{kind}_workspace_bytes", n, cout, h, w, cin))
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=g.device) if ws_bytes else None
-    _lib.call("svbrdf_conv3x3_input_grad", _lib.ptr(g), _lib.ptr(y), ACT[act], n, cout, h, w, _lib.ptr(packed_t), cin,
-              _lib.ptr(gx), _lib.ptr(ws), ws_bytes, _lib.stream_handle(g.device))
+    _lib.call(f"svbrdf_conv3x3_input_grad{kind}", _lib.ptr(g), _lib.ptr(y), ACT[act], n, cout, h, w,
+              _lib.ptr(packed_t if split_t is None else split_t), cin, _lib.ptr(gx), _lib.ptr(ws), ws_bytes,
+              _lib.stream_handle(g.device))
     return gx
 
 
@@ -137,8 +203,9 @@ class Conv3x3Function(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, bias, noise, noise_strength, act):
-        packed = pack3x3(weight)
-        y = conv3x3_packed(x, packed, int(weight.shape[0]), bias, noise, noise_strength, act)
+        n, _, h, w = x.shape
+        cout, cin = (int(s) for s in weight.shape[:2])
+        y = _conv3x3(x, *_pack_for(n, h, w, weight), cin, cout, bias, noise, noise_strength, act)
         ctx.save_for_backward(x, weight, noise, y)
         ctx.noise_strength, ctx.act = float(noise_strength), act
         return y
@@ -151,11 +218,13 @@ class Conv3x3Function(torch.autograd.Function):
         if not need_gz:
             # only dL/dx: the gate is applied inside the convolution
             if ctx.needs_input_grad[0]:
-                gx = conv3x3_input_grad(grad_y, y, pack3x3(weight, transpose=True), int(weight.shape[1]), ctx.act)
+                n, _, h, w = y.shape
+                gx = _input_grad(grad_y, y, *_pack_for(n, h, w, weight, transpose=True), int(weight.shape[1]), ctx.act)
             return gx, None, None, None, None, None
         gz = _act_grad(grad_y.contiguous(), y, ctx.act).contiguous()
         if ctx.needs_input_grad[0]:
-            gx = conv3x3_packed(gz, pack3x3(weight, transpose=True), int(weight.shape[1]))
+            n, _, h, w = y.shape
+            gx = _conv3x3(gz, *_pack_for(n, h, w, weight, transpose=True), int(weight.shape[0]), int(weight.shape[1]))
         if ctx.needs_input_grad[1]:
             gw = conv3x3_wgrad(x, gz, int(weight.shape[0]))
         if ctx.needs_input_grad[3] and noise is not None:
@@ -203,8 +272,10 @@ class ModConv3x3Function(torch.autograd.Function):
         if weight.requires_grad:
             raise ValueError("ModConv3x3Function keeps the base weight frozen; use conv3x3 with explicitly "
                              "modulated weights to train it")
-        packed = pack3x3(weight, style, scale, demodulate)
-        y = conv3x3_packed(x, packed, int(weight.shape[0]), bias, noise, noise_strength, act)
+        n, _, h, w = x.shape
+        cout, cin = (int(s) for s in weight.shape[:2])
+        y = _conv3x3(x, *_pack_for(n, h, w, weight, style, scale, demodulate), cin, cout, bias, noise,
+                     noise_strength, act)
         ctx.save_for_backward(x, style, weight, noise, y)
         ctx.scale, ctx.demodulate = float(scale), bool(demodulate)
         ctx.noise_strength, ctx.act = float(noise_strength), act
@@ -218,14 +289,15 @@ class ModConv3x3Function(torch.autograd.Function):
         need_gx, need_gs = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         need_gn = ctx.needs_input_grad[6] and noise is not None
         if need_gx:
-            packed_t = pack3x3(weight, style, ctx.scale, ctx.demodulate, transpose=True)
+            n, _, h, w = y.shape
+            packed_t = _pack_for(n, h, w, weight, style, ctx.scale, ctx.demodulate, transpose=True)
         if not (need_gs or need_gn):
             if need_gx:
-                gx = conv3x3_input_grad(grad_y, y, packed_t, cin, ctx.act)
+                gx = _input_grad(grad_y, y, *packed_t, cin, ctx.act)
             return gx, None, None, None, None, None, None, None, None
         gz = _act_grad(grad_y.contiguous(), y, ctx.act).contiguous()
         if need_gx:
-            gx = conv3x3_packed(gz, packed_t, cin)
+            gx = _conv3x3(gz, *packed_t, int(weight.shape[0]), cin)
         if need_gs:
             gw = conv3x3_wgrad(x, gz, int(weight.shape[0]))
             gstyle = modulation_grad(weight, style, ctx.scale, ctx.demodulate, gw).reshape(style.shape)
@@ -298,7 +370,9 @@ def avgpool2(x):
 class _FrozenConvFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, layer):
-        y = conv3x3_packed(x, layer.packed, layer.cout, layer.bias, None, 0.0, layer.act)
+        n, _, h, w = x.shape
+        split = layer.split if _takes_split(n, layer.cin, h, w, layer.cout) else None   # None below 32 channels
+        y = _conv3x3(x, layer.packed, split, layer.cin, layer.cout, layer.bias, None, 0.0, layer.act)
         ctx.save_for_backward(y)
         ctx.layer = layer
         return y
@@ -307,7 +381,9 @@ class _FrozenConvFunction(torch.autograd.Function):
     def backward(ctx, grad_y):
         (y,) = ctx.saved_tensors
         layer = ctx.layer
-        return conv3x3_input_grad(grad_y, y, layer.packed_t, layer.cin, layer.act), None
+        n, cout, h, w = y.shape
+        split_t = layer.split_t if _takes_split(n, cout, h, w, layer.cin) else None
+        return _input_grad(grad_y, y, layer.packed_t, split_t, layer.cin, layer.act), None
 
 
 class Conv3x3(torch.nn.Module):
@@ -324,6 +400,15 @@ class Conv3x3(torch.nn.Module):
         self.act = act
         self.packed = pack3x3(self.weight)
         self.packed_t = pack3x3(self.weight, transpose=True)
+        # the layout of the bf16 matrix cores beside them, for the sizes that take that path
+        self.split = self.split_t = None
+        if min(self.cin, self.cout) >= 32:
+            # one buffer for both; their sizes are multiples of 64 floats but for the factors' room
+            sizes = [int(_lib.query("svbrdf_conv3x3_split_weights_bytes", *c)) // 256 * 64 + 64
+                     for c in ((self.cin, self.cout), (self.cout, self.cin))]
+            both = torch.empty(sum(sizes), dtype=torch.float32, device=self.weight.device)
+            self.split = _split_packed(self.packed, both[:sizes[0]])
+            self.split_t = _split_packed(self.packed_t, both[sizes[0]:])
 
     def forward(self, x):
         return _FrozenConvFunction.apply(x, self)

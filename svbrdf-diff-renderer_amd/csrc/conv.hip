@@ -50,19 +50,13 @@
 #include <algorithm>
 #include <cstdint>
 
-#include "common.hpp"
-#include "../../include/svbrdf_hip.h"
+#include "conv_common.hpp"
 
-using svbrdf_internal::check_launch;
-using svbrdf_internal::fail;
+using namespace svbrdf_internal;
 
 namespace {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
-
-constexpr int kThreads = 256;   // four waves
-constexpr int kMaxChannels = 4096;
-constexpr int kMaxSide = 8192;
+constexpr int kThreads = kConvThreads;
 
 // ---------------------------------------------------------------------------
 // Weight packing.  The demodulation factor of an output channel is a block
@@ -251,42 +245,10 @@ __global__ __launch_bounds__(kThreads) void modulation_cols_kernel(const float *
 
 // ---------------------------------------------------------------------------
 // The convolution.
-struct ConvArgs {
-    const float *x;       // [N, Cin, H, W]
-    const float *w;       // [9][Cin][Cout]
-    const float *bias;    // [Cout] or null
-    const float *noise;   // [H, W] or null
-    float noise_strength;
-    int act;              // SVBRDF_ACT_*
-    // input gate: x is read as x * (gate > 0 ? gate_pos : gate_neg) where gate
-    // is not null ([N, Cin, H, W], the forward output of the layer whose input
-    // gradient this convolution computes: the activation's derivative)
-    const float *gate;
-    float gate_pos, gate_neg;
-    float *y;             // [N, Cout, H, W]
-    float *part;          // [slices][N, Cout, H, W] partial sums when K is split, else null
-    int n, cin, cout, h, w_;
-    int tw, th, tiles_x;  // pixel tile: th rows x tw columns, tw * th = BN
-    int slices, cps;      // K slices (blockIdx.z = image x slices + slice) of cps chunks each
-};
-
 // LDS floats per staged channel of the input tile: (th + 2) (tw + 2) =
 // BN + 2 (th + tw) + 4 with 4 <= tw <= 32 (so th + tw <= 32 + BN / 4).
 template <int BN>
 constexpr int halo_floats() { return BN + 2 * (32 + BN / 4) + 4; }
-
-__device__ __forceinline__ float activate(float v, int act) {
-    if (act == SVBRDF_ACT_RELU) return v > 0.0f ? v : 0.0f;
-    if (act == SVBRDF_ACT_LRELU) return (v > 0.0f ? v : v * 0.2f) * 1.41421356237309515f;
-    return v;
-}
-
-// the epilogue of output channel co at pixel p: noise, bias, activation
-__device__ __forceinline__ float finish(const ConvArgs &a, float v, int co, size_t p) {
-    if (a.noise) v = v + a.noise_strength * a.noise[p];
-    if (a.bias) v = v + a.bias[co];
-    return activate(v, a.act);
-}
 
 // Block tile BM output channels x BN pixels (th rows x tw columns), four
 // waves of (BM/2) x (BN/2).  K runs over chunks of KC input channels; each
@@ -814,20 +776,11 @@ __global__ __launch_bounds__(kThreads) void upsample2_blur_adjoint_kernel(const 
     gx[e] = acc;
 }
 
-int pick_tile_width(int w) {
-    int tw = 4;
-    while (tw < w && tw < 32) tw *= 2;
-    return tw;
-}
-
 #ifndef SVBRDF_CONV_KC
 #define SVBRDF_CONV_KC 4   // input channels per staged chunk
 #endif
 constexpr int kKC = SVBRDF_CONV_KC;
-constexpr int kDirectMaxCout = 8;          // conv3x3_direct_kernel up to this many output channels
 constexpr int kMinChunksPerSlice = 2;
-constexpr int kMaxSlices = 64;
-constexpr int kComputeUnits = 256;   // MI355X
 
 // How one convolution runs: the tile shape, the tiling of the image and the
 // K split.  The workspace query and the launch share it.
@@ -961,6 +914,31 @@ void launch_mfma(const ConvArgs &a, const ConvPlan &p, hipStream_t s) {
 
 }  // namespace
 
+namespace svbrdf_internal {
+
+void launch_split_sum(const ConvArgs &a, hipStream_t s) {
+    const size_t total = (size_t)a.n * a.cout * a.h * a.w_;
+    hipLaunchKernelGGL(conv_split_sum_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                       s, a);
+}
+
+ConvArgs input_grad_args(const float *grad_y, const float *y, int activation, int n, int cout, int height, int width,
+                         int cin, float *grad_x) {
+    ConvArgs a{};
+    // the convolution of dL/dy (cout channels) with the flipped, transposed
+    // weights, its input gated by the activation's derivative at y
+    a.x = grad_y; a.act = SVBRDF_ACT_NONE; a.y = grad_x;
+    a.n = n; a.cin = cout; a.cout = cin; a.h = height; a.w_ = width;
+    if (activation != SVBRDF_ACT_NONE) {
+        a.gate = y;
+        a.gate_pos = activation == SVBRDF_ACT_LRELU ? 1.41421356237309515f : 1.0f;
+        a.gate_neg = activation == SVBRDF_ACT_LRELU ? 0.2f * 1.41421356237309515f : 0.0f;
+    }
+    return a;
+}
+
+}  // namespace svbrdf_internal
+
 extern "C" {
 
 int svbrdf_conv3x3_pack(const float *weight, int cout, int cin, const float *style, float scale, int demodulate,
@@ -1026,11 +1004,6 @@ int svbrdf_conv3x3_modulation_grad(const float *weight, int cout, int cin, const
     return check_launch(what);
 }
 
-static bool conv_shape_ok(int n, int cin, int height, int width, int cout) {
-    return n >= 1 && n <= 65535 && cin >= 1 && cout >= 1 && cin <= kMaxChannels && cout <= kMaxChannels &&
-           height >= 1 && width >= 1 && height <= kMaxSide && width <= kMaxSide;
-}
-
 size_t svbrdf_conv3x3_workspace_bytes(int n, int cin, int height, int width, int cout) {
     if (!conv_shape_ok(n, cin, height, width, cout)) return 0;
     return plan_conv(n, cin, height, width, cout).part_floats * sizeof(float);
@@ -1066,11 +1039,7 @@ static int run_conv(const char *what, ConvArgs a, void *workspace, size_t worksp
     else if (p.bm == 128) launch_mfma<128, 64>(a, p, s);
     else if (p.bn == 128) launch_mfma<64, 128>(a, p, s);
     else launch_mfma<64, 64>(a, p, s);
-    if (p.slices > 1) {
-        const size_t total = (size_t)a.n * a.cout * a.h * a.w_;
-        hipLaunchKernelGGL(conv_split_sum_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)),
-                           dim3(kThreads), 0, s, a);
-    }
+    if (p.slices > 1) launch_split_sum(a, s);
     return check_launch(what);
 }
 
@@ -1092,16 +1061,8 @@ int svbrdf_conv3x3_input_grad(const float *grad_y, const float *y, int activatio
     if (!grad_y || !y || !packed_t || !grad_x) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
     if (activation < SVBRDF_ACT_NONE || activation > SVBRDF_ACT_LRELU)
         return fail(SVBRDF_EINVAL, "%s: unknown activation %d", what, activation);
-    ConvArgs a{};
-    // the convolution of dL/dy (cout channels) with the flipped, transposed
-    // weights, its input gated by the activation's derivative at y
-    a.x = grad_y; a.w = packed_t; a.act = SVBRDF_ACT_NONE; a.y = grad_x;
-    a.n = n; a.cin = cout; a.cout = cin; a.h = height; a.w_ = width;
-    if (activation != SVBRDF_ACT_NONE) {
-        a.gate = y;
-        a.gate_pos = activation == SVBRDF_ACT_LRELU ? 1.41421356237309515f : 1.0f;
-        a.gate_neg = activation == SVBRDF_ACT_LRELU ? 0.2f * 1.41421356237309515f : 0.0f;
-    }
+    ConvArgs a = input_grad_args(grad_y, y, activation, n, cout, height, width, cin, grad_x);
+    a.w = packed_t;
     return run_conv(what, a, workspace, workspace_bytes, (hipStream_t)stream);
 }
 

@@ -1,0 +1,680 @@
+// conv_split.hip -- the 3x3 convolution of conv.hip (stride 1, zero padding
+// 1, the same epilogues and input gate) at fp32 precision on the bf16 matrix
+// cores.
+//
+// v_mfma_f32_32x32x2f32 runs at 135 TFLOP/s on an MI355X, v_mfma_f32_32x32x16_bf16
+// at 1,970 (both measured from registers).  An fp32 value is the sum of three
+// bf16 values, x = h + m + l: each is the rounding of what the ones before
+// leave, 8 significant bits apiece, 24 in all.  A product is then
+//   x w = hh' + (hm' + mh') + (hl' + mm' + lh') + O(2^-25 |x w|),
+// six bf16 products that the matrix core multiplies exactly and accumulates
+// in fp32, at 1,970 / 6 = 328 TFLOP/s.  bf16 has fp32's exponent, so there is
+// no scaling and no range to check.
+//
+// Precision.  The hh' products and the five small ones have accumulators of
+// their own, so the sum is rounded at its own size once per 16 products (the
+// fp32 instruction: once per product pair).  The bf16 instruction drops what
+// it shifts out of its adder towards minus infinity, a bias that the adjoint
+// of an upsampling adds up coherently; so the weights of every odd chunk are
+// negated and the accumulators with them, and the bias of one chunk cancels
+// the next one's.  Relative error against 64 bits (fp32 instruction / this;
+// normal values, 3 x 3 taps): 64 channels 2.9e-7 / 1.6e-7, 128: 6.1e-7 /
+// 2.0e-7, 256: 8.6e-7 / 2.9e-7, 512 at 64^2: 6.0e-7 (in K slices) / 2.9e-7;
+// with log-normal magnitudes (sigma 3) 5.7e-7 / 2.3e-7.  The mean error is
+// below 2e-10 of sum |x w|.  With one accumulator per sum and no sign
+// change it was 5.2e-7 at 128 channels with a mean of -3e-9, and the W+
+// gradient through the 13 layers of the generator was 3.1e-5 off; it is
+// 1.0e-6, and 1.4e-6 on the fp32 instruction.
+//
+// Infinities and NaN, and finite values that round to infinity in bf16
+// (above 3.39e38), do not split; a wave whose sums come out non-finite
+// repeats its tile from the fp32 inputs on the fp32 instruction
+// (redo_fp32), so they spread exactly as in conv.hip.
+//
+// Kernels
+//   split_factor_kernel   the demodulation factor of each output channel.
+//   split_pack_kernel     weights -> the matrix core's operand order, split:
+//                         [K chunk of 16][tap][h, m, l][32 outputs][lane][8].
+//   conv3x3_split_kernel  the convolution.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
+#include <cstdint>
+#include <type_traits>
+
+#include "conv_common.hpp"
+
+using namespace svbrdf_internal;
+
+namespace {
+
+constexpr int kThreads = kConvThreads;
+constexpr int kKC = 16;   // input channels per chunk: one MFMA's K
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+
+__host__ __device__ constexpr int chunks_of(int k) { return (k + kKC - 1) / kKC; }
+// The first of a chunk's 16 channels.  The last chunk of a K that is no
+// multiple of 16 reaches back: its weights for the channels of the chunk
+// before are zero, so every chunk reads 16 channels that exist.
+__host__ __device__ constexpr int chunk_base(int chunk, int k) { return chunk * kKC + kKC <= k ? chunk * kKC : k - kKC; }
+// groups of 32 output channels; even, so that a wave's 64 channels exist
+__host__ __device__ constexpr int groups_of(int m) { return (m + 63) / 64 * 2; }
+
+__device__ __forceinline__ float bf_lo(unsigned p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float bf_hi(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
+
+// h + m + l of two finite values, as packed bf16 pairs.  No contraction: the
+// value is the rounded product that a caller passes, not the product itself.
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l) {
+#pragma clang fp contract(off)
+    h = __builtin_bit_cast(unsigned, v2bf{(__bf16)a, (__bf16)b});
+    a -= bf_lo(h);
+    b -= bf_hi(h);
+    m = __builtin_bit_cast(unsigned, v2bf{(__bf16)a, (__bf16)b});
+    a -= bf_lo(m);
+    b -= bf_hi(m);
+    l = __builtin_bit_cast(unsigned, v2bf{(__bf16)a, (__bf16)b});
+}
+
+// ---------------------------------------------------------------------------
+// Weights.  The factor of an output channel is the one of conv.hip's packing:
+// the same per-thread order, so the same bits.
+__global__ __launch_bounds__(kThreads) void split_factor_kernel(const float *__restrict__ w, int cin,
+                                                                const float *__restrict__ style, float scale,
+                                                                float *__restrict__ factor) {
+    __shared__ float red[kThreads / 64];
+    const int n = cin * 9;
+    const float *wc = w + (size_t)blockIdx.x * n;
+    float acc = 0.0f;
+    for (int e = threadIdx.x; e < n; e += kThreads) {
+        const float v = wc[e] * scale * (style ? style[e / 9] : 1.0f);
+        acc += v * v;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) factor[blockIdx.x] = rsqrtf(((red[0] + red[1]) + red[2]) + red[3] + 1e-8f);
+}
+
+enum PackForm {
+    kNatural,      // [M, K, 3, 3]
+    kTransposed,   // [K, M, 3, 3], taps flipped: the input gradient's weights
+    kPacked,       // [9][K][M]: svbrdf_conv3x3_pack's output
+};
+
+// One block per 32 outputs and 16-channel chunk: the source rows go to LDS as
+// they lie in memory (runs of 144, 288 or 32 floats), then each thread writes
+// the 16 bytes of a lane's operand for one tap and term: 1 KB per wave and
+// store, contiguous.  A bandwidth-bound pass over 10 bytes per weight.
+template <PackForm FORM>
+__global__ __launch_bounds__(kThreads) void split_pack_kernel(const float *__restrict__ w, int m_total, int k_total,
+                                                              const float *__restrict__ style, float scale,
+                                                              const float *__restrict__ factor,
+                                                              uint4 *__restrict__ out) {
+    constexpr int ROWS = FORM == kNatural ? 32 : FORM == kTransposed ? kKC : 9 * kKC;
+    constexpr int RUN = FORM == kNatural ? kKC * 9 : FORM == kTransposed ? 32 * 9 : 32;
+    constexpr int PITCH = RUN + 1;
+    __shared__ float tile[ROWS * PITCH];
+    const int groups = groups_of(m_total);
+    const int m0 = blockIdx.x * 32, chunk = blockIdx.y;
+    const int k0 = chunk_base(chunk, k_total), skip = chunk * kKC - k0;   // channels of the chunk before
+    for (int e = threadIdx.x; e < ROWS * RUN; e += kThreads) {
+        const int r = e / RUN, c = e - r * RUN;
+        float v = 0.0f;
+        if constexpr (FORM == kNatural) {
+            if (m0 + r < m_total && c / 9 >= skip) v = w[((size_t)(m0 + r) * k_total + k0) * 9 + c];
+        } else if constexpr (FORM == kTransposed) {
+            if (r >= skip && m0 + c / 9 < m_total) v = w[((size_t)(k0 + r) * m_total + m0) * 9 + c];
+        } else {
+            const int t = r / kKC, k = r % kKC;
+            if (k >= skip && m0 + c < m_total) v = w[((size_t)t * k_total + k0 + k) * m_total + m0 + c];
+        }
+        tile[r * PITCH + c] = v;
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < 9 * 64; q += kThreads) {
+        const int t = q / 64, lane = q & 63;
+        const int mm = lane & 31, kk = (lane >> 5) * 8;
+        const int m = min(m0 + mm, m_total - 1);   // padding rows hold zeros
+        uint4 term[3];
+        unsigned *h = &term[0].x, *md = &term[1].x, *l = &term[2].x;
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            float v[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int k = k0 + kk + j + i;
+                if constexpr (FORM == kPacked) {
+                    v[i] = tile[(t * kKC + kk + j + i) * PITCH + mm];
+                } else if constexpr (FORM == kNatural) {
+                    v[i] = tile[mm * PITCH + (kk + j + i) * 9 + t] * scale * (style ? style[k] : 1.0f) *
+                           (factor ? factor[m] : 1.0f);
+                } else {
+                    v[i] = tile[(kk + j + i) * PITCH + mm * 9 + (8 - t)] * scale * (style ? style[m] : 1.0f) *
+                           (factor ? factor[k] : 1.0f);
+                }
+                v[i] = chunk & 1 ? -v[i] : v[i];
+            }
+            split_pair(v[0], v[1], h[j / 2], md[j / 2], l[j / 2]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                // a value whose rounding is infinite: infinities and NaN keep
+                // h alone; a finite one takes the largest bf16 and its rest,
+                // so that h + m + l is the value itself for redo_fp32
+                const unsigned sh = i * 16, keep = 0xffff0000u >> sh;
+                if (((h[j / 2] >> sh) & 0x7f80u) != 0x7f80u) continue;
+                md[j / 2] &= keep;
+                l[j / 2] &= keep;
+                if (fabsf(v[i]) <= FLT_MAX) {
+                    const unsigned top = (__float_as_uint(v[i]) >> 16);   // towards zero: finite
+                    const float rest = v[i] - __uint_as_float(top << 16);
+                    const unsigned mid = __float_as_uint(rest) >> 16;
+                    const unsigned low = __float_as_uint(rest - __uint_as_float(mid << 16)) >> 16;
+                    h[j / 2] = (h[j / 2] & keep) | (top << sh);
+                    md[j / 2] |= mid << sh;
+                    l[j / 2] |= low << sh;
+                }
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+            out[(((size_t)(chunk * 9 + t) * 3 + s) * groups + blockIdx.x) * 64 + lane] = term[s];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The convolution.  Block tile 64 WM output channels x 64 WN pixels (th rows x
+// tw columns), four waves of 64 x 64 (2 x 2 MFMA tiles of 32 x 32).  Per chunk
+// of 16 input channels the block splits its input tile with a one-pixel halo
+// into LDS, in the operand's order: plane (term, half of the 16 channels),
+// then pixel, 16 bytes each, so a lane's operand for a tap is one aligned
+// ds_read_b128 and the lanes of a half-wave read consecutive ones.  The
+// weights come straight from global memory, already in operand order (1 KB
+// per wave and load, L1 / L2 hits: the blocks of an output group walk the
+// same chunks), one tap ahead of their use.  The next chunk's input loads are
+// issued before this chunk's 9 x 24 MFMAs and split into the other LDS buffer
+// beside the last taps' MFMAs, so a block has one short barrier per chunk.
+//
+// Bound by the matrix cores, and those by power: 63 % busy at 1.94 GHz (peak
+// 2.4), where all-register MFMAs reach 1.88.  9 x 64 -> 64 at 256^2: 224 us =
+// 194 TFLOP/s of fp32 products (fp32 instruction 387 us), 256 -> 128 at 256^2:
+// 170 us, 227 TFLOP/s (333 us).  Splitting after the MFMAs instead of beside
+// them: 249 and 189 us; weights loaded where they are used: 310 and 234 us.
+// Three waves per SIMD (168 registers) gain nothing: 227 and 179 us.
+constexpr int halo_pixels(int wn) { return wn == 4 ? 340 : 204; }   // largest (th + 2)(tw + 2), see plan
+
+struct SplitArgs {
+    ConvArgs c;
+    const uint4 *w;   // split_pack_kernel's output
+};
+
+// The fp32 value of a split weight: output m, input channel k, tap t.
+__device__ __forceinline__ float split_weight(const uint4 *w, int groups, int k_total, int m, int k, int t) {
+    const int chunk = k / kKC, kk = k - chunk_base(chunk, k_total);
+    const size_t base = ((size_t)(chunk * 9 + t) * 3 * groups + m / 32) * 64 + (m & 31) + 32 * (kk >> 3);
+    const size_t step = (size_t)groups * 64;
+    float v[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+        v[s] = __uint_as_float((unsigned)reinterpret_cast<const unsigned short *>(w + base + s * step)[kk & 7] << 16);
+    const float x = v[0] + (v[1] + v[2]);
+    return chunk & 1 ? -x : x;
+}
+
+// Element r of MFMA tile (i, j): row 8 (r / 4) + 4 (lane / 32) + r % 4, column
+// lane % 32.  ACT: the activation, or kPartial for a K slice's raw sums.
+constexpr int kPartial = -1;
+template <int ACT>
+__device__ __forceinline__ void store_rows(const ConvArgs &a, float *out, int com, const int (&oy)[2],
+                                           const int (&ox)[2], const v16f (&acc)[2][2]) {
+    const int half = ((threadIdx.x >> 5) & 1) * 4;
+    const size_t HW = (size_t)a.h * a.w_;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (oy[j] >= a.h || ox[j] >= a.w_) continue;
+        const unsigned p = (unsigned)(oy[j] * a.w_ + ox[j]);
+        // the lane's byte offset from a row's first pixel, at most 5 planes
+        const unsigned off = (p + (unsigned)half * (unsigned)HW) * 4u;
+        float nz = 0.0f;
+        if (ACT != kPartial && a.noise) nz = a.noise_strength * a.noise[p];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = com + i * 32 + (r >> 2) * 8 + (r & 3);
+                if (row + half >= a.cout) continue;
+                float v = acc[i][j][r];
+                if constexpr (ACT != kPartial) {
+                    v = v + nz;
+                    if (a.bias) v = v + a.bias[row + half];
+                    v = activate(v, ACT);
+                }
+                *reinterpret_cast<float *>(reinterpret_cast<char *>(out + (size_t)row * HW) + off) = v;
+            }
+    }
+}
+
+__device__ __forceinline__ void store_tile(const ConvArgs &a, int img, int slice, int com, const int (&oy)[2],
+                                           const int (&ox)[2], const v16f (&acc)[2][2]) {
+    const size_t image = (size_t)a.cout * a.h * a.w_;
+    float *y = a.y + img * image;
+    if (a.part) store_rows<kPartial>(a, a.part + ((size_t)slice * a.n + img) * image, com, oy, ox, acc);
+    else if (a.act == SVBRDF_ACT_RELU) store_rows<SVBRDF_ACT_RELU>(a, y, com, oy, ox, acc);
+    else if (a.act == SVBRDF_ACT_LRELU) store_rows<SVBRDF_ACT_LRELU>(a, y, com, oy, ox, acc);
+    else store_rows<SVBRDF_ACT_NONE>(a, y, com, oy, ox, acc);
+}
+
+// A wave's 64 x 64 tile again on the fp32 instruction, from the fp32 inputs:
+// only where the split sums were not finite.
+__device__ __forceinline__ void redo_fp32(const SplitArgs &s, int img, int slice, int com, const int (&oy)[2],
+                                          const int (&ox)[2], v16f (&acc)[2][2]) {
+    const ConvArgs &a = s.c;
+    const int lane = threadIdx.x & 63, groups = groups_of(a.cout);
+    const size_t HW = (size_t)a.h * a.w_;
+    const float *xi = a.x + (size_t)img * a.cin * HW;
+    const float *gi = a.gate ? a.gate + (size_t)img * a.cin * HW : nullptr;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    const int k_end = min((slice + 1) * a.cps * kKC, a.cin);
+#pragma unroll 1
+    for (int k0 = slice * a.cps * kKC; k0 < k_end; k0 += 2) {
+        const int k = k0 + (lane >> 5);
+#pragma unroll 1
+        for (int t = 0; t < 9; ++t) {
+            float av[2], bv[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int m = com + i * 32 + (lane & 31);
+                av[i] = k < k_end && m < a.cout ? split_weight(s.w, groups, a.cin, m, k, t) : 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int y = oy[j] + t / 3 - 1, x = ox[j] + t % 3 - 1;
+                bv[j] = 0.0f;
+                if (k < k_end && y >= 0 && y < a.h && x >= 0 && x < a.w_) {
+                    const size_t o = (size_t)k * HW + (size_t)y * a.w_ + x;
+                    bv[j] = gi ? xi[o] * (gi[o] > 0.0f ? a.gate_pos : a.gate_neg) : xi[o];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+        }
+    }
+}
+
+template <int WM, int WN, bool GATE>
+__global__ __launch_bounds__(kThreads, 2) void conv3x3_split_kernel(SplitArgs s) {
+    static_assert(WM * WN == 4, "four waves");
+    constexpr int HALO = halo_pixels(WN);
+    constexpr int PER = (2 * HALO + kThreads - 1) / kThreads;   // (pixel, channel octet) items per thread
+    __shared__ uint4 tile[2][3][2 * HALO + 1];   // and a slot that items past the last write to
+    const ConvArgs &a = s.c;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave - wm * WN;
+    const int img = blockIdx.z / a.slices, slice = blockIdx.z - img * a.slices;
+    const int groups = groups_of(a.cout);
+    const int com = (blockIdx.y * WM + wm) * 64;                 // the wave's first output channel
+    const int group = min(com / 32, groups - 2);                 // past the end: valid weights, nothing stored
+    const int tyi = blockIdx.x / a.tiles_x, txi = blockIdx.x - tyi * a.tiles_x;
+    const int y0 = tyi * a.th, x0 = txi * a.tw;
+    const int tw2 = a.tw + 2, hs = (a.th + 2) * tw2;
+    const int H = a.h, W = a.w_, HW = H * W;
+    const size_t img_base = (size_t)img * a.cin * HW;
+
+    // This thread's staging items: the byte offset of its pixel in its octet's
+    // first plane (0 and !in: outside the image, read and not used), and where
+    // it goes.  32 bits reach all of a chunk: 16 planes of at most 2^28 bytes.
+    unsigned off[PER];
+    int dst[PER];
+    bool in[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int q = tid + k * kThreads;
+        const int o = q >= hs ? 1 : 0, p = q - o * hs;
+        const int r = p / tw2, c = p - r * tw2;
+        const int yy = y0 - 1 + r, xx = x0 - 1 + c;
+        in[k] = q < 2 * hs && yy >= 0 && yy < H && xx >= 0 && xx < W;
+        off[k] = in[k] ? (o * 8u * (unsigned)HW + (unsigned)(yy * W + xx)) * 4u : 0u;
+        dst[k] = q < 2 * hs ? o * HALO + p : 2 * HALO;
+    }
+    float xr[PER][8];
+    unsigned open[PER];   // bit j: the gate of channel j is positive
+    auto load_chunk = [&](const float *src, int chunk) {
+        const char *xc = reinterpret_cast<const char *>(src + img_base + (size_t)chunk_base(chunk, a.cin) * HW);
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                xr[k][j] = *reinterpret_cast<const float *>(xc + (size_t)j * HW * 4 + off[k]);
+    };
+    // the gate passes through the same registers, a bit per value of it stays
+    auto take_gate = [&]() {
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            open[k] = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) open[k] |= xr[k][j] > 0.0f ? 1u << j : 0u;
+        }
+    };
+    auto store_item = [&](int k, int buf) {
+        uint4 t[3];
+        unsigned *h = &t[0].x, *m = &t[1].x, *l = &t[2].x;
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            float v[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                v[i] = xr[k][j + i];
+                if constexpr (GATE) v[i] = v[i] * (open[k] >> (j + i) & 1 ? a.gate_pos : a.gate_neg);
+                v[i] = in[k] ? v[i] : 0.0f;
+            }
+            split_pair(v[0], v[1], h[j / 2], m[j / 2], l[j / 2]);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) tile[buf][i][dst[k]] = t[i];
+    };
+
+    // the halo-tile pixel each lane feeds to the two MFMA columns of its wave
+    int pix[2], oy[2], ox[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int nn = wn * 64 + j * 32 + (lane & 31);
+        const int ty = nn / a.tw, tx = nn - ty * a.tw;
+        pix[j] = ty * tw2 + tx + (lane >> 5) * HALO;
+        oy[j] = y0 + ty;
+        ox[j] = x0 + tx;
+    }
+    // the h h' products and the five small ones, added at the end: one rounding
+    // at the sum's own size per 16 products
+    v16f acc[2][2], low[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0.0f;
+
+    const int n_chunks = chunks_of(a.cin);
+    const int c_begin = slice * a.cps, c_end = min(n_chunks, c_begin + a.cps);
+    const size_t term_step = (size_t)groups * 64, tap_step = 3 * term_step;
+    // the weights of the next tap to load; the scheduling barriers keep the
+    // loads a whole tap (768 matrix-core cycles) ahead of their use
+    const uint4 *wp = s.w + (size_t)group * 64 + (size_t)c_begin * 9 * tap_step;
+    const uint4 *const w_last = s.w + (size_t)group * 64 + ((size_t)c_end * 9 - 1) * tap_step;
+    v8bf wreg[2][2][3];   // [buffer][MFMA row][term]
+    auto load_weights = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) wreg[b][i][k] = __builtin_bit_cast(v8bf, (wp + k * term_step + i * 64)[lane]);
+        wp = wp < w_last ? wp + tap_step : w_last;
+    };
+    if constexpr (GATE) {
+        load_chunk(a.gate, c_begin);
+        take_gate();
+    }
+    load_chunk(a.x, c_begin);
+    load_weights(0);
+#pragma unroll
+    for (int k = 0; k < PER; ++k) store_item(k, 0);
+    __syncthreads();
+    auto run_chunk = [&](int c, auto last) {
+        constexpr bool LAST = decltype(last)::value;
+        const int buf = (c - c_begin) & 1;
+        const uint4 *T = &tile[buf][0][0];
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            load_weights((t + 1) & 1);
+            if constexpr (!LAST) {
+                if (t == 0) load_chunk(GATE ? a.gate : a.x, c + 1);
+                if (GATE && t == 3) {
+                    take_gate();
+                    load_chunk(a.x, c + 1);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            v8bf xv[2][3];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint4 *p = T + pix[j] + (t / 3) * tw2 + t % 3;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) xv[j][k] = __builtin_bit_cast(v8bf, p[k * (2 * HALO + 1)]);
+            }
+            constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        v16f &d = q < 5 ? low[i][j] : acc[i][j];
+                        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wreg[t & 1][i][TA[q]], xv[j][TB[q]], d, 0, 0, 0);
+                    }
+            // the next chunk's items are split beside the last taps' MFMAs
+            if (!LAST && t + PER >= 9) store_item(t + PER - 9, buf ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (!LAST) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        acc[i][j][r] = -acc[i][j][r];
+                        low[i][j][r] = -low[i][j][r];
+                    }
+            // nine taps: the next chunk's first weights are in the odd buffer
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) wreg[0][i][k] = wreg[1][i][k];
+            __syncthreads();
+        }
+    };
+    for (int c = c_begin; c + 1 < c_end; ++c) run_chunk(c, std::false_type{});
+    run_chunk(c_end - 1, std::true_type{});
+
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] += low[i][j][r];
+                acc[i][j][r] = c_end & 1 ? acc[i][j][r] : -acc[i][j][r];
+                bad |= !(fabsf(acc[i][j][r]) <= FLT_MAX);
+            }
+    if (__any(bad)) redo_fp32(s, img, slice, com, oy, ox, acc);
+    store_tile(a, img, slice, com, oy, ox, acc);
+}
+
+// How a convolution runs: the block tile, the tiling of the image, the K split.
+struct SplitPlan {
+    int wm, wn, tw, th, tiles_x, tiles_y, co_tiles, slices, cps;
+    size_t part_floats;
+};
+
+// Estimated time (us), fitted to a sweep of (block tile, slices) over the layer
+// shapes of the VGG-19 and StyleGAN2 networks on MI355X: a block's chunk takes
+// a compute unit 5.1 us whether one or two blocks share it; the last round of
+// blocks is partly hidden; ~6 us of launch, first loads and last stores; a
+// split adds the sum kernel and its pass over the partial sums.  Its pick was
+// within 6 % of the sweep's best on every shape (e.g. 512 -> 512 at 64 x 64:
+// 2 x 2 waves in 4 slices, 98 us; unsplit 180 us).
+double split_estimate_us(const SplitPlan &p, int n, size_t out_bytes) {
+    const double blocks = (double)p.tiles_x * p.tiles_y * p.co_tiles * n * p.slices;
+    const double rounds = blocks / kComputeUnits, full = std::ceil(rounds);
+    double t = 6.0 + (rounds + 2.0 * full) / 3.0 * (p.cps * (p.wm == 1 ? 5.25 : 5.1) + 0.6);
+    if (p.slices > 1) t += (double)(p.slices + 1) * out_bytes / 8.0e6 + 2.0;
+    return t;
+}
+
+SplitPlan plan_split(int n, int cin, int h, int w, int cout) {
+    SplitPlan best{};
+    const int n_chunks = chunks_of(cin);
+    const size_t out_bytes = (size_t)n * cout * h * w * sizeof(float);
+    const int max_slices = std::max(1, std::min({kMaxSlices, n_chunks, 65535 / n}));
+    double best_t = 0.0;
+    for (int wm = 2; wm >= 1; --wm) {
+        SplitPlan p{};
+        p.wm = wm;
+        p.wn = 4 / wm;
+        p.tw = pick_tile_width(w);
+        // 256-pixel tiles of 4 columns would need a 396-pixel halo tile
+        if (p.wn == 4 && p.tw < 8) continue;
+        p.th = 64 * p.wn / p.tw;
+        p.tiles_x = (w + p.tw - 1) / p.tw;
+        p.tiles_y = (h + p.th - 1) / p.th;
+        p.co_tiles = (cout + 64 * wm - 1) / (64 * wm);
+        for (int s = 1; s <= max_slices; ++s) {
+            p.cps = (n_chunks + s - 1) / s;
+            p.slices = (n_chunks + p.cps - 1) / p.cps;
+            if (p.slices != s) continue;
+            const double t = split_estimate_us(p, n, out_bytes);
+            if (best.wm == 0 || t < 0.98 * best_t) {
+                best = p;
+                best_t = t;
+            }
+        }
+    }
+    best.part_floats = best.slices > 1 ? (size_t)best.slices * n * cout * h * w : 0;
+    return best;
+}
+
+template <int WM, int WN>
+void launch_split(const SplitArgs &s, const SplitPlan &p, hipStream_t st) {
+    const dim3 grid((unsigned)(p.tiles_x * p.tiles_y), (unsigned)p.co_tiles, (unsigned)(s.c.n * p.slices));
+    if (s.c.gate) hipLaunchKernelGGL((conv3x3_split_kernel<WM, WN, true>), grid, dim3(kThreads), 0, st, s);
+    else hipLaunchKernelGGL((conv3x3_split_kernel<WM, WN, false>), grid, dim3(kThreads), 0, st, s);
+}
+
+int run_split(const char *what, ConvArgs a, const void *split, void *workspace, size_t workspace_bytes,
+              hipStream_t st) {
+    if (!conv_shape_ok(a.n, a.cin, a.h, a.w_, a.cout))
+        return fail(SVBRDF_ESHAPE, "%s: n=%d cin=%d cout=%d height=%d width=%d", what, a.n, a.cin, a.cout, a.h, a.w_);
+    if (a.cin < kKC)
+        return fail(SVBRDF_ESHAPE, "%s: %d input channels, the split path takes %d or more", what, a.cin, kKC);
+    if (a.act < SVBRDF_ACT_NONE || a.act > SVBRDF_ACT_LRELU)
+        return fail(SVBRDF_EINVAL, "%s: unknown activation %d", what, a.act);
+    if ((uintptr_t)split & 15u) return fail(SVBRDF_EINVAL, "%s: split weights must be 16-byte aligned", what);
+    const SplitPlan p = plan_split(a.n, a.cin, a.h, a.w_, a.cout);
+    const size_t need = p.part_floats * sizeof(float);
+    if (need && (!workspace || workspace_bytes < need))
+        return fail(SVBRDF_ESPACE, "%s: workspace of %zu bytes, this shape needs %zu "
+                    "(svbrdf_conv3x3_split_workspace_bytes)", what, workspace ? workspace_bytes : (size_t)0, need);
+    a.part = p.slices > 1 ? (float *)workspace : nullptr;
+    a.tw = p.tw; a.th = p.th; a.tiles_x = p.tiles_x; a.slices = p.slices; a.cps = p.cps;
+    const SplitArgs s{a, (const uint4 *)split};
+    if (p.wm == 1) launch_split<1, 4>(s, p, st);
+    else launch_split<2, 2>(s, p, st);
+    if (p.slices > 1) launch_split_sum(a, st);
+    return check_launch(what);
+}
+
+size_t split_floats(int k, int m) { return (size_t)chunks_of(k) * 9 * 3 * groups_of(m) * 64 * 4; }
+
+}  // namespace
+
+extern "C" {
+
+// Where this path is taken.  Below ~2 GFLOP a call is bound by its launches
+// and first loads, not the matrix cores, and the fp32 kernel's finer chunks
+// win (graph-timed, fp32 / split without the weights' 6-8 us: 64 -> 64 at 64^2
+// 12.5 / 14.1 us, 128 -> 128 at 32^2 13.1 / 15.1, 512 -> 512 at 16^2 25.5 /
+// 22.6; above it 512 -> 512 at 32^2 64.7 / 34.9, 512 -> 512 at 64^2 189 / 98,
+// 9 x 64 -> 64 at 256^2 387 / 224).  With fewer than 32 input channels the
+// 16-channel chunks are mostly padding, and the short sums are no more exact
+// than fp32's.
+int svbrdf_conv3x3_split_preferred(int n, int cin, int height, int width, int cout) {
+    if (!conv_shape_ok(n, cin, height, width, cout)) return 0;
+    return cout > kDirectMaxCout && cin >= 32 && 18.0 * n * cin * cout * height * width >= 2.0e9;
+}
+
+size_t svbrdf_conv3x3_split_weights_bytes(int cin, int cout) {
+    if (cin < 1 || cout < 1 || cin > kMaxChannels || cout > kMaxChannels) return 0;
+    // the split weights, then room for a demodulation factor per channel of either side
+    return (split_floats(cin, cout) + std::max(cin, cout)) * sizeof(float);
+}
+
+int svbrdf_conv3x3_pack_split(const float *weight, int cout, int cin, const float *style, float scale, int demodulate,
+                              int transpose, void *split, void *stream) {
+    const char *what = "svbrdf_conv3x3_pack_split";
+    if (!weight || !split) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    if (cout < 1 || cin < 1 || cout > kMaxChannels || cin > kMaxChannels)
+        return fail(SVBRDF_ESHAPE, "%s: cout=%d cin=%d outside [1, %d]", what, cout, cin, kMaxChannels);
+    if ((uintptr_t)split & 15u) return fail(SVBRDF_EINVAL, "%s: split weights must be 16-byte aligned", what);
+    hipStream_t s = (hipStream_t)stream;
+    const int m = transpose ? cin : cout, k = transpose ? cout : cin;
+    if (k < kKC) return fail(SVBRDF_ESHAPE, "%s: %d input channels, the split path takes %d or more", what, k, kKC);
+    float *factor = nullptr;
+    if (demodulate) {
+        factor = (float *)split + split_floats(k, m);
+        hipLaunchKernelGGL(split_factor_kernel, dim3((unsigned)cout), dim3(kThreads), 0, s, weight, cin, style, scale,
+                           factor);
+        if (int rc = check_launch(what)) return rc;
+    }
+    const dim3 grid((unsigned)groups_of(m), (unsigned)chunks_of(k));
+    if (transpose)
+        hipLaunchKernelGGL(split_pack_kernel<kTransposed>, grid, dim3(kThreads), 0, s, weight, m, k, style, scale,
+                           (const float *)factor, (uint4 *)split);
+    else
+        hipLaunchKernelGGL(split_pack_kernel<kNatural>, grid, dim3(kThreads), 0, s, weight, m, k, style, scale,
+                           (const float *)factor, (uint4 *)split);
+    return check_launch(what);
+}
+
+int svbrdf_conv3x3_split_packed(const float *packed, int cin, int cout, void *split, void *stream) {
+    const char *what = "svbrdf_conv3x3_split_packed";
+    if (!packed || !split) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    if (cout < 1 || cin < 1 || cout > kMaxChannels || cin > kMaxChannels)
+        return fail(SVBRDF_ESHAPE, "%s: cout=%d cin=%d outside [1, %d]", what, cout, cin, kMaxChannels);
+    if ((uintptr_t)split & 15u) return fail(SVBRDF_EINVAL, "%s: split weights must be 16-byte aligned", what);
+    if (cin < kKC) return fail(SVBRDF_ESHAPE, "%s: %d input channels, the split path takes %d or more", what, cin, kKC);
+    const dim3 grid((unsigned)groups_of(cout), (unsigned)chunks_of(cin));
+    hipLaunchKernelGGL(split_pack_kernel<kPacked>, grid, dim3(kThreads), 0, (hipStream_t)stream, packed, cout, cin,
+                       (const float *)nullptr, 1.0f, (const float *)nullptr, (uint4 *)split);
+    return check_launch(what);
+}
+
+size_t svbrdf_conv3x3_split_workspace_bytes(int n, int cin, int height, int width, int cout) {
+    if (!conv_shape_ok(n, cin, height, width, cout) || cin < kKC) return 0;
+    return plan_split(n, cin, height, width, cout).part_floats * sizeof(float);
+}
+
+int svbrdf_conv3x3_split(const float *x, int n, int cin, int height, int width, const void *split, int cout,
+                         const float *bias, const float *noise, float noise_strength, int activation, float *y,
+                         void *workspace, size_t workspace_bytes, void *stream) {
+    const char *what = "svbrdf_conv3x3_split";
+    if (!x || !split || !y) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    ConvArgs a{};
+    a.x = x; a.bias = bias; a.noise = noise; a.noise_strength = noise_strength; a.act = activation;
+    a.y = y; a.n = n; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
+    return run_split(what, a, split, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int svbrdf_conv3x3_input_grad_split(const float *grad_y, const float *y, int activation, int n, int cout, int height,
+                                    int width, const void *split_t, int cin, float *grad_x, void *workspace,
+                                    size_t workspace_bytes, void *stream) {
+    const char *what = "svbrdf_conv3x3_input_grad_split";
+    if (!grad_y || !y || !split_t || !grad_x) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    if (activation < SVBRDF_ACT_NONE || activation > SVBRDF_ACT_LRELU)
+        return fail(SVBRDF_EINVAL, "%s: unknown activation %d", what, activation);
+    const ConvArgs a = input_grad_args(grad_y, y, activation, n, cout, height, width, cin, grad_x);
+    return run_split(what, a, split_t, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+}  // extern "C"
