@@ -218,6 +218,13 @@ int svbrdf_fused_step_flush(void *state, int res, int n_views, float *loss_histo
 int svbrdf_resize_lanczos4_u8(const unsigned char *src, int src_h, int src_w, int channels,
                               unsigned char *dst, int dst_h, int dst_w, void *stream);
 
+/* The stage transition through 8-bit maps for an upscale (dst_res > res), in
+ * one pass: what svbrdf_textures_to_u8, svbrdf_resize_lanczos4_u8 of each map
+ * and svbrdf_textures_from_u8 give, bit for bit (save_textures_th then
+ * load_textures_th, src/svbrdf.py:150-189).  textures [9, res, res] ->
+ * out [9, dst_res, dst_res], dense and not overlapping. */
+int svbrdf_reload_textures(const float *textures, int res, float *out, int dst_res, void *stream);
+
 /* Coarse-to-fine stage chaining in memory: the reference chains stages
  * through 8-bit PNG files and a Lanczos-4 resize (src/scripts.py:83-85,
  * src/svbrdf.py:150-166, src/imageio.py:75-76; svbrdf_resize_lanczos4_u8

@@ -9,6 +9,7 @@
 // the host; every per-pixel step is here.
 //
 // Kernels (byte and float elementwise work, HBM-bound):
+//   reload_textures_kernel  maps -> 8 bits -> resize -> maps, fused (an upscale)
 //   resize_lanczos4_kernel  8-bit Lanczos-4 resample, 8x8 taps, integer-exact
 //   images_from_u8_kernel   [n, h, w, C] u8 -> [n, C', h, w] f32   C B read, 4 C' B written / px
 //   textures_from_u8_kernel 4 maps u8 -> [9, R, R] f32             10-12 B read, 36 B written / px
@@ -91,31 +92,33 @@ __device__ __forceinline__ void lanczos4_taps(float x, float (&w)[8]) {
     }
 }
 
-// The tile's 16 column and 16 row plans, one plan per thread of the first 32:
-// float weights, their sequential float sum and its reciprocal, then the
-// rounded 11-bit weights.
+// The plan of destination index d: float weights, their sequential float sum
+// and its reciprocal, then the rounded 11-bit weights.
+__device__ __forceinline__ void axis_plan(int d, int n_src, int n_dst, AxisPlan &plan) {
+    int first = 0;
+    float frac = 0.0f;
+    source_coord(d, n_src, n_dst, first, frac);
+    float w[8];
+    lanczos4_taps(frac, w);
+    float total = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) total = total + w[k];
+    const float inv = 1.0f / total;
+    plan.first = first;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float v = rintf((w[i] * inv) * (float)(1 << kCoefBits));
+        plan.w[i] = (int)fminf(fmaxf(v, -32768.0f), 32767.0f);
+    }
+}
+
+// The tile's 16 column and 16 row plans, one plan per thread of the first 32.
 __device__ void tile_plans(int x0, int y0, int sh, int sw, int dh, int dw, AxisPlan *plans) {
     const int plan = threadIdx.x;
     if (plan < kPlans) {
         const bool is_x = plan < kTile;
         const int d = is_x ? x0 + plan : y0 + plan - kTile;
-        if (d < (is_x ? dw : dh)) {
-            int first = 0;
-            float frac = 0.0f;
-            source_coord(d, is_x ? sw : sh, is_x ? dw : dh, first, frac);
-            float w[8];
-            lanczos4_taps(frac, w);
-            float total = 0.0f;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) total = total + w[k];
-            const float inv = 1.0f / total;
-            plans[plan].first = first;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float v = rintf((w[i] * inv) * (float)(1 << kCoefBits));
-                plans[plan].w[i] = (int)fminf(fmaxf(v, -32768.0f), 32767.0f);
-            }
-        }
+        if (d < (is_x ? dw : dh)) axis_plan(d, is_x ? sw : sh, is_x ? dw : dh, plans[plan]);
     }
     __syncthreads();
 }
@@ -485,6 +488,111 @@ __global__ __launch_bounds__(kBlock) void images_to_u8_x4_kernel(const float *__
     store_px4(out, g, b);
 }
 
+// ---------------------------------------------------------------------------
+// The stage transition in one pass: textures_to_u8, the Lanczos-4 resize of
+// the four maps and textures_from_u8 for an upscale of square maps, the same
+// arithmetic per value and so the same bits, without the maps' trips through
+// memory.  A block owns T x T output texels: it quantises the source texels
+// they need into LDS (12 bytes each: diffuse, normal, specular, roughness),
+// takes the horizontal 8-tap sums of those rows and the vertical ones of the
+// result, and decodes.  The plans (double-precision sine and cosine) are one
+// wave's work while the others quantise; u / 255 * 2 - 1 comes from a table of
+// the 256 quotients.  Bound by its integer and conversion arithmetic: 512^2 ->
+// 1024^2 takes 23 us (47 MB, 6 us at 8 TB/s; 24 with 256 threads for the 32-texel
+// tile, whose 4 blocks then half fill a compute unit); the six launches it
+// replaces took 67 (12 of them between kernels).
+constexpr int kMapBytes = 12;
+constexpr int kMapChannels = 10;
+
+template <int T, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void reload_textures_kernel(const float *__restrict__ tex, int src, int span,
+                                                                 float *__restrict__ out, int dst) {
+    __shared__ AxisPlan plans[2 * T];
+    __shared__ float table[256];
+    extern __shared__ uint32_t dynamic[];
+    uint32_t *texel = dynamic;                                              // [span][span][3]
+    int *hsum = reinterpret_cast<int *>(dynamic + 3 * span * span);         // [span][T][kMapChannels]
+    const int x0 = blockIdx.x * T, y0 = blockIdx.y * T;
+    const int cols = min(T, dst - x0), rows = min(T, dst - y0);
+    const size_t n_src = (size_t)src * src, n_dst = (size_t)dst * dst;
+    int c0, r0, c1, r1;
+    float unused;
+    source_coord(x0, src, dst, c0, unused);
+    source_coord(y0, src, dst, r0, unused);
+    source_coord(x0 + cols - 1, src, dst, c1, unused);
+    source_coord(y0 + rows - 1, src, dst, r1, unused);
+    const int nc = c1 + 8 - c0, nr = r1 + 8 - r0;                           // at most span
+    if (threadIdx.x < 256) table[threadIdx.x] = unit((uint8_t)threadIdx.x) * 2.0f - 1.0f;
+    constexpr int kQuantise = BLOCK - 64;
+    if (threadIdx.x >= kQuantise) {
+        const int plan = threadIdx.x - kQuantise;
+        if (plan < 2 * T) {
+            const int d = plan < T ? x0 + plan : y0 + plan - T;
+            if (d < dst) axis_plan(d, src, dst, plans[plan]);
+        }
+    } else {
+        for (int e = threadIdx.x; e < nc * nr; e += kQuantise) {
+            const int r = e / nc, c = e - r * nc;
+            const size_t p = (size_t)min(max(r0 + r, 0), src - 1) * src + min(max(c0 + c, 0), src - 1);
+            float t[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) t[k] = tex[k * n_src + p];
+            uint8_t d[3], n[3], s[3], g;
+            texel_to_u8(t, d, n, s, g);
+            uint32_t *q = texel + 3 * (r * nc + c);
+            q[0] = d[0] | (uint32_t)d[1] << 8 | (uint32_t)d[2] << 16 | (uint32_t)n[0] << 24;
+            q[1] = n[1] | (uint32_t)n[2] << 8 | (uint32_t)s[0] << 16 | (uint32_t)s[1] << 24;
+            q[2] = s[2] | (uint32_t)g << 8;
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < nr * T; e += BLOCK) {
+        const int r = e / T, x = e % T;
+        if (x >= cols) continue;
+        const AxisPlan &ax = plans[x];
+        const uint32_t *q = texel + 3 * (r * nc + ax.first - c0);
+        int h[kMapChannels];
+#pragma unroll
+        for (int c = 0; c < kMapChannels; ++c) h[c] = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int w = ax.w[j];
+#pragma unroll
+            for (int c = 0; c < kMapChannels; ++c)
+                h[c] += __mul24((int)(q[3 * j + c / 4] >> (8 * (c % 4)) & 0xffu), w);
+        }
+        int *o = hsum + e * kMapChannels;
+#pragma unroll
+        for (int c = 0; c < kMapChannels; ++c) o[c] = h[c];
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < rows * T; e += BLOCK) {
+        const int y = e / T, x = e % T;
+        if (x >= cols) continue;
+        const AxisPlan &ay = plans[T + y];
+        int acc[kMapChannels];
+#pragma unroll
+        for (int c = 0; c < kMapChannels; ++c) acc[c] = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int *h = hsum + ((ay.first + k - r0) * T + x) * kMapChannels;
+            const int w = ay.w[k];
+            // |h| < 2^21: a row of eight 11-bit weights sums to less than 2^13 in magnitude
+#pragma unroll
+            for (int c = 0; c < kMapChannels; ++c) acc[c] += __mul24(h[c], w);
+        }
+        float v[kMapChannels];
+#pragma unroll
+        for (int c = 0; c < kMapChannels; ++c) v[c] = table[finish(acc[c])];
+        // decode_normal: divided by the 2-norm
+        const float norm = sqrtf((v[3] * v[3] + v[4] * v[4]) + v[5] * v[5]);
+        const float texels[9] = {v[0], v[1], v[2], v[3] / norm, v[4] / norm, v[9], v[6], v[7], v[8]};
+        float *o = out + (size_t)(y0 + y) * dst + x0 + x;
+#pragma unroll
+        for (int c = 0; c < 9; ++c) __builtin_nontemporal_store(texels[c], o + c * n_dst);
+    }
+}
+
 // x2 bilinear upsample of n_planes planes, as torch's upsample_bilinear2d with
 // align_corners=False and scale_factor=2 computes it: source coordinate
 // max(0.5 (d + 0.5) - 0.5, 0) in float, its integer part and fraction as the
@@ -637,6 +745,40 @@ int svbrdf_resize_lanczos4_u8(const unsigned char *src, int src_h, int src_w, in
         case 3: hipLaunchKernelGGL(resize_lanczos4_kernel<3>, grid, dim3(kBlock), 0, s, src, src_h, src_w, dst, dst_h, dst_w); break;
         default: hipLaunchKernelGGL(resize_lanczos4_kernel<4>, grid, dim3(kBlock), 0, s, src, src_h, src_w, dst, dst_h, dst_w); break;
     }
+    return check_launch(what);
+}
+
+int svbrdf_reload_textures(const float *textures, int res, float *out, int dst_res, void *stream) {
+    const char *what = "svbrdf_reload_textures";
+    if (!textures || !out) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    if (res < 1 || dst_res > kMaxRes || dst_res <= res)
+        return fail(SVBRDF_ESHAPE, "%s: %d -> %d is no upscale to at most %d", what, res, dst_res, kMaxRes);
+    const uintptr_t s0 = (uintptr_t)textures, s1 = s0 + (size_t)9 * res * res * sizeof(float);
+    const uintptr_t d0 = (uintptr_t)out, d1 = d0 + (size_t)9 * dst_res * dst_res * sizeof(float);
+    if (s0 < d1 && d0 < s1) return fail(SVBRDF_EINVAL, "%s: source and destination overlap", what);
+    // Source texels along a tile's side: the rounded-down coordinates of its
+    // last and first texel are at most (tile - 1) scale + 2 apart (a float's
+    // rounding can carry one over an integer), then 8 taps.
+    const auto span_of = [&](int tile) { return (int)((tile - 1) * ((double)res / dst_res)) + 2 + 8; };
+    const auto lds_of = [&](int tile) {
+        const size_t span = span_of(tile);
+        return (3 * span * span + span * tile * kMapChannels) * sizeof(uint32_t);
+    };
+    // 32 x 32 tiles read each source texel least often; 16 x 16 where those
+    // would leave compute units without a block, or need over 60 KB of LDS
+    // (a scale near 1)
+    const long long wide = (dst_res + 31) / 32;
+    const int tile = wide * wide >= 512 && lds_of(32) <= 60 * 1024 ? 32 : 16;
+    const int span = span_of(tile);
+    const size_t lds = lds_of(tile);
+    const unsigned n = (unsigned)((dst_res + tile - 1) / tile);
+    hipStream_t s = (hipStream_t)stream;
+    if (tile == 32)
+        hipLaunchKernelGGL((reload_textures_kernel<32, 512>), dim3(n, n), dim3(512), lds, s, textures, res, span, out,
+                           dst_res);
+    else
+        hipLaunchKernelGGL((reload_textures_kernel<16, 256>), dim3(n, n), dim3(256), lds, s, textures, res, span, out,
+                           dst_res);
     return check_launch(what);
 }
 

@@ -91,6 +91,13 @@ def maps_u8_from_textures(textures):
 def reload_textures(textures, res):
     """save_textures_th then load_textures_th(res), in device memory: 8-bit
     quantisation of the maps, Lanczos-4 resize to res, decode."""
+    if isinstance(res, int) and textures.shape[-1] == textures.shape[-2] < res and textures.device.type == "cuda":
+        # an upscale: the three steps as one kernel, the same bits
+        src = textures.detach().to(torch.float32).reshape(9, *textures.shape[-2:]).contiguous()
+        out = torch.empty((1, 9, res, res), dtype=torch.float32, device=src.device)
+        _lib.call("svbrdf_reload_textures", _lib.ptr(src), src.shape[-1], _lib.ptr(out), res,
+                  _lib.stream_handle(src.device))
+        return out
     dif, nom, spe, rgh = maps_u8_from_textures(textures)
     return textures_from_maps_u8(dif, nom, spe, rgh, res)
 
