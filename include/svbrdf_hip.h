@@ -195,6 +195,15 @@ int svbrdf_fused_step(float *textures, float *exp_avg, float *exp_avg_sq,
                       int history_len, void *workspace, size_t workspace_bytes,
                       void *stream);
 
+/* n_steps iterations of svbrdf_fused_step, launched one after the other (the
+ * loop of src/svbrdf.py:57-71 without its side outputs); stops at the first
+ * failing one. */
+int svbrdf_fused_steps(int n_steps, float *textures, float *exp_avg, float *exp_avg_sq, const float *targets_prepared,
+                       int res, size_t texture_stride, size_t plane_stride, int n_views, float size,
+                       const float *camera_pos, const float *light_pos, float *light_pow, int loss_mode,
+                       int optim_light, double lr, double beta1, double beta2, double eps, void *state,
+                       float *loss_history, int history_len, void *workspace, size_t workspace_bytes, void *stream);
+
 /* Records the loss of the last step taken by svbrdf_fused_step when it is
  * still pending (no-op otherwise): state->loss and loss_history[t - 1].
  * Call it before reading losses on the host (no counterpart in the

@@ -58,6 +58,10 @@ SIGNATURES = {
                                          _vp, ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.c_double,
                                          ctypes.c_double, ctypes.c_double, _vp, _vp, ctypes.c_int, _vp,
                                          ctypes.c_size_t, _vp]),
+    "svbrdf_fused_steps": (ctypes.c_int, [ctypes.c_int, _vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_size_t,
+                                          ctypes.c_size_t, ctypes.c_int, ctypes.c_float, _vp, _vp, _vp, ctypes.c_int,
+                                          ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                                          ctypes.c_double, _vp, _vp, ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
     # batched step (svbrdf_material tables are passed as pointers)
     "svbrdf_fused_step_flush": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, _vp, ctypes.c_int, _vp,
                                                ctypes.c_size_t, _vp]),
@@ -150,17 +154,16 @@ def load():
 
 def call(name, *args):
     """Calls an int-returning entry point and raises on a non-zero status."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != OK:
-        msg = lib.svbrdf_last_error().decode(errors="replace")
+        msg = load().svbrdf_last_error().decode(errors="replace")
         if rc in (EINVAL, ESHAPE, ESPACE):
             raise ValueError(f"{name}: {msg}")
         raise SvbrdfHipError(name, rc, msg)
 
 
 def query(name, *args):
-    return getattr(load(), name)(*args)
+    return getattr(_lib or load(), name)(*args)
 
 
 def ptr(t):
@@ -182,4 +185,10 @@ def cuda_device(device, what="svbrdf_amd"):
 
 
 def stream_handle(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream's handle (hipStream_t).  With an indexed device the
+    raw handle is read directly, without building a torch Stream object: 0.2
+    against 2.1 us of a ~7 us call."""
+    index = getattr(device, "index", None)
+    if index is None or not torch.cuda.is_initialized():
+        return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(index))

@@ -501,7 +501,6 @@ __global__ __launch_bounds__(kBlock) void images_to_u8_x4_kernel(const float *__
 // 1024^2 takes 23 us (47 MB, 6 us at 8 TB/s; 24 with 256 threads for the 32-texel
 // tile, whose 4 blocks then half fill a compute unit); the six launches it
 // replaces took 67 (12 of them between kernels).
-constexpr int kMapBytes = 12;
 constexpr int kMapChannels = 10;
 
 template <int T, int BLOCK>

@@ -1466,6 +1466,21 @@ int svbrdf_fused_step(float *textures, float *exp_avg, float *exp_avg_sq, const 
     return check_launch("svbrdf_fused_step");
 }
 
+int svbrdf_fused_steps(int n_steps, float *textures, float *exp_avg, float *exp_avg_sq, const float *targets_prepared,
+                       int res, size_t texture_stride, size_t plane_stride, int n_views, float size,
+                       const float *camera_pos, const float *light_pos, float *light_pow, int loss_mode,
+                       int optim_light, double lr, double beta1, double beta2, double eps, void *state,
+                       float *loss_history, int history_len, void *workspace, size_t workspace_bytes, void *stream) {
+    if (n_steps < 0) return fail(SVBRDF_EINVAL, "svbrdf_fused_steps: n_steps=%d", n_steps);
+    for (int k = 0; k < n_steps; ++k)
+        if (int rc = svbrdf_fused_step(textures, exp_avg, exp_avg_sq, targets_prepared, res, texture_stride,
+                                       plane_stride, n_views, size, camera_pos, light_pos, light_pow, loss_mode,
+                                       optim_light, lr, beta1, beta2, eps, state, loss_history, history_len, workspace,
+                                       workspace_bytes, stream))
+            return rc;
+    return SVBRDF_OK;
+}
+
 int svbrdf_fused_step_flush(void *state, int res, int n_views, float *loss_history, int history_len,
                             const void *workspace, size_t workspace_bytes, void *stream) {
     if (!state || !workspace) return fail(SVBRDF_EINVAL, "svbrdf_fused_step_flush: null pointer argument");
