@@ -32,7 +32,7 @@
 //                         thread, all output channels in registers, on the
 //                         vector ALUs -- an MFMA tile of 64 output channels
 //                         would be mostly padding.
-//   upsample2_blur_kernel x2 upsampling by zero insertion and the [1, 3, 3, 1]
+//   upsample2_blur*_kernel x2 upsampling by zero insertion and the [1, 3, 3, 1]
 //                         binomial filter (gain 4): out(2p) = (x(p-1) + 3 x(p))/4,
 //                         out(2p+1) = (3 x(p) + x(p+1))/4 per axis, zero outside
 //                         the image; and its adjoint.
@@ -424,18 +424,35 @@ __global__ __launch_bounds__(kThreads) void conv3x3_mfma_kernel(ConvArgs a) {
     }
 }
 
-// Sum of the K slices' partial sums, in slice order, and the epilogue; one
-// output element per thread.
+// Sum of the K slices' partial sums, in slice order, and the epilogue; VEC
+// consecutive pixels of one channel per thread (4: H W a multiple of 4 and
+// 16-byte aligned pointers).  A memory-bound pass over slices + 1 copies of the
+// output: 3 slices of 9 x 256 -> 512 at 32^2 (75 MB) take
+// 16.2 us, 19.6 one by one.
+template <int VEC>
 __global__ __launch_bounds__(kThreads) void conv_split_sum_kernel(ConvArgs a) {
-    const size_t HW = (size_t)a.h * a.w_;
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const unsigned HW = (unsigned)a.h * (unsigned)a.w_;
     const size_t total = (size_t)a.n * a.cout * HW;
-    const size_t e = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    const size_t e = ((size_t)blockIdx.x * kThreads + threadIdx.x) * VEC;
     if (e >= total) return;
-    float v = a.part[e];
-    for (int s = 1; s < a.slices; ++s) v += a.part[(size_t)s * total + e];
-    const size_t p = e % HW;
-    const int co = (int)((e / HW) % a.cout);
-    a.y[e] = finish(a, v, co, p);
+    const auto slice = [&](int s) { return *reinterpret_cast<const vec *>(a.part + (size_t)s * total + e); };
+    vec v = slice(0);
+    int s = 1;
+    for (; s + 4 <= a.slices; s += 4) {   // four loads in flight
+        const vec p0 = slice(s), p1 = slice(s + 1), p2 = slice(s + 2), p3 = slice(s + 3);
+        v += p0;
+        v += p1;
+        v += p2;
+        v += p3;
+    }
+    for (; s < a.slices; ++s) v += slice(s);
+    const size_t plane = e / HW;
+    const unsigned p = (unsigned)(e - plane * HW);
+    const int co = (int)(plane % (unsigned)a.cout);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) v[i] = finish(a, v[i], co, p + i);
+    *reinterpret_cast<vec *>(a.y + e) = v;
 }
 
 // Direct convolution for Cout = CO <= 8: a 64 x 8 pixel block, two
@@ -747,6 +764,53 @@ __global__ __launch_bounds__(kThreads) void upsample2_blur_kernel(const float *_
     y[e] = wr0 * h0 + wr1 * h1;
 }
 
+// The same for an even width and 16-byte aligned output: input columns 2j and
+// 2j + 1 of kUpStrip rows per thread, so 2 kUpStrip float4 rows of the output
+// from kUpStrip + 2 input rows of four values, instead of four loads for each
+// output.  Bound by the output's bytes: 256 planes of 128^2 (84 MB) take
+// 17.3 us, 48.3 with an output per thread, which stays for odd widths and for
+// outputs of under 2^18 values, where it has the more threads (512 planes of
+// 4^2: 2.0 against 2.8 us).
+constexpr int kUpStrip = 2;
+
+__global__ __launch_bounds__(kThreads) void upsample2_blur_rows_kernel(const float *__restrict__ x, int planes, int h,
+                                                                       int w, float *__restrict__ y) {
+    const int half = w / 2, strips = (h + kUpStrip - 1) / kUpStrip;
+    const size_t e = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (e >= (size_t)planes * strips * half) return;
+    const int j = (int)(e % half), strip = (int)((e / half) % strips);
+    const size_t pl = e / ((size_t)half * strips);
+    const int p0 = strip * kUpStrip, c = 2 * j;
+    const float *s = x + pl * (size_t)h * w;
+    float f[kUpStrip + 2][4];   // the rows' outputs along the columns
+#pragma unroll
+    for (int r = 0; r < kUpStrip + 2; ++r) {
+        const int p = p0 - 1 + r;
+        const bool in = p >= 0 && p < h;
+        const float *row = s + (size_t)(in ? p : 0) * w;
+        const float2 mid = *reinterpret_cast<const float2 *>(row + c);
+        const float a = c > 0 ? row[c - 1] : 0.0f, d = c + 2 < w ? row[c + 2] : 0.0f;
+        f[r][0] = in ? 0.25f * a + 0.75f * mid.x : 0.0f;
+        f[r][1] = in ? 0.75f * mid.x + 0.25f * mid.y : 0.0f;
+        f[r][2] = in ? 0.25f * mid.x + 0.75f * mid.y : 0.0f;
+        f[r][3] = in ? 0.75f * mid.y + 0.25f * d : 0.0f;
+    }
+    float *o = y + pl * (size_t)4 * h * w + (size_t)(2 * p0) * (2 * w) + 2 * c;
+#pragma unroll
+    for (int r = 0; r < kUpStrip; ++r) {
+        if (p0 + r >= h) break;
+        float4 even, odd;
+        float *ev = &even.x, *od = &odd.x;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            ev[k] = 0.25f * f[r][k] + 0.75f * f[r + 1][k];
+            od[k] = 0.75f * f[r + 1][k] + 0.25f * f[r + 2][k];
+        }
+        *reinterpret_cast<float4 *>(o + (size_t)(2 * r) * (2 * w)) = even;
+        *reinterpret_cast<float4 *>(o + (size_t)(2 * r + 1) * (2 * w)) = odd;
+    }
+}
+
 // The adjoint: per axis dL/dx(p) = g(2p - 1)/4 + 3 g(2p)/4 + 3 g(2p + 1)/4 + g(2p + 2)/4,
 // terms outside the output dropped.
 __global__ __launch_bounds__(kThreads) void upsample2_blur_adjoint_kernel(const float *__restrict__ gy, int planes,
@@ -774,6 +838,40 @@ __global__ __launch_bounds__(kThreads) void upsample2_blur_adjoint_kernel(const 
         acc += wts[a] * racc;
     }
     gx[e] = acc;
+}
+
+// The adjoint for a width that is a multiple of 4 and 16-byte aligned tensors:
+// four neighbouring inputs per thread from four output rows of ten values, two
+// float4 and the two beside them.  23.2 us at 256 planes of 128^2, 45.7 with an
+// input per thread.
+__global__ __launch_bounds__(kThreads) void upsample2_blur_adjoint_rows_kernel(const float *__restrict__ gy, int planes,
+                                                                               int h, int w, float *__restrict__ gx) {
+    const int quarter = w / 4;
+    const size_t e = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (e >= (size_t)planes * h * quarter) return;
+    const int j = (int)(e % quarter), p = (int)((e / quarter) % h);
+    const size_t pl = e / ((size_t)quarter * h);
+    const int H2 = 2 * h, W2 = 2 * w, c = 8 * j;
+    const float *g = gy + pl * (size_t)H2 * W2;
+    const float wts[4] = {0.25f, 0.75f, 0.75f, 0.25f};
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const int oy = 2 * p - 1 + a;
+        const bool in = oy >= 0 && oy < H2;
+        const float *row = g + (size_t)(in ? oy : 0) * W2 + c;
+        const float4 lo = *reinterpret_cast<const float4 *>(row), hi = *reinterpret_cast<const float4 *>(row + 4);
+        const float v[10] = {c > 0 ? row[-1] : 0.0f, lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w,
+                             c + 8 < W2 ? row[8] : 0.0f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float r = 0.0f;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) r += wts[b] * v[2 * k + b];
+            if (in) acc[k] += wts[a] * r;
+        }
+    }
+    *reinterpret_cast<float4 *>(gx + (pl * h + p) * (size_t)w + 4 * j) = make_float4(acc[0], acc[1], acc[2], acc[3]);
 }
 
 #ifndef SVBRDF_CONV_KC
@@ -918,8 +1016,11 @@ namespace svbrdf_internal {
 
 void launch_split_sum(const ConvArgs &a, hipStream_t s) {
     const size_t total = (size_t)a.n * a.cout * a.h * a.w_;
-    hipLaunchKernelGGL(conv_split_sum_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                       s, a);
+    const bool vec = (size_t)a.h * a.w_ % 4 == 0 && (((uintptr_t)a.part | (uintptr_t)a.y) & 15u) == 0;
+    const size_t threads = vec ? total / 4 : total;
+    const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
+    if (vec) hipLaunchKernelGGL(conv_split_sum_kernel<4>, grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL(conv_split_sum_kernel<1>, grid, dim3(kThreads), 0, s, a);
 }
 
 ConvArgs input_grad_args(const float *grad_y, const float *y, int activation, int n, int cout, int height, int width,
@@ -1129,6 +1230,13 @@ int svbrdf_upsample2_blur(const float *x, int planes, int height, int width, flo
     if (planes < 1 || height < 1 || width < 1 || height > kMaxSide / 2 || width > kMaxSide / 2 ||
         (size_t)planes * 4 * height * width > ((size_t)1 << 34))
         return fail(SVBRDF_ESHAPE, "%s: planes=%d height=%d width=%d", what, planes, height, width);
+    if (width % 2 == 0 && (size_t)planes * 4 * height * width >= (1u << 18) && ((uintptr_t)x & 7u) == 0 &&
+        ((uintptr_t)y & 15u) == 0) {
+        const size_t threads = (size_t)planes * ((height + kUpStrip - 1) / kUpStrip) * (width / 2);
+        hipLaunchKernelGGL(upsample2_blur_rows_kernel, dim3((unsigned)((threads + kThreads - 1) / kThreads)),
+                           dim3(kThreads), 0, (hipStream_t)stream, x, planes, height, width, y);
+        return check_launch(what);
+    }
     const size_t total = (size_t)planes * 4 * height * width;
     hipLaunchKernelGGL(upsample2_blur_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0,
                        (hipStream_t)stream, x, planes, height, width, y);
@@ -1142,6 +1250,12 @@ int svbrdf_upsample2_blur_adjoint(const float *grad_y, int planes, int height, i
     if (planes < 1 || height < 1 || width < 1 || height > kMaxSide / 2 || width > kMaxSide / 2 ||
         (size_t)planes * 4 * height * width > ((size_t)1 << 34))
         return fail(SVBRDF_ESHAPE, "%s: planes=%d height=%d width=%d", what, planes, height, width);
+    if (width % 4 == 0 && (((uintptr_t)grad_y | (uintptr_t)grad_x) & 15u) == 0) {
+        const size_t threads = (size_t)planes * height * (width / 4);
+        hipLaunchKernelGGL(upsample2_blur_adjoint_rows_kernel, dim3((unsigned)((threads + kThreads - 1) / kThreads)),
+                           dim3(kThreads), 0, (hipStream_t)stream, grad_y, planes, height, width, grad_x);
+        return check_launch(what);
+    }
     const size_t total = (size_t)planes * height * width;
     hipLaunchKernelGGL(upsample2_blur_adjoint_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)),
                        dim3(kThreads), 0, (hipStream_t)stream, grad_y, planes, height, width, grad_x);
