@@ -499,6 +499,33 @@ int svbrdf_upsample2_blur(const float *x, int planes, int height, int width, flo
 int svbrdf_upsample2_blur_adjoint(const float *grad_y, int planes, int height, int width, float *grad_x,
                                   void *stream);
 
+/* The style layers of the synthesis network (the affine part of
+ * ModulateConvBlock, src/higan_models/stylegan2_generator_network.py:585-760) in
+ * one launch: styles[offset + r] = scale * dot(weight[r], latent[row]) +
+ * bias_scale * bias[r] for each of n_layers (at most 32) layers; weight [rows,
+ * dim] 16-byte aligned, latent [latent_rows, dim], dim a multiple of 4.  The
+ * layers are a host array.  And the gradient with respect to the latent from
+ * grad_styles (laid out as styles): workspace of
+ * svbrdf_style_layers_grad_workspace_bytes, 16-byte aligned. */
+typedef struct svbrdf_style_layer {
+    const float *weight, *bias;
+    int rows, offset, row;
+    float scale, bias_scale;
+} svbrdf_style_layer;
+int svbrdf_style_layers(const svbrdf_style_layer *layers, int n_layers, const float *latent, int latent_rows, int dim,
+                        float *styles, void *stream);
+size_t svbrdf_style_layers_grad_workspace_bytes(const svbrdf_style_layer *layers, int n_layers, int dim);
+int svbrdf_style_layers_grad(const svbrdf_style_layer *layers, int n_layers, const float *grad_styles, int latent_rows,
+                             int dim, float *grad_latent, void *workspace, size_t workspace_bytes, void *stream);
+
+/* The synthesis network's 1x1 output convolution of one sample with its skip
+ * connection (src/higan_models/stylegan2_generator_network.py:340-356): y
+ * [cout, height, width] = sum over c of weight[o][c] * (style[c] * scale) *
+ * x[c], plus, where skip is not NULL, skip [cout, height / 2, width / 2]
+ * upsampled as svbrdf_upsample2_blur does.  cout up to 9, cin up to 768. */
+int svbrdf_torgb(const float *x, int cin, int height, int width, const float *weight, int cout, const float *style,
+                 float scale, const float *skip, float *y, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -114,6 +114,12 @@ SIGNATURES = {
     "svbrdf_avgpool2": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp]),
     "svbrdf_avgpool2_adjoint": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp]),
     "svbrdf_upsample2_blur": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp]),
+    "svbrdf_style_layers": (ctypes.c_int, [_vp, ctypes.c_int, _vp, ctypes.c_int, ctypes.c_int, _vp, _vp]),
+    "svbrdf_style_layers_grad_workspace_bytes": (ctypes.c_size_t, [_vp, ctypes.c_int, ctypes.c_int]),
+    "svbrdf_style_layers_grad": (ctypes.c_int, [_vp, ctypes.c_int, _vp, ctypes.c_int, ctypes.c_int, _vp, _vp,
+                                                ctypes.c_size_t, _vp]),
+    "svbrdf_torgb": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, ctypes.c_int, _vp,
+                                    ctypes.c_float, _vp, _vp, _vp]),
     "svbrdf_upsample2_blur_adjoint": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp]),
 }
 

@@ -18,6 +18,7 @@ kernels of libsvbrdf_hip.so (csrc/conv.hip).
 * :class:`Conv3x3` -- a frozen 3x3 layer (VGG): weights packed once, in both
   layouts.
 """
+import numpy as np
 import torch
 
 from . import _lib
@@ -315,6 +316,94 @@ def modulated_conv3x3(x, style, weight, scale, demodulate=True, bias=None, noise
     return ModConv3x3Function.apply(x, style, weight, scale, demodulate, bias, noise, noise_strength, act)
 
 
+MAX_RGB = 9   # output channels of svbrdf_torgb
+_STYLE_LAYER = np.dtype([("weight", "<u8"), ("bias", "<u8"), ("rows", "<i4"), ("offset", "<i4"), ("row", "<i4"),
+                         ("scale", "<f4"), ("bias_scale", "<f4"), ("pad", "<i4")])   # svbrdf_style_layer
+
+
+class StyleLayersFunction(torch.autograd.Function):
+    """Every style layer of a synthesis pass in one launch: latent [1, L, dim],
+    the layers' weights [rows, dim] and biases [rows] and (latent row, scale,
+    bias scale) of each -> the styles side by side, [sum of rows].  The
+    weights are frozen; the backward gives dL/dlatent."""
+
+    @staticmethod
+    def _table(weights, biases, layers):
+        rows = [int(w.shape[0]) for w in weights]
+        table = np.zeros(len(weights), _STYLE_LAYER)
+        table["weight"] = [w.data_ptr() for w in weights]
+        table["bias"] = [b.data_ptr() for b in biases]
+        table["rows"] = rows
+        table["offset"] = np.cumsum([0] + rows[:-1])
+        table["row"], table["scale"], table["bias_scale"] = zip(*layers)
+        return table
+
+    @staticmethod
+    def forward(ctx, latent, weights, biases, layers):
+        x = latent.detach().contiguous()
+        table = StyleLayersFunction._table(weights, biases, layers)
+        out = torch.empty(int(table["rows"].sum()), dtype=torch.float32, device=x.device)
+        _lib.call("svbrdf_style_layers", table.ctypes.data, len(weights), _lib.ptr(x), int(x.shape[1]),
+                  int(x.shape[2]), _lib.ptr(out), _lib.stream_handle(x.device))
+        ctx.save_for_backward(*weights)
+        ctx.layers, ctx.shape = layers, tuple(x.shape)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        g = grad.contiguous()
+        weights = ctx.saved_tensors
+        table = StyleLayersFunction._table(weights, weights, ctx.layers)   # the biases are not read
+        _, n_rows, dim = ctx.shape
+        nb = int(_lib.query("svbrdf_style_layers_grad_workspace_bytes", table.ctypes.data, len(weights), dim))
+        ws = torch.empty(nb // 4, dtype=torch.float32, device=g.device)
+        out = torch.empty(ctx.shape, dtype=torch.float32, device=g.device)
+        _lib.call("svbrdf_style_layers_grad", table.ctypes.data, len(weights), _lib.ptr(g), n_rows, dim, _lib.ptr(out),
+                  _lib.ptr(ws), nb, _lib.stream_handle(g.device))
+        return out, None, None, None
+
+
+class ToRGBFunction(torch.autograd.Function):
+    """The 1x1 output convolution of one sample, its weight [cout, cin, 1, 1]
+    (frozen) scaled per input channel by style * scale, plus the upsampled
+    skip image (or None)."""
+
+    @staticmethod
+    def forward(ctx, x, style, weight, scale, skip):
+        x = x.contiguous()
+        st, wt = style.detach().contiguous(), weight.detach().contiguous()
+        sk = None if skip is None else skip.detach().contiguous()
+        for t, name in ((x, "x"), (st, "style"), (wt, "weight"), *(() if sk is None else ((sk, "skip"),))):
+            _check(t, name)
+        n, cin, h, w = (int(s) for s in x.shape)
+        cout = int(wt.shape[0])
+        if n != 1 or tuple(wt.shape) != (cout, cin, 1, 1) or st.numel() != cin:
+            raise ValueError(f"x {tuple(x.shape)}, weight {tuple(wt.shape)} and style {st.numel()} do not match")
+        if sk is not None and tuple(sk.shape) != (1, cout, h // 2, w // 2):
+            raise ValueError(f"skip {tuple(sk.shape)} is not half of [1, {cout}, {h}, {w}]")
+        y = torch.empty((1, cout, h, w), dtype=torch.float32, device=x.device)
+        _lib.call("svbrdf_torgb", _lib.ptr(x), cin, h, w, _lib.ptr(wt), cout, _lib.ptr(st), float(scale), _lib.ptr(sk),
+                  _lib.ptr(y), _lib.stream_handle(x.device))
+        ctx.save_for_backward(x, style, weight)
+        ctx.scale = float(scale)
+        return y
+
+    @staticmethod
+    def backward(ctx, grad_y):
+        x, style, weight = ctx.saved_tensors
+        g = grad_y.contiguous()
+        cout, cin = int(weight.shape[0]), int(weight.shape[1])
+        gm, wm = g.view(cout, -1), weight.view(cout, cin)
+        gx = gs = gskip = None
+        if ctx.needs_input_grad[0]:
+            gx = torch.mm((wm * (style.reshape(1, cin) * ctx.scale)).t(), gm).view(x.shape)
+        if ctx.needs_input_grad[1]:
+            gs = ((torch.mm(gm, x.view(cin, -1).t()) * wm).sum(dim=0) * ctx.scale).reshape(style.shape)
+        if ctx.needs_input_grad[4]:
+            gskip = Upsample2Function.adjoint(g)
+        return gx, gs, None, None, gskip
+
+
 class Upsample2Function(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):
@@ -327,6 +416,10 @@ class Upsample2Function(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_y):
+        return Upsample2Function.adjoint(grad_y)
+
+    @staticmethod
+    def adjoint(grad_y):
         g = grad_y.contiguous()
         n, c, h2, w2 = (int(s) for s in g.shape)
         gx = torch.empty((n, c, h2 // 2, w2 // 2), dtype=torch.float32, device=g.device)

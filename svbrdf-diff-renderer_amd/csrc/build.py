@@ -17,7 +17,7 @@ PKG = CSRC.parent
 ROOT = PKG.parent
 LIB = PKG / "libsvbrdf_hip.so"
 SOURCES = [CSRC / "svbrdf_hip.hip", CSRC / "codec.hip", CSRC / "conv.hip", CSRC / "conv_split.hip",
-           CSRC / "common.hip"]
+           CSRC / "generator.hip", CSRC / "common.hip"]
 HEADERS = [CSRC / "brdf.hpp", CSRC / "common.hpp", CSRC / "conv_common.hpp", ROOT / "include" / "svbrdf_hip.h"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")

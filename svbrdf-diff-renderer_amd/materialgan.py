@@ -96,7 +96,14 @@ class _ModConv(torch.nn.Module):
             wt = wt * torch.rsqrt((wt * wt).sum(dim=(1, 2, 3), keepdim=True) + 1e-8)
         return wt
 
-    def forward(self, x, w, bias=None, noise=None, noise_strength=0.0, act="none"):
+    def forward(self, x, w, bias=None, noise=None, noise_strength=0.0, act="none", style=None, skip=None):
+        """style: affine(w) where the caller has it already; skip: an image of
+        half the size whose x2 upsampling is added (1x1 layers)."""
+        if (self.k == 1 and style is not None and not self.demodulate and x.shape[0] == 1
+                and self.weight.shape[0] <= convnet.MAX_RGB):
+            return convnet.ToRGBFunction.apply(x, style, self.weight, self.scale, skip)
+        if self.k == 1 and skip is not None:
+            return convnet.upsample2(skip) + self.forward(x, w)
         if self.k == 1:
             # a 1x1 convolution is a plain GEMM: [Cout, Cin] x [Cin, H W] per
             # sample (torch.mm for the one sample: no broadcast copies)
@@ -108,7 +115,8 @@ class _ModConv(torch.nn.Module):
         # 3x3: the modulation and demodulation happen inside the HIP weight
         # packing, and the style's gradient comes from the HIP modulation
         # backward, instead of torch ops on the whole weight tensor
-        style = self.affine(w)
+        if style is None:
+            style = self.affine(w)
         if self.upsample:
             x = convnet.upsample2(x)
         return convnet.modulated_conv3x3(x, style, self.weight, self.scale, self.demodulate, bias, noise,
@@ -173,16 +181,37 @@ class StyleGAN2Generator(torch.nn.Module):
         # one unbind instead of an index per layer: its backward is one stack
         # of the per-layer gradients, not a zero-filled copy per layer
         ws = wp.unbind(1)
+        styles = self._styles(wp)
         for i, conv in enumerate(self.convs):
             # conv + noise_strength * noise + bias, leaky ReLU x sqrt(2), in one kernel
             x = conv(x, ws[min(wi, self.num_layers - 1)], bias=self.bias[i], noise=noises[i],
-                     noise_strength=self.noise_strength_values[i], act="lrelu")
+                     noise_strength=self.noise_strength_values[i], act="lrelu", style=styles[i])
             wi += 1
             if i == 0 or i % 2 == 0:
                 # toRGB after each resolution's last convolution, skip-summed
-                t = self.to_rgb[(i + 1) // 2](x, ws[min(wi, self.num_layers - 1)])
-                rgb = t if rgb is None else convnet.upsample2(rgb) + t
+                k = (i + 1) // 2
+                rgb = self.to_rgb[k](x, ws[min(wi, self.num_layers - 1)], style=styles[len(self.convs) + k], skip=rgb)
         return rgb
+
+    def _styles(self, wp):
+        """Every layer's style (the convolutions', then the toRGB layers'), [1,
+        rows] each, from one launch; None each, for the layers to compute
+        their own, where the latent is not one float32 W+ on the GPU or a
+        layer's weights are being trained."""
+        layers = [*self.convs, *self.to_rgb]
+        weights, biases = [c.affine.weight for c in layers], [c.affine.bias for c in layers]
+        if (wp.dim() != 3 or wp.shape[0] != 1 or wp.shape[1] < self.num_layers or wp.shape[2] != 512
+                or wp.dtype != torch.float32 or not wp.is_cuda
+                or any(t.requires_grad or t.device != wp.device or not t.is_contiguous() or t.dtype != torch.float32
+                       for t in [*weights, *biases, *(c.weight for c in layers)])):
+            return [None] * len(layers)
+        # convolution i reads latent row i, the toRGB layer behind it row i + 1
+        last = self.num_layers - 1
+        rows = [min(i, last) for i in range(len(self.convs))]
+        rows += [min(2 * k + 1, last) for k in range(len(self.to_rgb))]
+        scales = [(r, c.affine.scale, c.affine.lr_mul) for c, r in zip(layers, rows)]
+        out = convnet.StyleLayersFunction.apply(wp, weights, biases, scales)
+        return [s.view(1, -1) for s in out.split([w.shape[0] for w in weights])]
 
 
 class VGGLoss(torch.nn.Module):
