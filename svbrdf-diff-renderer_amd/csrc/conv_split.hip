@@ -90,7 +90,23 @@ __global__ __launch_bounds__(kThreads) void split_factor_kernel(const float *__r
     const int n = cin * 9;
     const float *wc = w + (size_t)blockIdx.x * n;
     float acc = 0.0f;
-    for (int e = threadIdx.x; e < n; e += kThreads) {
+    // six elements' loads in flight (512 rows of 512 channels: 8.1 -> 4.7 us)
+    constexpr int U = 6;
+    int e = threadIdx.x;
+    for (; e + (U - 1) * kThreads < n; e += U * kThreads) {
+        float v[U], sv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[u] = wc[e + u * kThreads];
+            sv[u] = style ? style[(e + u * kThreads) / 9] : 1.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float x = v[u] * scale * sv[u];
+            acc += x * x;
+        }
+    }
+    for (; e < n; e += kThreads) {
         const float v = wc[e] * scale * (style ? style[e / 9] : 1.0f);
         acc += v * v;
     }
@@ -110,7 +126,9 @@ enum PackForm {
 // One block per 32 outputs and 16-channel chunk: the source rows go to LDS as
 // they lie in memory (runs of 144, 288 or 32 floats), then each thread writes
 // the 16 bytes of a lane's operand for one tap and term: 1 KB per wave and
-// store, contiguous.  A bandwidth-bound pass over 10 bytes per weight.
+// store, contiguous.  A bandwidth-bound pass over 10 bytes per weight: 512 x
+// 512 (24 MB) in 7.0 us from the layer's weights, 9.6 from packed ones (12.4
+// and 14.0 with the loads one behind the other).
 template <PackForm FORM>
 __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float *__restrict__ w, int m_total, int k_total,
                                                               const float *__restrict__ style, float scale,
@@ -119,28 +137,56 @@ __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float *__res
     constexpr int ROWS = FORM == kNatural ? 32 : FORM == kTransposed ? kKC : 9 * kKC;
     constexpr int RUN = FORM == kNatural ? kKC * 9 : FORM == kTransposed ? 32 * 9 : 32;
     constexpr int PITCH = RUN + 1;
+    constexpr int PER = ROWS * RUN / kThreads;   // 18, whichever the form
+    static_assert(ROWS * RUN == PER * kThreads, "whole passes");
     __shared__ float tile[ROWS * PITCH];
+    __shared__ float by_m[32], by_k[kKC];        // a weight's factors by output and by input channel
     const int groups = groups_of(m_total);
     const int m0 = blockIdx.x * 32, chunk = blockIdx.y;
     const int k0 = chunk_base(chunk, k_total), skip = chunk * kKC - k0;   // channels of the chunk before
-    for (int e = threadIdx.x; e < ROWS * RUN; e += kThreads) {
+    float v[PER];   // all loads in flight: a valid address and a select
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = threadIdx.x + i * kThreads;
         const int r = e / RUN, c = e - r * RUN;
-        float v = 0.0f;
+        bool ok;
+        size_t o;
         if constexpr (FORM == kNatural) {
-            if (m0 + r < m_total && c / 9 >= skip) v = w[((size_t)(m0 + r) * k_total + k0) * 9 + c];
+            ok = m0 + r < m_total && c / 9 >= skip;
+            o = ((size_t)(m0 + r) * k_total + k0) * 9 + c;
         } else if constexpr (FORM == kTransposed) {
-            if (r >= skip && m0 + c / 9 < m_total) v = w[((size_t)(k0 + r) * m_total + m0) * 9 + c];
+            ok = r >= skip && m0 + c / 9 < m_total;
+            o = ((size_t)(k0 + r) * m_total + m0) * 9 + c;
         } else {
             const int t = r / kKC, k = r % kKC;
-            if (k >= skip && m0 + c < m_total) v = w[((size_t)t * k_total + k0 + k) * m_total + m0 + c];
+            ok = k >= skip && m0 + c < m_total;
+            o = ((size_t)t * k_total + k0 + k) * m_total + m0 + c;
         }
-        tile[r * PITCH + c] = v;
+        const float x = w[ok ? o : 0];
+        v[i] = ok ? x : 0.0f;
+    }
+    if constexpr (FORM != kPacked) {
+        // the style belongs to the layer's input channels, the demodulation
+        // factor to its output channels
+        if (threadIdx.x < 32) {
+            const int m = min(m0 + (int)threadIdx.x, m_total - 1);
+            const float *f = FORM == kNatural ? factor : style;
+            by_m[threadIdx.x] = f ? f[m] : 1.0f;
+        } else if (threadIdx.x < 32 + kKC) {
+            const float *f = FORM == kNatural ? style : factor;
+            by_k[threadIdx.x - 32] = f ? f[k0 + threadIdx.x - 32] : 1.0f;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = threadIdx.x + i * kThreads;
+        const int r = e / RUN, c = e - r * RUN;
+        tile[r * PITCH + c] = v[i];
     }
     __syncthreads();
     for (int q = threadIdx.x; q < 9 * 64; q += kThreads) {
         const int t = q / 64, lane = q & 63;
         const int mm = lane & 31, kk = (lane >> 5) * 8;
-        const int m = min(m0 + mm, m_total - 1);   // padding rows hold zeros
         uint4 term[3];
         unsigned *h = &term[0].x, *md = &term[1].x, *l = &term[2].x;
 #pragma unroll
@@ -148,16 +194,10 @@ __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float *__res
             float v[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int k = k0 + kk + j + i;
-                if constexpr (FORM == kPacked) {
-                    v[i] = tile[(t * kKC + kk + j + i) * PITCH + mm];
-                } else if constexpr (FORM == kNatural) {
-                    v[i] = tile[mm * PITCH + (kk + j + i) * 9 + t] * scale * (style ? style[k] : 1.0f) *
-                           (factor ? factor[m] : 1.0f);
-                } else {
-                    v[i] = tile[(kk + j + i) * PITCH + mm * 9 + (8 - t)] * scale * (style ? style[m] : 1.0f) *
-                           (factor ? factor[k] : 1.0f);
-                }
+                const int k = kk + j + i;
+                if constexpr (FORM == kPacked) v[i] = tile[(t * kKC + k) * PITCH + mm];
+                else if constexpr (FORM == kNatural) v[i] = tile[mm * PITCH + k * 9 + t] * scale * by_k[k] * by_m[mm];
+                else v[i] = tile[k * PITCH + mm * 9 + (8 - t)] * scale * by_m[mm] * by_k[k];
                 v[i] = chunk & 1 ? -v[i] : v[i];
             }
             split_pair(v[0], v[1], h[j / 2], md[j / 2], l[j / 2]);
