@@ -22,7 +22,8 @@
 //                         partial sums go to the caller's workspace;
 //   conv_split_sum_kernel then adds the slices in order and applies the
 //                         epilogue.
-//   conv3x3_wgrad_kernel  dL/dw of the convolution: per tap a GEMM over the
+//   conv3x3_wgrad_kernel  dL/dw of the convolution (narrow and small images; the
+//                         others: conv_split.hip): per tap a GEMM over the
 //                         pixels (M = Cout, N = Cin), the nine taps sharing
 //                         the dL/dy operand; wgrad_sum_kernel adds its
 //                         pixel slices.
@@ -685,21 +686,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
 // Sum of the weight-gradient slices: eight running sums over the slices
 // s = j mod 8 (eight loads in flight per trip), then combined in a fixed
-// order -- the same bits on every run.
+// order -- the same bits on every run, and for either VEC (4 consecutive values
+// per thread where the count is a multiple of 4 and the tensors are aligned:
+// 4 slices of 512 x 512 x 9 take 8.8 us, 11.3 one value per thread).
+template <int VEC>
 __global__ __launch_bounds__(kThreads) void wgrad_sum_kernel(const float *__restrict__ part, int slices, size_t total,
                                                              float *__restrict__ out) {
-    const size_t e = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const size_t e = ((size_t)blockIdx.x * kThreads + threadIdx.x) * VEC;
     if (e >= total) return;
-    float v[8];
+    vec v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = 0.0f;
-    int s = 0;
-    for (; s + 8 <= slices; s += 8) {
+    for (int s = 0; s < slices; s += 8) {
+        vec q[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] += part[(size_t)(s + j) * total + e];
+        for (int j = 0; j < 8; ++j) {
+            // past the last slice: its own values again, not added
+            const int k = s + j < slices ? s + j : slices - 1;
+            q[j] = *reinterpret_cast<const vec *>(part + (size_t)k * total + e);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (s + j < slices) v[j] += q[j];
     }
-    for (int j = 0; s + j < slices; ++j) v[j] += part[(size_t)(s + j) * total + e];
-    out[e] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    *reinterpret_cast<vec *>(out + e) = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
 }
 
 // ---------------------------------------------------------------------------
@@ -1181,8 +1192,21 @@ int svbrdf_conv3x3_input_grad(const float *grad_y, const float *y, int activatio
     return run_conv(what, a, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+// Where the weight gradient runs on split operands (conv_split.hip): its chunks
+// are 32 pixels wide, so below 16 columns most of their work is padding (us,
+// fp32 / split: 512 x 512 at 8^2 22 / 29, 16^2 41 / 38, 32^2 82 / 46, 64^2 223 /
+// 122; 256 -> 128 at 256^2 408 / 222; 128 x 128 at 32^2 27 / 20), and below 0.15
+// GFLOP both are launches and first loads.
+static bool wgrad_takes_split(int n, int cin, int h, int w, int cout) {
+    return w >= 16 && 18.0 * n * cin * cout * h * w >= 1.5e8;
+}
+
 size_t svbrdf_conv3x3_wgrad_workspace_bytes(int n, int cin, int height, int width, int cout) {
     if (!conv_shape_ok(n, cin, height, width, cout)) return 0;
+    if (wgrad_takes_split(n, cin, height, width, cout)) {
+        const int slices = plan_wgrad_split(n, cin, height, width, cout).slices;
+        return slices > 1 ? (size_t)slices * 9 * cin * cout * sizeof(float) : 0;
+    }
     return plan_wgrad(n, cin, height, width, cout).part_floats * sizeof(float);
 }
 
@@ -1192,24 +1216,38 @@ int svbrdf_conv3x3_wgrad(const float *x, const float *grad_z, int n, int cin, in
     if (!x || !grad_z || !grad_w) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
     if (!conv_shape_ok(n, cin, height, width, cout))
         return fail(SVBRDF_ESHAPE, "%s: n=%d cin=%d cout=%d height=%d width=%d", what, n, cin, cout, height, width);
-    const WgradPlan p = plan_wgrad(n, cin, height, width, cout);
-    const size_t need = p.part_floats * sizeof(float);
+    const size_t need = svbrdf_conv3x3_wgrad_workspace_bytes(n, cin, height, width, cout);
     if (need && (!workspace || workspace_bytes < need))
         return fail(SVBRDF_ESPACE, "%s: workspace of %zu bytes, this shape needs %zu "
                     "(svbrdf_conv3x3_wgrad_workspace_bytes)", what, workspace ? workspace_bytes : (size_t)0, need);
-    WgradArgs a{};
-    a.x = x; a.gz = grad_z; a.out = p.slices > 1 ? (float *)workspace : grad_w;
-    a.n = n; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
-    a.tiles_x = p.tiles_x; a.tiles_per_img = p.tiles_per_img; a.n_chunks = p.n_chunks;
-    a.cps = p.cps;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid((unsigned)p.co_tiles, (unsigned)p.ci_tiles, (unsigned)p.slices);
-    if (p.tw == 8) hipLaunchKernelGGL(conv3x3_wgrad_kernel<8>, grid, dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL(conv3x3_wgrad_kernel<4>, grid, dim3(kThreads), 0, s, a);
-    if (p.slices > 1) {
+    float *out = need ? (float *)workspace : grad_w;
+    int slices;
+    if (wgrad_takes_split(n, cin, height, width, cout)) {
+        const WgradSplitPlan p = plan_wgrad_split(n, cin, height, width, cout);
+        slices = p.slices;
+        launch_wgrad_split(p, x, grad_z, n, cin, height, width, cout, out, s);
+    } else {
+        const WgradPlan p = plan_wgrad(n, cin, height, width, cout);
+        slices = p.slices;
+        WgradArgs a{};
+        a.x = x; a.gz = grad_z; a.out = out;
+        a.n = n; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
+        a.tiles_x = p.tiles_x; a.tiles_per_img = p.tiles_per_img; a.n_chunks = p.n_chunks;
+        a.cps = p.cps;
+        const dim3 grid((unsigned)p.co_tiles, (unsigned)p.ci_tiles, (unsigned)p.slices);
+        if (p.tw == 8) hipLaunchKernelGGL(conv3x3_wgrad_kernel<8>, grid, dim3(kThreads), 0, s, a);
+        else hipLaunchKernelGGL(conv3x3_wgrad_kernel<4>, grid, dim3(kThreads), 0, s, a);
+    }
+    if (slices > 1) {
         const size_t total = (size_t)9 * cin * cout;
-        hipLaunchKernelGGL(wgrad_sum_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                           s, (const float *)workspace, p.slices, total, grad_w);
+        const bool vec = total % 4 == 0 && (((uintptr_t)workspace | (uintptr_t)grad_w) & 15u) == 0;
+        const size_t threads = vec ? total / 4 : total;
+        const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
+        if (vec) hipLaunchKernelGGL(wgrad_sum_kernel<4>, grid, dim3(kThreads), 0, s, (const float *)workspace, slices,
+                                    total, grad_w);
+        else hipLaunchKernelGGL(wgrad_sum_kernel<1>, grid, dim3(kThreads), 0, s, (const float *)workspace, slices, total,
+                                grad_w);
     }
     return check_launch(what);
 }

@@ -72,4 +72,15 @@ __attribute__((visibility("hidden"))) ConvArgs input_grad_args(const float *grad
                                                                int n, int cout, int height, int width, int cin,
                                                                float *grad_x);
 
+// The weight gradient on split operands (conv_split.hip): its tiling with the
+// estimated time, and the launch; out: [slices][Cout][Cin][9].
+struct WgradSplitPlan {
+    int strips, n_chunks, co_tiles, ci_tiles, slices, cps;
+    double us;
+};
+__attribute__((visibility("hidden"))) WgradSplitPlan plan_wgrad_split(int n, int cin, int h, int w, int cout);
+__attribute__((visibility("hidden"))) void launch_wgrad_split(const WgradSplitPlan &p, const float *x,
+                                                              const float *grad_z, int n, int cin, int h, int w,
+                                                              int cout, float *out, hipStream_t s);
+
 }  // namespace svbrdf_internal

@@ -36,6 +36,8 @@
 //   split_pack_kernel     weights -> the matrix core's operand order, split:
 //                         [K chunk of 16][tap][h, m, l][32 outputs][lane][8].
 //   conv3x3_split_kernel  the convolution.
+//   conv3x3_wgrad_split_kernel
+//                         its weight gradient.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -542,6 +544,288 @@ __global__ __launch_bounds__(kThreads, 2) void conv3x3_split_kernel(SplitArgs s)
     store_tile(a, img, slice, com, oy, ox, acc);
 }
 
+// ---------------------------------------------------------------------------
+// The weight gradient (conv.hip's conv3x3_wgrad_kernel) on split operands: per
+// tap a GEMM over the pixels, M = output channels, N = input channels.  A block
+// of twelve waves owns 64 x 64 (co, ci) for all nine taps: a wave 32 x 32 of
+// the three taps of one kernel row.  K runs over chunks of 32 pixels of one
+// image row, down a strip of the image: the chunk's dL/dz and the input row
+// below it go to LDS split, [term][row][pixel octet][channel] with 16 bytes of
+// eight pixels each, so a lane's operand is one ds_read_b128; the input rows
+// stay for the three chunks that read them (a ring of four).  The taps to the
+// left and right are an octet shifted by a pixel in registers (v_alignbit) with
+// the neighbouring octets' edge.  One block a compute unit: three waves per
+// matrix core hide each other's reads, shifts and splits.  The sums and dL/dz
+// change sign every second chunk, for the reason given above.
+// The sums leave through LDS: a lane's are 9 floats apart in the output.
+//
+// Matrix cores 41 % busy at 2.1 GHz; what is left is the operand reads behind
+// each chunk's barrier.  512 x 512 at 64^2: 122 us with the sum of 4 slices (159
+// TFLOP/s; the fp32 kernel 223), 256 -> 128 at 256^2 222 (408).  Re-reading all
+// three input rows for every chunk took 155 and 265, stores straight from the
+// accumulators 8 to 14 more.  Error against 64 bits: 9.0e-8 (fp32 1.8e-7) for
+// 128 x 128 at 64^2.
+constexpr int kWgThreads = 768;
+constexpr int kWgTile = 64;                      // output and input channels of a block
+constexpr int kWgPixels = 32;                    // pixels of a chunk
+constexpr int kWgOctets = kWgPixels / 8;
+// An octet's 64 channels, plus 32 bytes: the stores of neighbouring octets
+// meet different banks.
+constexpr int kWgStride = kWgTile + 2;           // in 16-byte units
+
+struct WgradSplitArgs {
+    const float *x, *gz;
+    float *out;
+    int n, cin, cout, h, w_;
+    int strips, n_chunks, cps;
+};
+
+__device__ __forceinline__ uint4 shifted_left(const uint4 &v, unsigned before) {   // pixels p - 1
+    return make_uint4(__builtin_amdgcn_alignbit(v.x, before, 16), __builtin_amdgcn_alignbit(v.y, v.x, 16),
+                      __builtin_amdgcn_alignbit(v.z, v.y, 16), __builtin_amdgcn_alignbit(v.w, v.z, 16));
+}
+__device__ __forceinline__ uint4 shifted_right(const uint4 &v, unsigned after) {   // pixels p + 1
+    return make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                      __builtin_amdgcn_alignbit(v.w, v.z, 16), __builtin_amdgcn_alignbit(after, v.w, 16));
+}
+
+// A wave's sums again on the fp32 instruction: only where they were not finite.
+__device__ __forceinline__ void redo_wgrad_fp32(const WgradSplitArgs &a, int c_begin, int c_end, int co, int ci, int dy,
+                                                v16f (&acc)[3]) {
+    const int lane = threadIdx.x & 63;
+    const size_t HW = (size_t)a.h * a.w_;
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
+#pragma unroll 1
+    for (int c = c_begin; c < c_end; ++c) {
+        const int y = c % a.h, strip = c / a.h % a.strips, img = c / a.h / a.strips;
+        const int yy = y + dy - 1;
+#pragma unroll 1
+        for (int k = 0; k < kWgPixels; k += 2) {
+            const int x = strip * kWgPixels + k + (lane >> 5);
+            float g = 0.0f;
+            if (co < a.cout && x < a.w_) g = a.gz[((size_t)img * a.cout + co) * HW + (size_t)y * a.w_ + x];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                const int xx = x + t - 1;
+                float v = 0.0f;
+                if (ci < a.cin && yy >= 0 && yy < a.h && xx >= 0 && xx < a.w_)
+                    v = a.x[((size_t)img * a.cin + ci) * HW + (size_t)yy * a.w_ + xx];
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(g, v, acc[t], 0, 0, 0);
+            }
+        }
+    }
+}
+
+// VEC: rows of a multiple of four pixels, 16-byte aligned tensors.
+template <bool VEC>
+__global__ __launch_bounds__(kWgThreads) void conv3x3_wgrad_split_kernel(WgradSplitArgs a) {
+    // the operands while the sums grow, the block's 64 x 64 x 9 sums afterwards
+    union Shared {
+        struct {
+            uint4 xs[4][3][kWgOctets + 2][kWgStride];   // [row mod 4][term][octet, one more at either end]
+            uint4 gs[2][3][kWgOctets][kWgStride];
+        };
+        float sums[kWgTile][kWgTile * 9];
+    };
+    __shared__ Shared lds;
+    auto &xs = lds.xs;
+    auto &gs = lds.gs;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int dy = wave >> 2, mh = (wave >> 1) & 1, nh = wave & 1;
+    const int co0 = blockIdx.x * kWgTile, ci0 = blockIdx.y * kWgTile, slice = blockIdx.z;
+    const int H = a.h, W = a.w_;
+    const size_t HW = (size_t)H * W;
+    const int c_begin = slice * a.cps, c_end = min(a.n_chunks, c_begin + a.cps);
+
+    // Staging: the first 256 threads an octet of an input row each, the next
+    // 256 one of dL/dz, 128 more one of the pixels beside the row.
+    const int role = wave >> 2;                              // 0: input, 1: dL/dz, 2: edges (half of them)
+    const int s_oct = tid & 3, s_ch = (tid >> 2) & 63;
+    const int e_side = tid & 1, e_ch = (tid >> 1) & 63;
+    const bool has_edge = tid >= 512 && tid < 640;
+    float v[8];
+    auto load_octet = [&](float (&v)[8], const float *row, int x0, bool ok) {
+        if constexpr (VEC) {
+            const bool lo = ok && x0 < W, hi = ok && x0 + 4 < W;
+            const float4 p = *reinterpret_cast<const float4 *>(lo ? row + x0 : row);
+            const float4 q = *reinterpret_cast<const float4 *>(hi ? row + x0 + 4 : row);
+            v[0] = lo ? p.x : 0.0f; v[1] = lo ? p.y : 0.0f; v[2] = lo ? p.z : 0.0f; v[3] = lo ? p.w : 0.0f;
+            v[4] = hi ? q.x : 0.0f; v[5] = hi ? q.y : 0.0f; v[6] = hi ? q.z : 0.0f; v[7] = hi ? q.w : 0.0f;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const bool in = ok && x0 + j < W;
+                const float p = row[in ? x0 + j : 0];
+                v[j] = in ? p : 0.0f;
+            }
+        }
+    };
+    // input row yy of a strip (zero outside the image)
+    auto load_input = [&](float (&v)[8], int img, int strip, int yy) {
+        const float *xi = a.x + (size_t)img * a.cin * HW;
+        const int x0 = strip * kWgPixels;
+        if (role == 0) {
+            const bool ok = ci0 + s_ch < a.cin && yy >= 0 && yy < H;
+            load_octet(v, xi + (ok ? (size_t)(ci0 + s_ch) * HW + (size_t)yy * W : 0), x0 + s_oct * 8, ok);
+        } else if (has_edge) {
+            const int xx = e_side ? x0 + kWgPixels : x0 - 1;
+            const bool ok = ci0 + e_ch < a.cin && yy >= 0 && yy < H && xx >= 0 && xx < W;
+            const float p = xi[ok ? (size_t)(ci0 + e_ch) * HW + (size_t)yy * W + xx : 0];
+            v[0] = ok ? p : 0.0f;
+        }
+    };
+    auto load_grad = [&](int img, int strip, int y) {
+        if (role != 1) return;
+        const bool ok = co0 + s_ch < a.cout;
+        const float *gi = a.gz + (size_t)img * a.cout * HW;
+        load_octet(v, gi + (ok ? (size_t)(co0 + s_ch) * HW + (size_t)y * W : 0), strip * kWgPixels + s_oct * 8, ok);
+    };
+    auto split_octet = [&](const float (&v)[8], uint4 (&t)[3]) {
+        unsigned *h = &t[0].x, *m = &t[1].x, *l = &t[2].x;
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) split_pair(v[j], v[j + 1], h[j / 2], m[j / 2], l[j / 2]);
+    };
+    auto store_input = [&](const float (&v)[8], int yy) {
+        const int slot = (yy + 1) & 3;
+        if (role == 0) {
+            uint4 t[3];
+            split_octet(v, t);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) xs[slot][k][1 + s_oct][s_ch] = t[k];
+        } else if (has_edge) {
+            // the last pixel of the octet before, the first of the one after
+            unsigned t[3];
+            split_pair(e_side ? v[0] : 0.0f, e_side ? 0.0f : v[0], t[0], t[1], t[2]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                reinterpret_cast<unsigned *>(&xs[slot][k][e_side ? 1 + kWgOctets : 0][e_ch])[e_side ? 0 : 3] = t[k];
+        }
+    };
+    auto store_grad = [&](int buf, bool negative) {
+        if (role != 1) return;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = negative ? -v[j] : v[j];
+        uint4 t[3];
+        split_octet(v, t);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gs[buf][k][s_oct][s_ch] = t[k];
+    };
+
+    // counts negatively: every second pair of chunks
+    const auto negative = [&](int c) { return ((c - c_begin) & 2) != 0; };
+    int y = c_begin % H, strip = c_begin / H % a.strips, img = c_begin / H / a.strips;
+    {
+        // the first chunk, its loads all in flight
+        float rows[3][8];
+        load_grad(img, strip, y);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) load_input(rows[k], img, strip, y - 1 + k);
+        store_grad(0, false);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) store_input(rows[k], y - 1 + k);
+    }
+    bool fresh = false;      // a chunk starts a strip: its input rows are not in the ring
+    v16f acc[3], low[3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][r] = low[t][r] = 0.0f;
+    for (int c = c_begin; c < c_end; ++c) {
+        const int buf = (c - c_begin) & 1;
+        if (fresh) {
+            for (int k = 0; k < 3; ++k) {
+                load_input(v, img, strip, y - 1 + k);
+                store_input(v, y - 1 + k);
+            }
+        }
+        __syncthreads();
+        // the next chunk: its dL/dz, and its last input row unless it starts a strip
+        int y1 = y + 1, strip1 = strip, img1 = img;
+        if (y1 == H) {
+            y1 = 0;
+            if (++strip1 == a.strips) {
+                strip1 = 0;
+                ++img1;
+            }
+        }
+        const bool more = c + 1 < c_end;
+        fresh = y1 == 0;
+        if (more) {
+            load_grad(img1, strip1, y1);
+            if (!fresh) load_input(v, img, strip, y + 2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < kWgPixels / 16; ++ks) {
+            const int q = 2 * ks + (lane >> 5);
+            v8bf g[3], b[3][3];   // [term], [tap][term]
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                g[k] = __builtin_bit_cast(v8bf, gs[buf][k][q][mh * 32 + (lane & 31)]);
+                const uint4 *col = &xs[(y + dy) & 3][k][q][nh * 32 + (lane & 31)];
+                const uint4 u = col[kWgStride];
+                b[0][k] = __builtin_bit_cast(v8bf, shifted_left(u, col[0].w));
+                b[1][k] = __builtin_bit_cast(v8bf, u);
+                b[2][k] = __builtin_bit_cast(v8bf, shifted_right(u, col[2 * kWgStride].x));
+            }
+            constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int p = 0; p < 6; ++p)
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    v16f &d = p < 5 ? low[t] : acc[t];
+                    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(g[TA[p]], b[t][TB[p]], d, 0, 0, 0);
+                }
+        }
+        if (more) {
+            store_grad(buf ^ 1, negative(c + 1));
+            if (!fresh) store_input(v, y + 2);
+            if (negative(c) != negative(c + 1)) {
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        acc[t][r] = -acc[t][r];
+                        low[t][r] = -low[t][r];
+                    }
+            }
+            if (fresh) __syncthreads();   // every wave is done with the old strip's rows
+        }
+        y = y1;
+        strip = strip1;
+        img = img1;
+    }
+    const bool flip = c_end > c_begin && negative(c_end - 1);
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            acc[t][r] += low[t][r];
+            acc[t][r] = flip ? -acc[t][r] : acc[t][r];
+            bad |= !(fabsf(acc[t][r]) <= FLT_MAX);
+        }
+    const int ci = ci0 + nh * 32 + (lane & 31);
+    if (__any(bad)) redo_wgrad_fp32(a, c_begin, c_end, co0 + mh * 32 + (lane & 31), ci, dy, acc);
+    // through LDS: a row of the output is 64 x 9 consecutive values, a lane's are 9 apart
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int co = mh * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) lds.sums[co][(nh * 32 + (lane & 31)) * 9 + dy * 3 + t] = acc[t][r];
+    }
+    __syncthreads();
+    float *o = a.out + (size_t)slice * a.cout * a.cin * 9 + ((size_t)co0 * a.cin + ci0) * 9;
+    const int rows = min(kWgTile, a.cout - co0), run = min(kWgTile, a.cin - ci0) * 9;
+#pragma unroll 1
+    for (int r = wave; r < rows; r += kWgThreads / 64)
+        for (int e = lane; e < run; e += 64) o[(size_t)r * a.cin * 9 + e] = lds.sums[r][e];
+}
+
 // How a convolution runs: the block tile, the tiling of the image, the K split.
 struct SplitPlan {
     int wm, wn, tw, th, tiles_x, tiles_y, co_tiles, slices, cps;
@@ -628,6 +912,43 @@ int run_split(const char *what, ConvArgs a, const void *split, void *workspace, 
 size_t split_floats(int k, int m) { return (size_t)chunks_of(k) * 9 * 3 * groups_of(m) * 64 * 4; }
 
 }  // namespace
+
+namespace svbrdf_internal {
+
+WgradSplitPlan plan_wgrad_split(int n, int cin, int h, int w, int cout) {
+    WgradSplitPlan p{};
+    p.strips = (w + kWgPixels - 1) / kWgPixels;
+    p.n_chunks = n * p.strips * h;
+    p.co_tiles = (cout + kWgTile - 1) / kWgTile;
+    p.ci_tiles = (cin + kWgTile - 1) / kWgTile;
+    const double blocks = (double)p.co_tiles * p.ci_tiles, out_bytes = 36.0 * cin * cout;
+    const int max_slices = std::max(1, std::min(256, p.n_chunks / 2));
+    for (int s = 1; s <= max_slices; ++s) {
+        const int cps = (p.n_chunks + s - 1) / s;
+        if ((p.n_chunks + cps - 1) / cps != s) continue;   // no empty slice
+        // measured: one block a compute unit at a time, a chunk 3.1 us, ~11 for
+        // the launch, the first loads and the last stores, then the slices' sum
+        double t = std::ceil(blocks * s / kComputeUnits) * (cps * 3.1 + 3.0) + 8.0;
+        if (s > 1) t += (s + 1) * out_bytes / 5.3e6 + 1.5;
+        if (s == 1 || t < 0.98 * p.us) {
+            p.us = t;
+            p.slices = s;
+            p.cps = cps;
+        }
+    }
+    return p;
+}
+
+void launch_wgrad_split(const WgradSplitPlan &p, const float *x, const float *grad_z, int n, int cin, int h, int w,
+                        int cout, float *out, hipStream_t s) {
+    const WgradSplitArgs a{x, grad_z, out, n, cin, cout, h, w, p.strips, p.n_chunks, p.cps};
+    const dim3 grid((unsigned)p.co_tiles, (unsigned)p.ci_tiles, (unsigned)p.slices);
+    const bool vec = w % 4 == 0 && (((uintptr_t)x | (uintptr_t)grad_z) & 15u) == 0;
+    if (vec) hipLaunchKernelGGL(conv3x3_wgrad_split_kernel<true>, grid, dim3(kWgThreads), 0, s, a);
+    else hipLaunchKernelGGL(conv3x3_wgrad_split_kernel<false>, grid, dim3(kWgThreads), 0, s, a);
+}
+
+}  // namespace svbrdf_internal
 
 extern "C" {
 

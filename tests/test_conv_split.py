@@ -181,3 +181,54 @@ def test_split_conv_spreads_infinities_like_fp32(pkg, where):
     # both sides' roundings: fp32's once per product pair
     bound = (_bound(cin) + 9 * cin / 2 * 2.0 ** -23) * scale + 1e-30
     assert bool(((y.double() - ref.double()).abs()[ok] <= bound[ok]).all())
+
+
+# n, cin, cout, h, w: channel tiles with remainders, strips of 32 columns with
+# remainders (vector rows and odd ones), strips that end inside a slice, slices
+# that start inside a strip, one-row images, a single slice
+WGRAD = [(1, 64, 64, 80, 32), (1, 70, 33, 90, 47), (2, 40, 130, 19, 45), (3, 65, 64, 9, 100), (1, 96, 200, 1, 700),
+         (1, 512, 512, 16, 16), (9, 16, 16, 64, 64), (1, 130, 128, 60, 20)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", WGRAD, ids=[f"{s[0]}x{s[1]}->{s[2]}@{s[3]}x{s[4]}" for s in WGRAD])
+def test_wgrad_split_against_fp64(pkg, shape):
+    """The weight gradient on split operands: one truncation of the running
+    sum per 16 pixels and those of the small sums, the slices' additions and the
+    split's roundings, relative to the sum of |x| |dL/dz|; the same bits twice."""
+    from svbrdf_amd import convnet
+    n, cin, cout, h, w = shape
+    assert w >= 16 and 18 * n * cin * cout * h * w >= 1.5e8        # the path under test
+    g = torch.Generator().manual_seed(sum(shape))
+    x, gz = torch.randn((n, cin, h, w), generator=g).to(DEV), torch.randn((n, cout, h, w), generator=g).to(DEV)
+    gw = convnet.conv3x3_wgrad(x, gz, cout)
+    assert torch.equal(gw, convnet.conv3x3_wgrad(x, gz, cout))
+
+    def exact(x, gz):
+        xp, z = F.pad(x.double(), (1, 1, 1, 1)), gz.double().transpose(0, 1).flatten(1)
+        taps = [z @ xp[:, :, a:a + h, b:b + w].transpose(0, 1).flatten(1).t().contiguous()
+                for a in range(3) for b in range(3)]
+        return torch.stack(taps, -1).view(cout, cin, 3, 3)
+
+    chunks = n * h * ((w + 31) // 32)
+    bound = (2 * chunks * (1 + 1 / 32) + 256 + 16) * 2.0 ** -23 * exact(x.abs(), gz.abs())
+    err = (gw.double() - exact(x, gz)).abs()        # a tap that meets no input row is 0 within 0
+    assert bool((err <= bound).all()), float((err / (bound + 1e-300)).max())
+
+
+@pytest.mark.gpu
+def test_wgrad_split_spreads_infinities_like_fp32(pkg):
+    """Non-finite inputs and gradients: the same NaN and signed infinities as a
+    plain convolution's weight gradient in FP64 has, the rest finite."""
+    from svbrdf_amd import convnet
+    x, _, _, _ = _layer((1, 48, 8, 40, 64), 3)
+    gz = torch.randn((1, 80, 40, 64), generator=torch.Generator().manual_seed(4)).to(DEV)
+    x[0, 5, 20, 30], x[0, 40, 39, 63], x[0, 47, 10, 33] = float("inf"), float("nan"), -3.4e38
+    gz[0, 70, 7, 8] = float("-inf")
+    gz[0, :, 9:12, 32:35] *= 2.0 ** -10       # around the large value: finite products
+    gw = convnet.conv3x3_wgrad(x, gz, 80)
+    xp, z = F.pad(x.double(), (1, 1, 1, 1)), gz.double()[0].flatten(1)
+    want = torch.stack([(z[:, None] * xp[0, :, a:a + 40, b:b + 64].flatten(1)[None]).sum(-1)
+                        for a in range(3) for b in range(3)], -1).view(80, 48, 3, 3)
+    assert torch.equal(torch.isnan(gw), torch.isnan(want))
+    assert torch.equal(torch.isinf(gw), torch.isinf(want)) and torch.equal(gw[torch.isinf(gw)].double(), want[torch.isinf(want)])
