@@ -337,8 +337,8 @@ size_t svbrdf_batch_tile_count(const svbrdf_material *materials, int n_materials
 int svbrdf_batch_plan(svbrdf_material *materials, int n_materials, int tile_pixels, unsigned int *order,
                       unsigned int *tile_material, size_t n_tiles);
 
-/* Workspace: per-tile partial sums plus the ticket counter; must be zeroed
- * once before the first step (each step leaves the counter at zero). */
+/* Workspace: per-tile partial sums plus the ticket and arrival counters; must be
+ * zeroed once before the first step (each step leaves the counters at zero). */
 size_t svbrdf_batch_workspace_bytes(size_t n_tiles);
 
 /* Number of blocks that fit on the device at once for a kernel variant

@@ -203,6 +203,36 @@ __device__ __forceinline__ float block_sum(float x, float *lds) {
     return r;
 }
 
+// A block's partial sums of the loss and, with OPT_LIGHT, dL/dP, each in
+// block_sum's order but behind one barrier instead of two each; valid in
+// thread 0.  The caller puts a barrier between this and the next use of lds.
+template <bool OPT_LIGHT>
+__device__ __forceinline__ float4 block_partial(float loss, const float (&gP)[3], float (*lds)[4]) {
+    constexpr int NQ = OPT_LIGHT ? 4 : 1;
+    float x[4] = {loss, gP[0], gP[1], gP[2]};
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) x[q] += __shfl_xor(x[q], off, 64);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+        if (lane == 0) lds[wave][q] = x[q];
+    __syncthreads();
+    float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (threadIdx.x != 0) return r;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) {
+        r.x += lds[w][0];
+        if constexpr (OPT_LIGHT) {
+            r.y += lds[w][1];
+            r.z += lds[w][2];
+            r.w += lds[w][3];
+        }
+    }
+    return r;
+}
+
 // The same for a double over a 256-thread block.
 __device__ __forceinline__ double block_sum_d(double x, double *lds) {
 #pragma unroll
@@ -846,21 +876,22 @@ __device__ __forceinline__ float4 *partial_buffer(void *ws, unsigned nb, unsigne
 // then the wave and the block combine in index order.  Every reader of a
 // step's partials (the next step's block 0, the flush, the light finalize)
 // uses this routine, so they agree to the bit.  Result valid in thread 0.
-template <int NQ, int BLOCK = kBlock>
-__device__ void reduce_partials(const float4 *__restrict__ parts, unsigned n, double (&tot)[NQ],
-                                double (*lds)[BLOCK / 64]) {
+// wave_sums leaves the waves' sums in LDS, behind a barrier.
+template <int NQ, int BLOCK>
+__device__ void wave_sums(const float4 *__restrict__ parts, unsigned n, double (*lds)[BLOCK / 64]) {
     double acc[NQ];
 #pragma unroll
     for (int c = 0; c < NQ; ++c) acc[c] = 0.0;
-    for (unsigned b0 = threadIdx.x; b0 < n; b0 += 4 * BLOCK) {
-        float4 q[4];
+    constexpr int U = 4;   // loads in flight
+    for (unsigned b0 = threadIdx.x; b0 < n; b0 += U * BLOCK) {
+        float4 q[U];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
             const unsigned b = b0 + u * BLOCK;
             q[u] = b < n ? parts[b] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
             acc[0] += q[u].x;
             if constexpr (NQ == 4) { acc[1] += q[u].y; acc[2] += q[u].z; acc[3] += q[u].w; }
         }
@@ -874,6 +905,12 @@ __device__ void reduce_partials(const float4 *__restrict__ parts, unsigned n, do
         if (lane == 0) lds[c][wave] = x;
     }
     __syncthreads();
+}
+
+template <int NQ, int BLOCK = kBlock>
+__device__ void reduce_partials(const float4 *__restrict__ parts, unsigned n, double (&tot)[NQ],
+                                double (*lds)[BLOCK / 64]) {
+    wave_sums<NQ, BLOCK>(parts, n, lds);
 #pragma unroll
     for (int c = 0; c < NQ; ++c) {
         tot[c] = 0.0;
@@ -919,7 +956,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SVBRDF_F
     const float *__restrict__ light, float *__restrict__ lpow, StepConsts c, svbrdf_step_state *st, void *ws,
     float *loss_history, int history_len) {
     constexpr int NPIX = SVBRDF_FUSED_NPIX;
-    __shared__ float lds[kBlock / 64];
+    __shared__ float lds[kBlock / 64][4];
     const unsigned npix = (unsigned)res * (unsigned)res;
     const double count = c.count;
     // d mean / d element, times d out^... / d ln img = 1/2.2 (folded once)
@@ -946,14 +983,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SVBRDF_F
     else
         fused_pixels<LOSS, OPT_LIGHT, false, NPIX, SVBRDF_FUSED_UNROLL>(px, tex, exp_avg, exp_avg_sq, tgt, tps, ps,
                                                                          n_views, cam, light, P, K2, sc, loss, gPs);
-    const float bl = block_sum(loss, lds);
-    float bp[3] = {0.f, 0.f, 0.f};
-    if (OPT_LIGHT) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) bp[c] = block_sum(gPs[c], lds);
-    }
+    const float4 part = block_partial<OPT_LIGHT>(loss, gPs, lds);
     if (threadIdx.x != 0) return;
-    partial_buffer(ws, gridDim.x, t & 1u)[blockIdx.x] = make_float4(bl, bp[0], bp[1], bp[2]);
+    partial_buffer(ws, gridDim.x, t & 1u)[blockIdx.x] = part;
     if constexpr (!OPT_LIGHT) {
         unsigned *counters = static_cast<unsigned *>(ws);
         const unsigned nb = gridDim.x, g = blockIdx.x % kArrivalGroups;
@@ -970,42 +1002,55 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SVBRDF_F
     }
 }
 
-// One block of kFinalizeBlock threads, after a light-optimising step:
-// reduces that step's partials in the fixed order of reduce_partials (at this
-// block size: the light path's only reader), records the loss, takes the
-// light-power Adam step (one param group with the maps, src/svbrdf.py:50)
-// and advances the state.  The next step needs the new light power in every
-// block, so this sits between two step launches; 1,024 threads take the
-// 4,096 partials of a 1024^2 step in one round of loads.
+// One block, after a light-optimising step: reduces that step's partials in
+// the fixed order of reduce_partials, records the loss, takes the light-power
+// Adam step (one param group with the maps, src/svbrdf.py:50) and advances
+// the state.  The next step needs the new light power in every block, so this
+// sits between two step launches and its latency counts.  At most
+// kFinalizeNarrow partials are one round of loads for 256 threads, and fewer
+// waves meet at the barrier; above it 1,024 threads take the 4,096 partials of
+// a 1024^2 step in one round.  The quantities' serial tail is side by side in
+// four lanes.  Light-optimising steps, 9 views, 256^2 / 512^2 / 1024^2: 12.4 /
+// 23.2 / 58.5 us with 1,024 threads, 11.8 / 22.5 / 60.8 with 256; with the
+// blocks' sums behind one barrier (block_partial) 11.1 / 22.0 / 58.6 by this
+// rule.
 constexpr int kFinalizeBlock = 1024;
-template <bool OPT_LIGHT>
-__global__ __launch_bounds__(kFinalizeBlock) void finalize_step_kernel(void *ws, unsigned n_partials, StepConsts k,
-                                                                      float *__restrict__ lpow,
-                                                                      svbrdf_step_state *st, float *loss_history,
-                                                                      int history_len) {
-    constexpr int NQ = OPT_LIGHT ? 4 : 1;
-    __shared__ double lds[NQ][kFinalizeBlock / 64];
+constexpr unsigned kFinalizeNarrow = 1024;
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void finalize_step_kernel(void *ws, unsigned n_partials, StepConsts k,
+                                                               float *__restrict__ lpow, svbrdf_step_state *st,
+                                                               float *loss_history, int history_len) {
+    __shared__ double lds[4][BLOCK / 64];
     const float step_f = st->step;
     const unsigned t = (unsigned)step_f;
-    double tot[NQ];
-    reduce_partials<NQ, kFinalizeBlock>(partial_buffer(ws, n_partials, t & 1u), n_partials, tot, lds);
-    if (threadIdx.x != 0) return;
-    record_loss(st, t + 1, tot[0], k.count, loss_history, history_len);
-    if constexpr (OPT_LIGHT) {
-        // Adam on light_pow with the same scalars as the maps
-        const StepScalars sc = step_scalars(st, k);
-        for (int c = 0; c < 3; ++c) {
+    const StepScalars sc = step_scalars(st, k);   // read before the state moves on
+    const double beta1_pow = st->beta1_pow * k.beta1, beta2_pow = st->beta2_pow * k.beta2;
+    wave_sums<4, BLOCK>(partial_buffer(ws, n_partials, t & 1u), n_partials, lds);
+    const int tid = (int)threadIdx.x;
+    if (tid < 4) {
+        // one quantity per lane, summed and applied side by side
+        double tot = 0.0;
+        for (int w = 0; w < BLOCK / 64; ++w) tot += lds[tid][w];
+        if (tid == 0) {
+            record_loss(st, t + 1, tot, k.count, loss_history, history_len);
+        } else {
+            const int c = tid - 1;
             float pp = lpow[c], mm = st->light_exp_avg[c], vv = st->light_exp_avg_sq[c];
-            const float g = (float)tot[1 + c];
+            const float g = (float)tot;
             adam_update(pp, mm, vv, g, sc.w1, sc.beta2, sc.om_beta2, sc.inv_bc2_sqrt, sc.eps, sc.neg_step);
             lpow[c] = pp;
             st->light_exp_avg[c] = mm;
             st->light_exp_avg_sq[c] = vv;
             st->light_grad[c] = g;
         }
+    } else if (tid == 64) {
+        // another wave: every thread has read what it needs of the state
+        st->step = step_f + 1.0f;
+        st->beta1_pow = beta1_pow;
+        st->beta2_pow = beta2_pow;
+        set_bias_corrections(st);
+        st->pending_step = 0u;
     }
-    advance_step(st, step_f + 1.0f, k.beta1, k.beta2);
-    st->pending_step = 0u;
 }
 
 // One block: records the loss of the last completed step when its partials
@@ -1035,7 +1080,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NPIX == 
     const svbrdf_material *__restrict__ mats, const unsigned *__restrict__ order,
     const unsigned *__restrict__ tile_mat, unsigned n_tiles, int tile_pixels, unsigned *__restrict__ queue,
     float4 *__restrict__ partials, StepConsts c, const svbrdf_step_state *__restrict__ st) {
-    __shared__ float lds[kBlock / 64];
+    __shared__ float lds[kBlock / 64][4];
     __shared__ unsigned s_slot;
     const StepScalars sc = step_scalars(st, c);
     // The ticket is read back through readfirstlane so that the loop exit is a
@@ -1071,16 +1116,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NPIX == 
                                                                    mt.targets_prepared, tps, ps, mt.n_views,
                                                                    mt.camera_pos, mt.light_pos, P, K2, sc, loss, gPs);
         }
-        // block_sum ends with a barrier, so every thread has read s_slot before
-        // thread 0 overwrites it with the next ticket
-        const float bl = block_sum(loss, lds);
-        float bp[3] = {0.f, 0.f, 0.f};
-        if (OPT_LIGHT) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) bp[c] = block_sum(gPs[c], lds);
-        }
+        // behind its barrier every thread has read s_slot, which thread 0
+        // overwrites with the next ticket
+        const float4 part = block_partial<OPT_LIGHT>(loss, gPs, lds);
         if (threadIdx.x == 0) {
-            partials[id] = make_float4(bl, bp[0], bp[1], bp[2]);
+            partials[id] = part;
             s_slot = atomicAdd(queue, 1u);
         }
         __syncthreads();
@@ -1098,7 +1138,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SVBRDF_F
     const svbrdf_material *__restrict__ mats, const unsigned *__restrict__ order,
     const unsigned *__restrict__ tile_mat, float4 *__restrict__ partials, StepConsts c,
     const svbrdf_step_state *__restrict__ st) {
-    __shared__ float lds[kBlock / 64];
+    __shared__ float lds[kBlock / 64][4];
     const StepScalars sc = step_scalars(st, c);
     const unsigned id = order[blockIdx.x];
     const svbrdf_material mt = mats[tile_mat[id]];
@@ -1119,24 +1159,24 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SVBRDF_F
         fused_pixels<LOSS, OPT_LIGHT, false, 1, UNROLL>(px, mt.textures, mt.exp_avg, mt.exp_avg_sq,
                                                         mt.targets_prepared, tps, ps, mt.n_views, mt.camera_pos,
                                                         mt.light_pos, P, K2, sc, loss, gPs);
-    const float bl = block_sum(loss, lds);
-    float bp[3] = {0.f, 0.f, 0.f};
-    if (OPT_LIGHT) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) bp[c] = block_sum(gPs[c], lds);
-    }
-    if (threadIdx.x == 0) partials[id] = make_float4(bl, bp[0], bp[1], bp[2]);
+    const float4 part = block_partial<OPT_LIGHT>(loss, gPs, lds);
+    if (threadIdx.x == 0) partials[id] = part;
 }
 
 // Block m sums material m's tile partials in tile order (fixed, so the loss is
-// bit-reproducible) and records its loss; reads the step count only.  With
+// bit-reproducible), eight loads in flight per thread, and records its loss.
+// The block that arrives last (every block has read the state by then)
+// advances the shared step state and re-arms the counters: bound by latency,
+// so one launch after the step kernel instead of two (six materials of 256^2
+// to 1024^2, an iteration with its step: 133.2 -> 131.7 us).  With
 // OPT_LIGHT it also sums the tiles' dL/dlight_pow and takes material m's
 // Adam step on its light power (one param group with the maps,
 // src/svbrdf.py:50: the maps' step scalars), moments in mt.light_adam.
 template <bool OPT_LIGHT>
 __global__ __launch_bounds__(kBlock) void batch_reduce_kernel(const svbrdf_material *__restrict__ mats,
                                                               const float4 *__restrict__ partials, StepConsts k,
-                                                              const svbrdf_step_state *__restrict__ st,
+                                                              svbrdf_step_state *__restrict__ st,
+                                                              unsigned *__restrict__ queue,
                                                               float *__restrict__ losses,
                                                               float *__restrict__ loss_history, int history_len,
                                                               int n_materials) {
@@ -1146,13 +1186,22 @@ __global__ __launch_bounds__(kBlock) void batch_reduce_kernel(const svbrdf_mater
     double acc[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
-    for (unsigned b = threadIdx.x; b < mt.n_tiles; b += kBlock) {
-        const float4 v = partials[mt.tile_begin + b];
-        acc[0] += (double)v.x;
-        if constexpr (OPT_LIGHT) {
-            acc[1] += (double)v.y;
-            acc[2] += (double)v.z;
-            acc[3] += (double)v.w;
+    constexpr int U = 8;
+    for (unsigned b0 = threadIdx.x; b0 < mt.n_tiles; b0 += U * kBlock) {
+        float4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const unsigned b = b0 + u * kBlock;
+            v[u] = b < mt.n_tiles ? partials[mt.tile_begin + b] : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            acc[0] += (double)v[u].x;
+            if constexpr (OPT_LIGHT) {
+                acc[1] += (double)v[u].y;
+                acc[2] += (double)v[u].z;
+                acc[3] += (double)v[u].w;
+            }
         }
     }
     double tot[NQ];
@@ -1165,27 +1214,25 @@ __global__ __launch_bounds__(kBlock) void batch_reduce_kernel(const svbrdf_mater
     const int t = (int)st->step;   // completed steps before this one
     if (loss_history && t < history_len) loss_history[(size_t)t * n_materials + blockIdx.x] = L;
     if constexpr (OPT_LIGHT) {
-        if (!mt.light_adam) return;
-        const StepScalars sc = step_scalars(st, k);
-        for (int c = 0; c < 3; ++c) {
-            float pp = mt.light_pow[c], mm = mt.light_adam[c], vv = mt.light_adam[3 + c];
-            adam_update(pp, mm, vv, (float)tot[1 + c], sc.w1, sc.beta2, sc.om_beta2, sc.inv_bc2_sqrt, sc.eps,
-                        sc.neg_step);
-            mt.light_pow[c] = pp;
-            mt.light_adam[c] = mm;
-            mt.light_adam[3 + c] = vv;
+        if (mt.light_adam) {
+            const StepScalars sc = step_scalars(st, k);
+            for (int c = 0; c < 3; ++c) {
+                float pp = mt.light_pow[c], mm = mt.light_adam[c], vv = mt.light_adam[3 + c];
+                adam_update(pp, mm, vv, (float)tot[1 + c], sc.w1, sc.beta2, sc.om_beta2, sc.inv_bc2_sqrt, sc.eps,
+                            sc.neg_step);
+                mt.light_pow[c] = pp;
+                mt.light_adam[c] = mm;
+                mt.light_adam[3 + c] = vv;
+            }
         }
     }
-}
-
-// Advances the shared step state and re-arms the ticket counter.
-__global__ void batch_advance_kernel(svbrdf_step_state *__restrict__ st, unsigned *__restrict__ queue, double beta1,
-                                     double beta2) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    st->step = st->step + 1.0f;
-    st->beta1_pow *= beta1;
-    st->beta2_pow *= beta2;
-    set_bias_corrections(st);
+    // nothing above may still be in flight when this block is counted
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    unsigned *arrived = queue + kCounterStride;
+    if (atomicAdd(arrived, 1u) != gridDim.x - 1) return;
+    __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    advance_step(st, (float)t + 1.0f, k.beta1, k.beta2);
     *queue = 0u;
 }
 
@@ -1460,8 +1507,12 @@ int svbrdf_fused_step(float *textures, float *exp_avg, float *exp_avg_sq, const 
 #undef SVBRDF_LAUNCH_STEP
     if ((rc = check_launch("svbrdf_fused_step"))) return rc;
     if (optim_light) {
-        hipLaunchKernelGGL(finalize_step_kernel<true>, dim3(1), dim3(kFinalizeBlock), 0, s, workspace, nb, consts,
-                           light_pow, st, loss_history, history_len);
+        if (nb <= kFinalizeNarrow)
+            hipLaunchKernelGGL(finalize_step_kernel<kBlock>, dim3(1), dim3(kBlock), 0, s, workspace, nb, consts,
+                               light_pow, st, loss_history, history_len);
+        else
+            hipLaunchKernelGGL(finalize_step_kernel<kFinalizeBlock>, dim3(1), dim3(kFinalizeBlock), 0, s, workspace,
+                               nb, consts, light_pow, st, loss_history, history_len);
     }
     return check_launch("svbrdf_fused_step");
 }
@@ -1554,6 +1605,7 @@ int svbrdf_batch_plan(svbrdf_material *materials, int n_materials, int tile_pixe
     return SVBRDF_OK;
 }
 
+// the tiles' partial sums, the ticket counter and, a cache line on, the arrival counter
 size_t svbrdf_batch_workspace_bytes(size_t n_tiles) { return batch_partials_bytes(n_tiles) + 256; }
 
 int svbrdf_batch_max_blocks_per_cu(int loss_mode, int optim_light, int pixels_per_thread, int views_per_trip) {
@@ -1615,12 +1667,10 @@ int svbrdf_batch_step(const svbrdf_material *materials, int n_materials, const u
     if ((rc = check_launch(what))) return rc;
     if (optim_light)
         hipLaunchKernelGGL(batch_reduce_kernel<true>, dim3(n_materials), dim3(kBlock), 0, s, materials, partials,
-                           consts, st, losses, loss_history, history_len, n_materials);
+                           consts, st, queue, losses, loss_history, history_len, n_materials);
     else
         hipLaunchKernelGGL(batch_reduce_kernel<false>, dim3(n_materials), dim3(kBlock), 0, s, materials, partials,
-                           consts, st, losses, loss_history, history_len, n_materials);
-    if ((rc = check_launch(what))) return rc;
-    hipLaunchKernelGGL(batch_advance_kernel, dim3(1), dim3(64), 0, s, st, queue, beta1, beta2);
+                           consts, st, queue, losses, loss_history, history_len, n_materials);
     return check_launch(what);
 }
 
