@@ -27,6 +27,8 @@
 //                         pixels (M = Cout, N = Cin), the nine taps sharing
 //                         the dL/dy operand; wgrad_sum_kernel adds its
 //                         pixel slices.
+//   conv3x3_few_kernel    the same convolution for at most 4 input channels (a
+//                         layer that reads the RGB image), weights in registers.
 //   conv3x3_direct_kernel the same convolution for at most 8 output channels
 //                         (the input gradient of a layer that reads the RGB
 //                         image): input tiles staged in LDS, two pixels per
@@ -556,6 +558,119 @@ void launch_direct(const ConvArgs &a, hipStream_t s) {
     else hipLaunchKernelGGL((conv3x3_direct_kernel<CO, false>), grid, dim3(kThreads), 0, s, a);
 }
 
+// The convolution for CIN <= 4 input channels (a network's first layer, which
+// reads the RGB image): the whole K of 9 CIN products is 5 to 18 steps of
+// v_mfma_f32_32x32x2f32, so there is nothing to stage.  A wave keeps the
+// weights of 64 output channels in registers and walks tiles of 32 consecutive
+// pixels (of the image as one row of H W: no padding on odd widths), whose
+// window it reads straight from the caches, the next tile's loads in flight
+// beside this one's stores.  Bound by those stores (3.3 TB/s) behind 14 us of
+// matrix work.  3 -> 64 channels with ReLU: 9 x 256^2 48.6 us (the staged kernel
+// above 72.4), 1 x 1024^2 88 (117), 1 x 64^2 5.5 (6.9); 4 -> 512 at 8^2 5.3 (6.7):
+// the faster one at every size tried, so it takes all of them.  On the way: 32
+// 64-bit addresses and bias loads per tile 110, scalar weights on the vector ALUs
+// 198.
+constexpr int kFewMaxCin = 4;
+template <int CIN, int ACT>
+__global__ __launch_bounds__(kThreads, 4) void conv3x3_few_kernel(ConvArgs a, int tiles) {
+    __shared__ float4 bias[16];
+    constexpr int K = 9 * CIN, STEPS = (K + 1) / 2;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int half = lane >> 5, col = lane & 31, img = blockIdx.z, co0 = blockIdx.y * 64;
+    const int H = a.h, W = a.w_, HW = H * W;
+    if (threadIdx.x < 64) {
+        const int co = co0 + (int)threadIdx.x;
+        reinterpret_cast<float *>(bias)[threadIdx.x] = a.bias && co < a.cout ? a.bias[co] : 0.0f;
+    }
+    __syncthreads();
+    float wr[STEPS][2];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int k = 2 * s + half, co = co0 + i * 32 + col;
+            const float v = a.w[(size_t)min(k, K - 1) * a.cout + min(co, a.cout - 1)];
+            wr[s][i] = k < K && co < a.cout ? v : 0.0f;
+        }
+    const float *xi = a.x + (size_t)img * CIN * HW;
+    const float *gi = a.gate ? a.gate + (size_t)img * CIN * HW : nullptr;
+    float xv[STEPS];
+    const auto load = [&](int tile) {
+        const int p = min(tile * 32 + col, HW - 1), y = p / W, x = p - y * W;
+        const bool my[3] = {y > 0, true, y + 1 < H}, mx[3] = {x > 0, true, x + 1 < W};
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            // row k = tap * CIN + ci of the packed weights
+            constexpr int last = K - 1;
+            const int k0 = 2 * s, k1 = 2 * s + 1 < K ? 2 * s + 1 : last;
+            const int t0 = k0 / CIN, t1 = k1 / CIN;
+            const int o0 = (k0 % CIN) * HW + (t0 / 3 - 1) * W + t0 % 3 - 1;
+            const int o1 = (k1 % CIN) * HW + (t1 / 3 - 1) * W + t1 % 3 - 1;
+            const bool in = half ? 2 * s + 1 < K && my[t1 / 3] && mx[t1 % 3] : my[t0 / 3] && mx[t0 % 3];
+            // 32 bits of byte offset reach 4 planes of at most 2^28 bytes
+            const unsigned o = in ? (unsigned)(p + (half ? o1 : o0)) * 4u : 0u;   // outside the image: read and not used
+            float v = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(xi) + o);
+            if (gi) {
+                const float g = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(gi) + o);
+                v *= g > 0.0f ? a.gate_pos : a.gate_neg;
+            }
+            xv[s] = in ? v : 0.0f;
+        }
+    };
+    const int stride = gridDim.x * (kThreads / 64);
+    int tile = blockIdx.x * (kThreads / 64) + wave;
+    if (tile < tiles) load(tile);
+    for (; tile < tiles; tile += stride) {
+        v16f acc[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(wr[s][i], xv[s], acc[i], 0, 0, 0);
+        if (tile + stride < tiles) load(tile + stride);
+        const int p = tile * 32 + col;
+        if (p >= HW) continue;
+        // the lane's byte offset from a row's first pixel, at most 5 planes
+        const unsigned off = ((unsigned)p + (unsigned)(half * 4) * (unsigned)HW) * 4u;
+        char *row = reinterpret_cast<char *>(a.y + ((size_t)img * a.cout + co0) * HW);
+        size_t pitch = (size_t)HW * 4;
+        asm volatile("" : "+s"(pitch));   // the rows' addresses are not kept from tile to tile: 64 scalar registers
+        const float nz = a.noise ? a.noise_strength * a.noise[p] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int c = i * 32 + g * 8 + half * 4;
+                const float4 b = bias[c / 4];
+                const float v[4] = {acc[i][4 * g] + nz + b.x, acc[i][4 * g + 1] + nz + b.y,
+                                    acc[i][4 * g + 2] + nz + b.z, acc[i][4 * g + 3] + nz + b.w};
+#pragma unroll
+                for (int r = 0; r < 4; ++r, row += pitch)
+                    if (co0 + c + r < a.cout) *reinterpret_cast<float *>(row + off) = activate(v[r], ACT);
+                row += 4 * pitch;   // the other half's
+            }
+    }
+}
+
+template <int CIN>
+void launch_few(const ConvArgs &a, hipStream_t s) {
+    const int tiles = (a.h * a.w_ + 31) / 32, co_groups = (a.cout + 63) / 64;
+    // as many waves as the device holds (four per SIMD), each walking its tiles
+    const long long want = (long long)kComputeUnits * 4 / ((long long)a.n * co_groups) + 1;
+    const int blocks = (int)std::min<long long>((tiles + 3) / 4, want);
+    const dim3 grid((unsigned)blocks, (unsigned)co_groups, (unsigned)a.n);
+    if (a.act == SVBRDF_ACT_RELU)
+        hipLaunchKernelGGL((conv3x3_few_kernel<CIN, SVBRDF_ACT_RELU>), grid, dim3(kThreads), 0, s, a, tiles);
+    else if (a.act == SVBRDF_ACT_LRELU)
+        hipLaunchKernelGGL((conv3x3_few_kernel<CIN, SVBRDF_ACT_LRELU>), grid, dim3(kThreads), 0, s, a, tiles);
+    else
+        hipLaunchKernelGGL((conv3x3_few_kernel<CIN, SVBRDF_ACT_NONE>), grid, dim3(kThreads), 0, s, a, tiles);
+}
+
 // ---------------------------------------------------------------------------
 // Weight gradient: dL/dw[co][ci][t] = sum over images and pixels p of
 // gz[co][p] x[ci][p + shift(t)] (gz = dL/d(pre-activation), zero padding).
@@ -906,7 +1021,7 @@ constexpr int kMinChunksPerSlice = 2;
 // How one convolution runs: the tile shape, the tiling of the image and the
 // K split.  The workspace query and the launch share it.
 struct ConvPlan {
-    bool direct;
+    bool direct, few;
     int bm, bn, tw, th, tiles_x, tiles_y, co_tiles;
     int slices, cps;
     size_t part_floats;   // workspace floats (0 without a K split)
@@ -940,6 +1055,10 @@ ConvPlan plan_conv(int n, int cin, int h, int w, int cout) {
     best.slices = 1;
     if (cout <= kDirectMaxCout) {
         best.direct = true;
+        return best;
+    }
+    if (cin <= kFewMaxCin) {
+        best.few = true;
         return best;
     }
     const int n_chunks = (cin + kKC - 1) / kKC;
@@ -1158,6 +1277,15 @@ static int run_conv(const char *what, ConvArgs a, void *workspace, size_t worksp
             case 6: launch_direct<6>(a, s); break;
             case 7: launch_direct<7>(a, s); break;
             default: launch_direct<8>(a, s); break;
+        }
+        return check_launch(what);
+    }
+    if (p.few) {
+        switch (a.cin) {
+            case 1: launch_few<1>(a, s); break;
+            case 2: launch_few<2>(a, s); break;
+            case 3: launch_few<3>(a, s); break;
+            default: launch_few<4>(a, s); break;
         }
         return check_launch(what);
     }
