@@ -464,6 +464,14 @@ size_t svbrdf_conv3x3_split_workspace_bytes(int n, int cin, int height, int widt
 int svbrdf_conv3x3_split(const float *x, int n, int cin, int height, int width, const void *split, int cout,
                          const float *bias, const float *noise, float noise_strength, int activation, float *y,
                          void *workspace, size_t workspace_bytes, void *stream);
+/* svbrdf_conv3x3 (split null: weights in packed) or svbrdf_conv3x3_split, with a
+ * second copy of the output times tap_scale written to tap [n, cout, height,
+ * width] beside y: a feature map's slice of a weighted feature vector.
+ * Workspace: the query of the path taken. */
+int svbrdf_conv3x3_tapped(const float *x, int n, int cin, int height, int width, const float *packed,
+                          const void *split, int cout, const float *bias, const float *noise, float noise_strength,
+                          int activation, float *y, float *tap, float tap_scale, void *workspace,
+                          size_t workspace_bytes, void *stream);
 int svbrdf_conv3x3_input_grad_split(const float *grad_y, const float *y, int activation, int n, int cout, int height,
                                     int width, const void *split_t, int cin, float *grad_x, void *workspace,
                                     size_t workspace_bytes, void *stream);

@@ -105,6 +105,9 @@ SIGNATURES = {
     "svbrdf_conv3x3_split": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp,
                                             ctypes.c_int, _vp, _vp, ctypes.c_float, ctypes.c_int, _vp, _vp,
                                             ctypes.c_size_t, _vp]),
+    "svbrdf_conv3x3_tapped": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp,
+                                             ctypes.c_int, _vp, _vp, ctypes.c_float, ctypes.c_int, _vp, _vp,
+                                             ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
     "svbrdf_conv3x3_input_grad_split": (ctypes.c_int, [_vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                                        ctypes.c_int, ctypes.c_int, _vp, ctypes.c_int, _vp, _vp,
                                                        ctypes.c_size_t, _vp]),

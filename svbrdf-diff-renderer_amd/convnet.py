@@ -103,9 +103,11 @@ def conv3x3_packed(x, packed, cout, bias=None, noise=None, noise_strength=0.0, a
     return _conv3x3(x, packed, split, cin, cout, bias, noise, noise_strength, act)
 
 
-def _conv3x3(x, packed, split, cin, cout, bias=None, noise=None, noise_strength=0.0, act="none"):
+def _conv3x3(x, packed, split, cin, cout, bias=None, noise=None, noise_strength=0.0, act="none", tap=None,
+             tap_scale=1.0):
     """conv3x3_packed on the split weights, or on the packed ones where those
-    are None; cin, cout: the weights'."""
+    are None; cin, cout: the weights'.  tap: a flat tensor of the output's
+    size that receives tap_scale times it."""
     x = x.contiguous()
     _check(x, "x")
     n, channels, h, w = (int(s) for s in x.shape)
@@ -125,6 +127,15 @@ def _conv3x3(x, packed, split, cin, cout, bias=None, noise=None, noise_strength=
     kind = "svbrdf_conv3x3" if split is None else "svbrdf_conv3x3_split"
     ws_bytes = int(_lib.query(f"{kind}_workspace_bytes", n, cin, h, w, cout))
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
+    if tap is not None:
+        _check(tap, "tap")
+        if tap.numel() != y.numel() or tap.device != x.device or not tap.is_contiguous():
+            raise ValueError(f"tap must hold {y.numel()} contiguous values on {x.device}, got {tap.numel()} on "
+                             f"{tap.device}")
+        _lib.call("svbrdf_conv3x3_tapped", _lib.ptr(x), n, cin, h, w, _lib.ptr(packed), _lib.ptr(split), cout,
+                  _lib.ptr(bias), _lib.ptr(noise), float(noise_strength), ACT[act], _lib.ptr(y), _lib.ptr(tap),
+                  float(tap_scale), _lib.ptr(ws), ws_bytes, _lib.stream_handle(x.device))
+        return y
     _lib.call(kind, _lib.ptr(x), n, cin, h, w, _lib.ptr(packed if split is None else split), cout, _lib.ptr(bias),
               _lib.ptr(noise), float(noise_strength), ACT[act], _lib.ptr(y), _lib.ptr(ws), ws_bytes,
               _lib.stream_handle(x.device))
@@ -462,10 +473,10 @@ def avgpool2(x):
 
 class _FrozenConvFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, layer):
+    def forward(ctx, x, layer, tap=None, tap_scale=1.0):
         n, _, h, w = x.shape
         split = layer.split if _takes_split(n, layer.cin, h, w, layer.cout) else None   # None below 32 channels
-        y = _conv3x3(x, layer.packed, split, layer.cin, layer.cout, layer.bias, None, 0.0, layer.act)
+        y = _conv3x3(x, layer.packed, split, layer.cin, layer.cout, layer.bias, None, 0.0, layer.act, tap, tap_scale)
         ctx.save_for_backward(y)
         ctx.layer = layer
         return y
@@ -476,7 +487,7 @@ class _FrozenConvFunction(torch.autograd.Function):
         layer = ctx.layer
         n, cout, h, w = y.shape
         split_t = layer.split_t if _takes_split(n, cout, h, w, layer.cin) else None
-        return _input_grad(grad_y, y, layer.packed_t, split_t, layer.cin, layer.act), None
+        return _input_grad(grad_y, y, layer.packed_t, split_t, layer.cin, layer.act), None, None, None
 
 
 class Conv3x3(torch.nn.Module):
@@ -503,5 +514,11 @@ class Conv3x3(torch.nn.Module):
             self.split = _split_packed(self.packed, both[:sizes[0]])
             self.split_t = _split_packed(self.packed_t, both[sizes[0]:])
 
-    def forward(self, x):
-        return _FrozenConvFunction.apply(x, self)
+    def forward(self, x, tap=None, tap_scale=1.0):
+        """The layer; tap: a flat tensor that also receives tap_scale times
+        the output, outside autograd only."""
+        if tap is None:
+            return _FrozenConvFunction.apply(x, self)
+        if torch.is_grad_enabled() and x.requires_grad:
+            raise ValueError("tap is written outside autograd: not with an input that requires a gradient")
+        return _FrozenConvFunction.apply(x, self, tap, tap_scale)

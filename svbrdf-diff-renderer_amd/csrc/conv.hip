@@ -52,6 +52,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "conv_common.hpp"
 
@@ -420,6 +421,7 @@ __global__ __launch_bounds__(kThreads) void conv3x3_mfma_kernel(ConvArgs a) {
     // and column n = lane % 32 of that 32 x 32 tile.  A K slice stores its raw
     // partial sums instead.
     float *yi = a.part ? a.part + ((size_t)slice * a.n + img) * a.cout * HW : a.y + (size_t)img * a.cout * HW;
+    float *ti = a.tap && !a.part ? a.tap + (size_t)img * a.cout * HW : nullptr;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         const int nn = wn * (BN / 2) + j * 32 + (lane & 31);
@@ -433,7 +435,9 @@ __global__ __launch_bounds__(kThreads) void conv3x3_mfma_kernel(ConvArgs a) {
             for (int r = 0; r < 16; ++r) {
                 const int co = co0 + wm * (BM / 2) + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
                 if (co >= a.cout) continue;
-                yi[(size_t)co * HW + p] = a.part ? acc[i][j][r] : finish(a, acc[i][j][r], co, p);
+                const float v = a.part ? acc[i][j][r] : finish(a, acc[i][j][r], co, p);
+                yi[(size_t)co * HW + p] = v;
+                if (ti) ti[(size_t)co * HW + p] = v * a.tap_scale;
             }
         }
     }
@@ -468,6 +472,15 @@ __global__ __launch_bounds__(kThreads) void conv_split_sum_kernel(ConvArgs a) {
 #pragma unroll
     for (int i = 0; i < VEC; ++i) v[i] = finish(a, v[i], co, p + i);
     *reinterpret_cast<vec *>(a.y + e) = v;
+    if (a.tap) *reinterpret_cast<vec *>(a.tap + e) = v * a.tap_scale;
+}
+
+// one output through the epilogue, and its second copy
+__device__ __forceinline__ void store_one(const ConvArgs &a, float acc, int co, int img, size_t p) {
+    const size_t e = ((size_t)img * a.cout + co) * ((size_t)a.h * a.w_) + p;
+    const float v = finish(a, acc, co, p);
+    a.y[e] = v;
+    if (a.tap) a.tap[e] = v * a.tap_scale;
 }
 
 // Direct convolution for Cout = CO <= 8: a 64 x 8 pixel block, two
@@ -539,13 +552,12 @@ __global__ __launch_bounds__(kThreads) void conv3x3_direct_kernel(ConvArgs a) {
     }
     const int xx = bx0 + tx, y0 = by0 + ty;
     if (xx >= W || y0 >= H) return;
-    float *yi = a.y + (size_t)img * CO * HW;
     const size_t p0 = (size_t)y0 * W + xx;
 #pragma unroll
-    for (int co = 0; co < CO; ++co) yi[(size_t)co * HW + p0] = finish(a, acc0[co], co, p0);
+    for (int co = 0; co < CO; ++co) store_one(a, acc0[co], co, img, p0);
     if (y0 + 1 < H) {
 #pragma unroll
-        for (int co = 0; co < CO; ++co) yi[(size_t)co * HW + p0 + W] = finish(a, acc1[co], co, p0 + W);
+        for (int co = 0; co < CO; ++co) store_one(a, acc1[co], co, img, p0 + W);
     }
 }
 
@@ -636,23 +648,30 @@ __global__ __launch_bounds__(kThreads, 4) void conv3x3_few_kernel(ConvArgs a, in
         if (p >= HW) continue;
         // the lane's byte offset from a row's first pixel, at most 5 planes
         const unsigned off = ((unsigned)p + (unsigned)(half * 4) * (unsigned)HW) * 4u;
-        char *row = reinterpret_cast<char *>(a.y + ((size_t)img * a.cout + co0) * HW);
-        size_t pitch = (size_t)HW * 4;
-        asm volatile("" : "+s"(pitch));   // the rows' addresses are not kept from tile to tile: 64 scalar registers
         const float nz = a.noise ? a.noise_strength * a.noise[p] : 0.0f;
+        const auto store = [&](float *out, auto scaled) {
+            char *row = reinterpret_cast<char *>(out + ((size_t)img * a.cout + co0) * HW);
+            size_t pitch = (size_t)HW * 4;
+            asm volatile("" : "+s"(pitch));   // the rows' addresses are not kept from tile to tile: 64 scalar registers
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int c = i * 32 + g * 8 + half * 4;
-                const float4 b = bias[c / 4];
-                const float v[4] = {acc[i][4 * g] + nz + b.x, acc[i][4 * g + 1] + nz + b.y,
-                                    acc[i][4 * g + 2] + nz + b.z, acc[i][4 * g + 3] + nz + b.w};
+                for (int g = 0; g < 4; ++g) {
+                    const int c = i * 32 + g * 8 + half * 4;
+                    const float4 b = bias[c / 4];
+                    const float v[4] = {acc[i][4 * g] + nz + b.x, acc[i][4 * g + 1] + nz + b.y,
+                                        acc[i][4 * g + 2] + nz + b.z, acc[i][4 * g + 3] + nz + b.w};
 #pragma unroll
-                for (int r = 0; r < 4; ++r, row += pitch)
-                    if (co0 + c + r < a.cout) *reinterpret_cast<float *>(row + off) = activate(v[r], ACT);
-                row += 4 * pitch;   // the other half's
-            }
+                    for (int r = 0; r < 4; ++r, row += pitch) {
+                        const float u = activate(v[r], ACT);
+                        if (co0 + c + r < a.cout)
+                            *reinterpret_cast<float *>(row + off) = decltype(scaled)::value ? u * a.tap_scale : u;
+                    }
+                    row += 4 * pitch;   // the other half's
+                }
+        };
+        store(a.y, std::false_type{});
+        if (a.tap) store(a.tap, std::true_type{});
     }
 }
 
@@ -1158,11 +1177,54 @@ namespace svbrdf_internal {
 
 void launch_split_sum(const ConvArgs &a, hipStream_t s) {
     const size_t total = (size_t)a.n * a.cout * a.h * a.w_;
-    const bool vec = (size_t)a.h * a.w_ % 4 == 0 && (((uintptr_t)a.part | (uintptr_t)a.y) & 15u) == 0;
+    const bool vec = (size_t)a.h * a.w_ % 4 == 0 && (((uintptr_t)a.part | (uintptr_t)a.y | (uintptr_t)a.tap) & 15u) == 0;
     const size_t threads = vec ? total / 4 : total;
     const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
     if (vec) hipLaunchKernelGGL(conv_split_sum_kernel<4>, grid, dim3(kThreads), 0, s, a);
     else hipLaunchKernelGGL(conv_split_sum_kernel<1>, grid, dim3(kThreads), 0, s, a);
+}
+
+int run_conv(const char *what, ConvArgs a, void *workspace, size_t workspace_bytes, hipStream_t s) {
+    if (!conv_shape_ok(a.n, a.cin, a.h, a.w_, a.cout))
+        return fail(SVBRDF_ESHAPE, "%s: n=%d cin=%d cout=%d height=%d width=%d", what, a.n, a.cin, a.cout, a.h,
+                    a.w_);
+    if (a.act < SVBRDF_ACT_NONE || a.act > SVBRDF_ACT_LRELU)
+        return fail(SVBRDF_EINVAL, "%s: unknown activation %d", what, a.act);
+    const ConvPlan p = plan_conv(a.n, a.cin, a.h, a.w_, a.cout);
+    const size_t need = p.part_floats * sizeof(float);
+    if (need && (!workspace || workspace_bytes < need))
+        return fail(SVBRDF_ESPACE, "%s: workspace of %zu bytes, this shape needs %zu "
+                    "(svbrdf_conv3x3_workspace_bytes)", what, workspace ? workspace_bytes : (size_t)0, need);
+    a.part = p.slices > 1 ? (float *)workspace : nullptr;
+    a.tw = p.tw; a.th = p.th; a.tiles_x = p.tiles_x; a.slices = p.slices; a.cps = p.cps;
+    if (p.direct) {
+        switch (a.cout) {
+            case 1: launch_direct<1>(a, s); break;
+            case 2: launch_direct<2>(a, s); break;
+            case 3: launch_direct<3>(a, s); break;
+            case 4: launch_direct<4>(a, s); break;
+            case 5: launch_direct<5>(a, s); break;
+            case 6: launch_direct<6>(a, s); break;
+            case 7: launch_direct<7>(a, s); break;
+            default: launch_direct<8>(a, s); break;
+        }
+        return check_launch(what);
+    }
+    if (p.few) {
+        switch (a.cin) {
+            case 1: launch_few<1>(a, s); break;
+            case 2: launch_few<2>(a, s); break;
+            case 3: launch_few<3>(a, s); break;
+            default: launch_few<4>(a, s); break;
+        }
+        return check_launch(what);
+    }
+    if (p.bm == 128 && p.bn == 128) launch_mfma<128, 128>(a, p, s);
+    else if (p.bm == 128) launch_mfma<128, 64>(a, p, s);
+    else if (p.bn == 128) launch_mfma<64, 128>(a, p, s);
+    else launch_mfma<64, 64>(a, p, s);
+    if (p.slices > 1) launch_split_sum(a, s);
+    return check_launch(what);
 }
 
 ConvArgs input_grad_args(const float *grad_y, const float *y, int activation, int n, int cout, int height, int width,
@@ -1252,49 +1314,6 @@ int svbrdf_conv3x3_modulation_grad(const float *weight, int cout, int cin, const
 size_t svbrdf_conv3x3_workspace_bytes(int n, int cin, int height, int width, int cout) {
     if (!conv_shape_ok(n, cin, height, width, cout)) return 0;
     return plan_conv(n, cin, height, width, cout).part_floats * sizeof(float);
-}
-
-static int run_conv(const char *what, ConvArgs a, void *workspace, size_t workspace_bytes, hipStream_t s) {
-    if (!conv_shape_ok(a.n, a.cin, a.h, a.w_, a.cout))
-        return fail(SVBRDF_ESHAPE, "%s: n=%d cin=%d cout=%d height=%d width=%d", what, a.n, a.cin, a.cout, a.h,
-                    a.w_);
-    if (a.act < SVBRDF_ACT_NONE || a.act > SVBRDF_ACT_LRELU)
-        return fail(SVBRDF_EINVAL, "%s: unknown activation %d", what, a.act);
-    const ConvPlan p = plan_conv(a.n, a.cin, a.h, a.w_, a.cout);
-    const size_t need = p.part_floats * sizeof(float);
-    if (need && (!workspace || workspace_bytes < need))
-        return fail(SVBRDF_ESPACE, "%s: workspace of %zu bytes, this shape needs %zu "
-                    "(svbrdf_conv3x3_workspace_bytes)", what, workspace ? workspace_bytes : (size_t)0, need);
-    a.part = p.slices > 1 ? (float *)workspace : nullptr;
-    a.tw = p.tw; a.th = p.th; a.tiles_x = p.tiles_x; a.slices = p.slices; a.cps = p.cps;
-    if (p.direct) {
-        switch (a.cout) {
-            case 1: launch_direct<1>(a, s); break;
-            case 2: launch_direct<2>(a, s); break;
-            case 3: launch_direct<3>(a, s); break;
-            case 4: launch_direct<4>(a, s); break;
-            case 5: launch_direct<5>(a, s); break;
-            case 6: launch_direct<6>(a, s); break;
-            case 7: launch_direct<7>(a, s); break;
-            default: launch_direct<8>(a, s); break;
-        }
-        return check_launch(what);
-    }
-    if (p.few) {
-        switch (a.cin) {
-            case 1: launch_few<1>(a, s); break;
-            case 2: launch_few<2>(a, s); break;
-            case 3: launch_few<3>(a, s); break;
-            default: launch_few<4>(a, s); break;
-        }
-        return check_launch(what);
-    }
-    if (p.bm == 128 && p.bn == 128) launch_mfma<128, 128>(a, p, s);
-    else if (p.bm == 128) launch_mfma<128, 64>(a, p, s);
-    else if (p.bn == 128) launch_mfma<64, 128>(a, p, s);
-    else launch_mfma<64, 64>(a, p, s);
-    if (p.slices > 1) launch_split_sum(a, s);
-    return check_launch(what);
 }
 
 int svbrdf_conv3x3(const float *x, int n, int cin, int height, int width, const float *packed, int cout,

@@ -34,6 +34,8 @@ struct ConvArgs {
     const float *gate;
     float gate_pos, gate_neg;
     float *y;             // [N, Cout, H, W]
+    float *tap;           // a second copy of y, times tap_scale, or null
+    float tap_scale;
     float *part;          // [slices][N, Cout, H, W] partial sums when K is split, else null
     int n, cin, cout, h, w_;
     int tw, th, tiles_x;  // pixel tile: th rows x tw columns
@@ -66,6 +68,10 @@ inline bool conv_shape_ok(int n, int cin, int height, int width, int cout) {
 
 // Adds the K slices' partial sums a.part in slice order and applies the epilogue (conv.hip).
 __attribute__((visibility("hidden"))) void launch_split_sum(const ConvArgs &a, hipStream_t s);
+
+// Checks, plans and launches a convolution on the fp32 instruction (conv.hip).
+__attribute__((visibility("hidden"))) int run_conv(const char *what, ConvArgs a, void *workspace,
+                                                   size_t workspace_bytes, hipStream_t s);
 
 // Fills the epilogue-independent arguments of an input-gradient call (conv.hip).
 __attribute__((visibility("hidden"))) ConvArgs input_grad_args(const float *grad_y, const float *y, int activation,

@@ -271,7 +271,7 @@ __device__ __forceinline__ float split_weight(const uint4 *w, int groups, int k_
 // Element r of MFMA tile (i, j): row 8 (r / 4) + 4 (lane / 32) + r % 4, column
 // lane % 32.  ACT: the activation, or kPartial for a K slice's raw sums.
 constexpr int kPartial = -1;
-template <int ACT>
+template <int ACT, bool TAP = false>
 __device__ __forceinline__ void store_rows(const ConvArgs &a, float *out, int com, const int (&oy)[2],
                                            const int (&ox)[2], const v16f (&acc)[2][2]) {
     const int half = ((threadIdx.x >> 5) & 1) * 4;
@@ -295,20 +295,27 @@ __device__ __forceinline__ void store_rows(const ConvArgs &a, float *out, int co
                     v = v + nz;
                     if (a.bias) v = v + a.bias[row + half];
                     v = activate(v, ACT);
+                    if (TAP) v = v * a.tap_scale;
                 }
                 *reinterpret_cast<float *>(reinterpret_cast<char *>(out + (size_t)row * HW) + off) = v;
             }
     }
 }
 
+template <int ACT>
+__device__ __forceinline__ void store_outputs(const ConvArgs &a, size_t first, int com, const int (&oy)[2],
+                                              const int (&ox)[2], const v16f (&acc)[2][2]) {
+    store_rows<ACT>(a, a.y + first, com, oy, ox, acc);
+    if (a.tap) store_rows<ACT, true>(a, a.tap + first, com, oy, ox, acc);
+}
+
 __device__ __forceinline__ void store_tile(const ConvArgs &a, int img, int slice, int com, const int (&oy)[2],
                                            const int (&ox)[2], const v16f (&acc)[2][2]) {
     const size_t image = (size_t)a.cout * a.h * a.w_;
-    float *y = a.y + img * image;
     if (a.part) store_rows<kPartial>(a, a.part + ((size_t)slice * a.n + img) * image, com, oy, ox, acc);
-    else if (a.act == SVBRDF_ACT_RELU) store_rows<SVBRDF_ACT_RELU>(a, y, com, oy, ox, acc);
-    else if (a.act == SVBRDF_ACT_LRELU) store_rows<SVBRDF_ACT_LRELU>(a, y, com, oy, ox, acc);
-    else store_rows<SVBRDF_ACT_NONE>(a, y, com, oy, ox, acc);
+    else if (a.act == SVBRDF_ACT_RELU) store_outputs<SVBRDF_ACT_RELU>(a, img * image, com, oy, ox, acc);
+    else if (a.act == SVBRDF_ACT_LRELU) store_outputs<SVBRDF_ACT_LRELU>(a, img * image, com, oy, ox, acc);
+    else store_outputs<SVBRDF_ACT_NONE>(a, img * image, com, oy, ox, acc);
 }
 
 // A wave's 64 x 64 tile again on the fp32 instruction, from the fp32 inputs:
@@ -1025,6 +1032,19 @@ int svbrdf_conv3x3_split(const float *x, int n, int cin, int height, int width, 
     a.x = x; a.bias = bias; a.noise = noise; a.noise_strength = noise_strength; a.act = activation;
     a.y = y; a.n = n; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
     return run_split(what, a, split, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int svbrdf_conv3x3_tapped(const float *x, int n, int cin, int height, int width, const float *packed,
+                          const void *split, int cout, const float *bias, const float *noise, float noise_strength,
+                          int activation, float *y, float *tap, float tap_scale, void *workspace,
+                          size_t workspace_bytes, void *stream) {
+    const char *what = "svbrdf_conv3x3_tapped";
+    if (!x || (!packed && !split) || !y || !tap) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    ConvArgs a{};
+    a.x = x; a.w = packed; a.bias = bias; a.noise = noise; a.noise_strength = noise_strength; a.act = activation;
+    a.y = y; a.tap = tap; a.tap_scale = tap_scale; a.n = n; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
+    return split ? run_split(what, a, split, workspace, workspace_bytes, (hipStream_t)stream)
+                 : run_conv(what, a, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int svbrdf_conv3x3_input_grad_split(const float *grad_y, const float *y, int activation, int n, int cout, int height,

@@ -240,25 +240,47 @@ class VGGLoss(torch.nn.Module):
     def normalize(self, im):
         return (im - self.mean) / self.std
 
-    def _features(self, x):
-        feats = []
+    def _features(self, x, vector=None):
+        """The hooked layers' outputs; with `vector` also their weighted
+        concatenation, which the convolutions write beside their outputs."""
+        feats, at = [], 0
         for step in self.plan:
             if step == "P":
                 x = convnet.avgpool2(x)
                 continue
-            x = self.convs[step](x)
+            if vector is not None and step in self.HOOKS and len(feats) < len(self.weights):
+                size = x.shape[0] * self.convs[step].cout * x.shape[2] * x.shape[3]
+                x = self.convs[step](x, vector[at:at + size], self.weights[len(feats)])
+                at += size
+            else:
+                x = self.convs[step](x)
             if step in self.HOOKS:
                 feats.append(x.flatten())
         return feats
 
+    def _vector(self, x):
+        """An uninitialised feature vector for the images x [N, 3, H, W]."""
+        n, _, h, w = x.shape
+        size, hooks = 0, self.HOOKS[:len(self.weights)]
+        for step in self.plan:
+            if step == "P":
+                h, w = h // 2, w // 2
+            elif step in hooks:
+                size += n * self.convs[step].cout * h * w
+        return torch.empty(size, dtype=torch.float32, device=x.device)
+
     def compute_feature_vector(self, x):
-        return torch.cat([f * w for f, w in zip(self._features(x), self.weights)])
+        if not self.weights or (torch.is_grad_enabled() and x.requires_grad):
+            return torch.cat([f * w for f, w in zip(self._features(x), self.weights)])
+        vector = self._vector(x)
+        self._features(x, vector)
+        return vector
 
     def load(self, im):
         with torch.no_grad():
-            feats = self._features(self.normalize(im))
-            self.im_feature = torch.cat([f * w for f, w in zip(feats, self.weights)])
-            self._targets = feats
+            im = self.normalize(im)
+            self.im_feature = self._vector(im)
+            self._targets = self._features(im, self.im_feature)
 
     def forward(self, x):
         # mean((w_l f_l - w_l t_l)^2) over the concatenated vector, taken per
