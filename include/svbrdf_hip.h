@@ -526,6 +526,17 @@ size_t svbrdf_style_layers_grad_workspace_bytes(const svbrdf_style_layer *layers
 int svbrdf_style_layers_grad(const svbrdf_style_layer *layers, int n_layers, const float *grad_styles, int latent_rows,
                              int dim, float *grad_latent, void *workspace, size_t workspace_bytes, void *stream);
 
+/* The modulated 3x3 convolution of one sample of at most 128 pixels from the
+ * weights [cout, cin, 3, 3] themselves: what svbrdf_conv3x3_pack (style, scale,
+ * demodulate as there) and svbrdf_conv3x3 compute, without packed weights.
+ * weight 16-byte aligned, cin a multiple of 8.  The workspace query gives 0 for
+ * a shape that is not taken. */
+size_t svbrdf_modconv3x3_small_workspace_bytes(int cin, int height, int width, int cout);
+int svbrdf_modconv3x3_small(const float *x, int cin, int height, int width, const float *weight, int cout,
+                            const float *style, float scale, int demodulate, const float *bias, const float *noise,
+                            float noise_strength, int activation, float *y, void *workspace, size_t workspace_bytes,
+                            void *stream);
+
 /* The synthesis network's 1x1 output convolution of one sample with its skip
  * connection (src/higan_models/stylegan2_generator_network.py:340-356): y
  * [cout, height, width] = sum over c of weight[o][c] * (style[c] * scale) *

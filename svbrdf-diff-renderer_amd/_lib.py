@@ -121,6 +121,10 @@ SIGNATURES = {
     "svbrdf_style_layers_grad_workspace_bytes": (ctypes.c_size_t, [_vp, ctypes.c_int, ctypes.c_int]),
     "svbrdf_style_layers_grad": (ctypes.c_int, [_vp, ctypes.c_int, _vp, ctypes.c_int, ctypes.c_int, _vp, _vp,
                                                 ctypes.c_size_t, _vp]),
+    "svbrdf_modconv3x3_small_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 4),
+    "svbrdf_modconv3x3_small": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, ctypes.c_int, _vp,
+                                               ctypes.c_float, ctypes.c_int, _vp, _vp, ctypes.c_float, ctypes.c_int,
+                                               _vp, _vp, ctypes.c_size_t, _vp]),
     "svbrdf_torgb": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, ctypes.c_int, _vp,
                                     ctypes.c_float, _vp, _vp, _vp]),
     "svbrdf_upsample2_blur_adjoint": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp]),

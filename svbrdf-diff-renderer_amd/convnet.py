@@ -103,24 +103,30 @@ def conv3x3_packed(x, packed, cout, bias=None, noise=None, noise_strength=0.0, a
     return _conv3x3(x, packed, split, cin, cout, bias, noise, noise_strength, act)
 
 
-def _conv3x3(x, packed, split, cin, cout, bias=None, noise=None, noise_strength=0.0, act="none", tap=None,
-             tap_scale=1.0):
-    """conv3x3_packed on the split weights, or on the packed ones where those
-    are None; cin, cout: the weights'.  tap: a flat tensor of the output's
-    size that receives tap_scale times it."""
+def _conv_inputs(x, bias, noise):
+    """A convolution's input, bias and noise as the kernels read them."""
     x = x.contiguous()
     _check(x, "x")
-    n, channels, h, w = (int(s) for s in x.shape)
-    if channels != cin:
-        raise ValueError(f"x has {channels} channels, the weights Cin={cin}")
     if bias is not None:
         bias = bias.detach().reshape(-1).contiguous()
         _check(bias, "bias")
     if noise is not None:
         noise = noise.detach().reshape(-1).contiguous()
         _check(noise, "noise")
-        if noise.numel() != h * w:
-            raise ValueError(f"noise must have {h * w} values, got {noise.numel()}")
+        if noise.numel() != x.shape[2] * x.shape[3]:
+            raise ValueError(f"noise must have {x.shape[2] * x.shape[3]} values, got {noise.numel()}")
+    return x, bias, noise
+
+
+def _conv3x3(x, packed, split, cin, cout, bias=None, noise=None, noise_strength=0.0, act="none", tap=None,
+             tap_scale=1.0):
+    """conv3x3_packed on the split weights, or on the packed ones where those
+    are None; cin, cout: the weights'.  tap: a flat tensor of the output's
+    size that receives tap_scale times it."""
+    n, channels, h, w = (int(s) for s in x.shape)
+    if channels != cin:
+        raise ValueError(f"x has {channels} channels, the weights Cin={cin}")
+    x, bias, noise = _conv_inputs(x, bias, noise)
     y = torch.empty((n, cout, h, w), dtype=torch.float32, device=x.device)
     # K-split partial sums of small images (torch's caching allocator makes
     # this a free-list lookup after the first call)
@@ -269,6 +275,27 @@ def modulation_grad(weight, style, scale, demodulate, grad_weight):
     return out
 
 
+def _small_modconv(x, weight, style, scale, demodulate, bias, noise, noise_strength, act):
+    """A modulated convolution of a few pixels from the weights themselves;
+    None for the shapes that pack them (svbrdf_modconv3x3_small takes one
+    sample of at most 128 pixels, channels in eights, aligned weights)."""
+    wt, st = _pack_inputs(weight, style)
+    cout, cin = int(wt.shape[0]), int(wt.shape[1])
+    n, channels, h, w = (int(s) for s in x.shape)
+    if n != 1 or channels != cin or wt.data_ptr() % 16:
+        return None
+    ws_bytes = int(_lib.query("svbrdf_modconv3x3_small_workspace_bytes", cin, h, w, cout))
+    if not ws_bytes:
+        return None
+    x, bias, noise = _conv_inputs(x, bias, noise)
+    y = torch.empty((1, cout, h, w), dtype=torch.float32, device=x.device)
+    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device)
+    _lib.call("svbrdf_modconv3x3_small", _lib.ptr(x), cin, h, w, _lib.ptr(wt), cout, _lib.ptr(st), float(scale),
+              int(bool(demodulate)), _lib.ptr(bias), _lib.ptr(noise), float(noise_strength), ACT[act], _lib.ptr(y),
+              _lib.ptr(ws), ws_bytes, _lib.stream_handle(x.device))
+    return y
+
+
 class ModConv3x3Function(torch.autograd.Function):
     """The modulated 3x3 convolution of a StyleGAN2 block (batch 1):
     y = act(conv3x3(x, w') + noise_strength * noise + bias) with
@@ -286,8 +313,10 @@ class ModConv3x3Function(torch.autograd.Function):
                              "modulated weights to train it")
         n, _, h, w = x.shape
         cout, cin = (int(s) for s in weight.shape[:2])
-        y = _conv3x3(x, *_pack_for(n, h, w, weight, style, scale, demodulate), cin, cout, bias, noise,
-                     noise_strength, act)
+        y = _small_modconv(x, weight, style, scale, demodulate, bias, noise, noise_strength, act)
+        if y is None:
+            y = _conv3x3(x, *_pack_for(n, h, w, weight, style, scale, demodulate), cin, cout, bias, noise,
+                         noise_strength, act)
         ctx.save_for_backward(x, style, weight, noise, y)
         ctx.scale, ctx.demodulate = float(scale), bool(demodulate)
         ctx.noise_strength, ctx.act = float(noise_strength), act

@@ -7,6 +7,10 @@
 //   style_kernel          every layer's style, one matrix-vector product per
 //                         layer, in one launch; style_grad_kernel and
 //                         style_grad_sum_kernel: dL/dlatent.
+//   modconv_small_kernel  a modulated 3x3 convolution of at most 128 pixels
+//                         straight from the network's weights, and
+//                         modconv_small_sum_kernel: its K slices' sum with
+//                         the demodulation and the epilogue.
 //   torgb_kernel          the 1x1 convolution to the output channels with its
 //                         style, plus the x2 upsampled skip image.
 #include <hip/hip_runtime.h>
@@ -14,11 +18,9 @@
 #include <algorithm>
 #include <cstdint>
 
-#include "common.hpp"
-#include "../../include/svbrdf_hip.h"
+#include "conv_common.hpp"
 
-using svbrdf_internal::check_launch;
-using svbrdf_internal::fail;
+using namespace svbrdf_internal;
 
 namespace {
 
@@ -211,6 +213,171 @@ int check_layers(const char *what, const svbrdf_style_layer *layers, int n_layer
     return SVBRDF_OK;
 }
 
+// ---------------------------------------------------------------------------
+// The modulated 3x3 convolution of the generator's first layers (4 x 4 and
+// 8 x 8 pixels, 512 channels).  There the weights are the work: packing them
+// with the style reads and writes all of them before the convolution reads
+// them again.  Here a lane's weights go from the [Cout][Cin][3][3] layout
+// straight to the MFMA's operand, 16 bytes along K = Cin x 9 at a time (lane
+// half h takes the k = 8 q + 4 h + j of step (q, j)), times scale and style in
+// the packing's order, and the squares for the demodulation factor are summed
+// on the way; the factor multiplies the sums instead of the weights.  Input
+// channels are staged in LDS with a one-pixel halo.  Up to 64 pixels the block's
+// four waves split K and add up through LDS, above that they split the pixels.
+// K is split over the blocks too; modconv_small_sum_kernel adds the slices.
+// Bound by the latency of one or a few rounds (weights, staging, 36 steps).
+// 512 -> 512, this path / packed: 4 x 4 10.8 / 29.0 us, 8 x 8 15.9 / 29.7, 11 x 11
+// 24.7 / 36.0; 256 -> 256 at 4 x 4 9.7 / 17.9, 96 -> 96 at 8 x 8 13.9 / 13.8. Its
+// redundant weight loads grow with the pixels and the packed path's do not: at
+// 16 x 16 37.1 / 39.2 in a loop and no gain between other kernels, so it ends at
+// 128. Prefetching the next round's weights or 512 blocks: no gain.
+constexpr int kSmallMaxPixels = 128;
+constexpr int kSmallUnit = 8;          // input channels of a wave's round: 72 products, 9 x 16 bytes
+constexpr int kSmallBlocks = 256;
+
+struct SmallArgs {
+    const float *x, *w, *style;
+    float scale;
+    int cin, cout, h, w_, rounds, slices;   // rounds: per slice
+    float *part, *squares;                  // [slices][Cout][H W], [slices][Cout]
+};
+
+template <int NT, bool SPLITK>
+__global__ __launch_bounds__(256) void modconv_small_kernel(SmallArgs a) {
+    constexpr int CI = SPLITK ? 4 * kSmallUnit : kSmallUnit;   // channels staged a round
+    constexpr int HALO = SPLITK ? 3 * 66 : 3 * 130;            // the largest (h + 2) (w + 2)
+    __shared__ float xs[CI * HALO];
+    __shared__ float sq4[4][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31, co0 = blockIdx.x * 32, slice = blockIdx.y;
+    const int H = a.h, W = a.w_, P = H * W, w2 = W + 2, PH = (H + 2) * w2;
+    const float *wrow = a.w + (size_t)min(co0 + col, a.cout - 1) * a.cin * 9;
+    const int unit0 = SPLITK ? wave * kSmallUnit : 0;          // the wave's channels of a round
+    int base[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int p = min(((SPLITK ? 0 : wave * NT) + n) * 32 + col, P - 1);
+        base[n] = unit0 * PH + p / W * w2 + p % W;
+    }
+    v16f acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][r] = 0.0f;
+    float sq = 0.0f;
+    const int c_end = min((slice + 1) * a.rounds * CI, a.cin);
+    for (int c0 = slice * a.rounds * CI; c0 < c_end; c0 += CI) {
+        // Cin is a multiple of a unit: a wave's channels all exist or none does
+        const int cu = c0 + unit0;
+        const bool any = cu < a.cin;
+        const float4 *wv = reinterpret_cast<const float4 *>(wrow + (size_t)(any ? cu : 0) * 9) + half;
+        float4 v[9];
+        float st[kSmallUnit];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) v[q] = wv[2 * q];
+#pragma unroll
+        for (int c = 0; c < kSmallUnit; ++c) st[c] = a.style ? a.style[(any ? cu : 0) + c] : 1.0f;
+        for (int e = tid; e < CI * PH; e += 256) {
+            const int c = e / PH, q = e - c * PH, y = q / w2 - 1, x = q % w2 - 1;
+            const bool in = c0 + c < a.cin && y >= 0 && y < H && x >= 0 && x < W;
+            const float t = a.x[in ? (size_t)(c0 + c) * P + y * W + x : 0];
+            xs[e] = in ? t : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const float wq[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int k0 = 8 * q + j, k1 = k0 + 4, c0k = k0 / 9, t0 = k0 % 9, c1k = k1 / 9, t1 = k1 % 9;
+                float m = wq[j] * a.scale * (half ? st[c1k] : st[c0k]);
+                m = any ? m : 0.0f;
+                sq += m * m;
+                const int off = half ? c1k * PH + t1 / 3 * w2 + t1 % 3 : c0k * PH + t0 / 3 * w2 + t0 % 3;
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(m, xs[base[n] + off], acc[n], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    sq += __shfl_xor(sq, 32, 64);
+    if constexpr (SPLITK) {
+        if (half == 0) sq4[wave][col] = sq;
+        if (wave > 0)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) xs[((wave - 1) * NT + n) * 1024 + r * 64 + lane] = acc[n][r];
+        __syncthreads();
+        if (wave > 0) return;
+        sq = ((sq4[0][col] + sq4[1][col]) + sq4[2][col]) + sq4[3][col];
+#pragma unroll
+        for (int v = 0; v < 3; ++v)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[n][r] += xs[(v * NT + n) * 1024 + r * 64 + lane];
+    }
+    if (wave == 0 && half == 0 && co0 + col < a.cout) a.squares[(size_t)slice * a.cout + co0 + col] = sq;
+    // element r of a tile: row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
+    float *out = a.part + (size_t)slice * a.cout * P;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int p = ((SPLITK ? 0 : wave * NT) + n) * 32 + col;
+        if (p >= P) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int co = co0 + (r >> 2) * 8 + half * 4 + (r & 3);
+            if (co < a.cout) out[(size_t)co * P + p] = acc[n][r];
+        }
+    }
+}
+
+// c: the epilogue's arguments; c.part and squares as written above.
+__global__ __launch_bounds__(256) void modconv_small_sum_kernel(ConvArgs c, const float *__restrict__ squares,
+                                                                int demodulate) {
+    const int P = c.h * c.w_, total = c.cout * P, e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= total) return;
+    const int co = e / P;
+    float v = 0.0f, sq = 0.0f;
+    for (int s0 = 0; s0 < c.slices; s0 += 8) {   // eight loads of each in flight
+        float pv[8], qv[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int s = min(s0 + u, c.slices - 1);
+            pv[u] = c.part[(size_t)s * total + e];
+            qv[u] = squares[(size_t)s * c.cout + co];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (s0 + u < c.slices) {
+                v += pv[u];
+                sq += qv[u];
+            }
+        }
+    }
+    if (demodulate) v *= rsqrtf(sq + 1e-8f);
+    c.y[e] = finish(c, v, co, e - co * P);
+}
+
+struct SmallPlan {
+    bool taken;
+    int co_tiles, rounds, slices;
+};
+
+SmallPlan plan_small(int cin, int h, int w, int cout) {
+    SmallPlan p{};
+    if (!conv_shape_ok(1, cin, h, w, cout) || (long long)h * w > kSmallMaxPixels || cin % kSmallUnit) return p;
+    const int ci = h * w <= 64 ? 4 * kSmallUnit : kSmallUnit, total = (cin + ci - 1) / ci;
+    p.taken = true;
+    p.co_tiles = (cout + 31) / 32;
+    const int want = std::max(1, std::min(total, kSmallBlocks / p.co_tiles));
+    p.rounds = (total + want - 1) / want;
+    p.slices = (total + p.rounds - 1) / p.rounds;
+    return p;
+}
+
 }  // namespace
 
 extern "C" {
@@ -252,6 +419,47 @@ int svbrdf_style_layers_grad(const svbrdf_style_layer *layers, int n_layers, con
     if (int rc = check_launch(what)) return rc;
     hipLaunchKernelGGL(style_grad_sum_kernel, dim3((unsigned)(dim + 255) / 256, (unsigned)latent_rows), dim3(256), 0, s,
                        t, (const float *)workspace, dim, grad_latent);
+    return check_launch(what);
+}
+
+size_t svbrdf_modconv3x3_small_workspace_bytes(int cin, int height, int width, int cout) {
+    const SmallPlan p = plan_small(cin, height, width, cout);
+    return p.taken ? (size_t)p.slices * cout * ((size_t)height * width + 1) * sizeof(float) : 0;
+}
+
+int svbrdf_modconv3x3_small(const float *x, int cin, int height, int width, const float *weight, int cout,
+                            const float *style, float scale, int demodulate, const float *bias, const float *noise,
+                            float noise_strength, int activation, float *y, void *workspace, size_t workspace_bytes,
+                            void *stream) {
+    const char *what = "svbrdf_modconv3x3_small";
+    if (!x || !weight || !y || !workspace) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    const size_t need = svbrdf_modconv3x3_small_workspace_bytes(cin, height, width, cout);
+    if (!need)
+        return fail(SVBRDF_ESHAPE, "%s: cin=%d (a multiple of %d) cout=%d height=%d width=%d (at most %d pixels)", what,
+                    cin, kSmallUnit, cout, height, width, kSmallMaxPixels);
+    if (activation < SVBRDF_ACT_NONE || activation > SVBRDF_ACT_LRELU)
+        return fail(SVBRDF_EINVAL, "%s: unknown activation %d", what, activation);
+    if (workspace_bytes < need)
+        return fail(SVBRDF_ESPACE, "%s: workspace of %zu bytes < %zu needed", what, workspace_bytes, need);
+    if ((uintptr_t)weight & 15u) return fail(SVBRDF_EINVAL, "%s: weight must be 16-byte aligned", what);
+    const SmallPlan p = plan_small(cin, height, width, cout);
+    const int P = height * width;
+    SmallArgs a{};
+    a.x = x; a.w = weight; a.style = style; a.scale = scale; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
+    a.rounds = p.rounds; a.slices = p.slices;
+    a.part = (float *)workspace;
+    a.squares = a.part + (size_t)p.slices * cout * P;
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 grid((unsigned)p.co_tiles, (unsigned)p.slices);
+    if (P <= 32) hipLaunchKernelGGL((modconv_small_kernel<1, true>), grid, dim3(256), 0, s, a);
+    else if (P <= 64) hipLaunchKernelGGL((modconv_small_kernel<2, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((modconv_small_kernel<1, false>), grid, dim3(256), 0, s, a);
+    if (int rc = check_launch(what)) return rc;
+    ConvArgs c{};
+    c.bias = bias; c.noise = noise; c.noise_strength = noise_strength; c.act = activation;
+    c.y = y; c.part = a.part; c.cout = cout; c.h = height; c.w_ = width; c.slices = p.slices;
+    hipLaunchKernelGGL(modconv_small_sum_kernel, dim3((unsigned)((cout * P + 255) / 256)), dim3(256), 0, s, c,
+                       (const float *)a.squares, demodulate);
     return check_launch(what);
 }
 
