@@ -1,5 +1,5 @@
 """Convolution layers of the MaterialGAN caller's networks on the matrix-core
-kernels of libsvbrdf_hip.so (csrc/conv.hip).
+kernels of libsvbrdf_hip.so (csrc/conv.hip, conv_split.hip, generator.hip).
 
 * :func:`conv3x3` -- a 3x3 convolution (stride 1, zero padding 1) with the
   fused epilogue of the reference's blocks: ``act(conv + noise_strength *
@@ -16,7 +16,10 @@ kernels of libsvbrdf_hip.so (csrc/conv.hip).
   filter (UpsamplingLayer, stylegan2_generator_network.py:419-479); forward
   and adjoint are HIP kernels.
 * :class:`Conv3x3` -- a frozen 3x3 layer (VGG): weights packed once, in both
-  layouts.
+  layouts; outside autograd it can write a second, scaled copy of its output.
+* :func:`modulated_conv3x3`, :class:`StyleLayersFunction`,
+  :class:`ToRGBFunction` -- a StyleGAN2 block's convolution, every layer's
+  style in one launch, and the output layer with its skip image.
 """
 import numpy as np
 import torch

@@ -31,11 +31,13 @@ The 3x3 convolutions of both networks run on the matrix-core kernels of
 :mod:`svbrdf_amd.convnet` (forward, input gradient and the generator's
 weight gradient, which the latent's gradient needs), with the noise, bias
 and leaky-ReLU epilogue fused; in the generator the style modulation and the
-demodulation happen inside the HIP weight packing, and dL/dstyle comes from
-the HIP modulation backward.  The x2 upsampling is a HIP kernel too.  The
-renderer is :class:`svbrdf_amd.Microfacet` (forward and adjoint kernels).
-The 1x1 toRGB convolutions (9 output channels: plain GEMMs, torch.matmul)
-and the fully connected mapping layers stay torch operations.
+demodulation happen inside the HIP weight packing (or, at a few pixels, inside
+the convolution), and dL/dstyle comes from the HIP modulation backward.  The
+styles of all layers, the 1x1 toRGB convolutions with their skip image and the
+x2 upsampling are HIP kernels too.  The renderer is
+:class:`svbrdf_amd.Microfacet` (forward and adjoint kernels).  The fully
+connected mapping layers stay torch operations, as do the style and toRGB
+layers of weights that are being trained.
 """
 import datetime
 import math

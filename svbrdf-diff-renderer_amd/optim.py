@@ -9,9 +9,10 @@ launch per iteration (:class:`FusedStep`).
 ``FusedStep`` owns the device-resident pieces of one optimisation problem:
 the prepared targets, Adam's moment buffers, the step state and the
 workspace (per-block partial sums of the last step and arrival counters).
-Its ``step()`` is graph-capturable (no host scalars change between
-iterations); ``capture(steps)`` records that many iterations in one HIP
-graph and ``replay()`` runs them.
+``run(n)`` launches n iterations from one library call.  Its ``step()`` is
+graph-capturable (no host scalars change between iterations);
+``capture(steps)`` records that many iterations in one HIP graph and
+``replay()`` runs them.
 """
 import ctypes
 import datetime
