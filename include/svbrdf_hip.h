@@ -472,6 +472,14 @@ int svbrdf_conv3x3_tapped(const float *x, int n, int cin, int height, int width,
                           const void *split, int cout, const float *bias, const float *noise, float noise_strength,
                           int activation, float *y, float *tap, float tap_scale, void *workspace,
                           size_t workspace_bytes, void *stream);
+/* svbrdf_conv3x3_split followed by svbrdf_avgpool2, in one kernel: pool [n,
+ * cout, height / 2, width / 2] receives the 2 x 2 averages of the output, which
+ * itself is written only where y is not null, and its scaled copy only where tap
+ * is not.  For the shapes svbrdf_conv3x3_split_pools accepts; no workspace. */
+int svbrdf_conv3x3_split_pools(int n, int cin, int height, int width, int cout);
+int svbrdf_conv3x3_pooled(const float *x, int n, int cin, int height, int width, const void *split, int cout,
+                          const float *bias, const float *noise, float noise_strength, int activation, float *y,
+                          float *tap, float tap_scale, float *pool, void *stream);
 int svbrdf_conv3x3_input_grad_split(const float *grad_y, const float *y, int activation, int n, int cout, int height,
                                     int width, const void *split_t, int cin, float *grad_x, void *workspace,
                                     size_t workspace_bytes, void *stream);

@@ -105,6 +105,10 @@ SIGNATURES = {
     "svbrdf_conv3x3_split": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp,
                                             ctypes.c_int, _vp, _vp, ctypes.c_float, ctypes.c_int, _vp, _vp,
                                             ctypes.c_size_t, _vp]),
+    "svbrdf_conv3x3_split_pools": (ctypes.c_int, [ctypes.c_int] * 5),
+    "svbrdf_conv3x3_pooled": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp,
+                                             ctypes.c_int, _vp, _vp, ctypes.c_float, ctypes.c_int, _vp, _vp,
+                                             ctypes.c_float, _vp, _vp]),
     "svbrdf_conv3x3_tapped": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp,
                                              ctypes.c_int, _vp, _vp, ctypes.c_float, ctypes.c_int, _vp, _vp,
                                              ctypes.c_float, _vp, ctypes.c_size_t, _vp]),

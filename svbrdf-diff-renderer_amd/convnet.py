@@ -106,6 +106,12 @@ def conv3x3_packed(x, packed, cout, bias=None, noise=None, noise_strength=0.0, a
     return _conv3x3(x, packed, split, cin, cout, bias, noise, noise_strength, act)
 
 
+def _check_tap(tap, x, size):
+    _check(tap, "tap")
+    if tap.numel() != size or tap.device != x.device or not tap.is_contiguous():
+        raise ValueError(f"tap must hold {size} contiguous values on {x.device}, got {tap.numel()} on {tap.device}")
+
+
 def _conv_inputs(x, bias, noise):
     """A convolution's input, bias and noise as the kernels read them."""
     x = x.contiguous()
@@ -137,10 +143,7 @@ def _conv3x3(x, packed, split, cin, cout, bias=None, noise=None, noise_strength=
     ws_bytes = int(_lib.query(f"{kind}_workspace_bytes", n, cin, h, w, cout))
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=x.device) if ws_bytes else None
     if tap is not None:
-        _check(tap, "tap")
-        if tap.numel() != y.numel() or tap.device != x.device or not tap.is_contiguous():
-            raise ValueError(f"tap must hold {y.numel()} contiguous values on {x.device}, got {tap.numel()} on "
-                             f"{tap.device}")
+        _check_tap(tap, x, y.numel())
         _lib.call("svbrdf_conv3x3_tapped", _lib.ptr(x), n, cin, h, w, _lib.ptr(packed), _lib.ptr(split), cout,
                   _lib.ptr(bias), _lib.ptr(noise), float(noise_strength), ACT[act], _lib.ptr(y), _lib.ptr(tap),
                   float(tap_scale), _lib.ptr(ws), ws_bytes, _lib.stream_handle(x.device))
@@ -522,6 +525,25 @@ class _FrozenConvFunction(torch.autograd.Function):
         return _input_grad(grad_y, y, layer.packed_t, split_t, layer.cin, layer.act), None, None, None
 
 
+class _PooledConvFunction(torch.autograd.Function):
+    """Conv3x3 and the 2x2 average pooling behind it, outside autograd: the
+    pooled output, and the output itself where `keep`."""
+
+    @staticmethod
+    def forward(ctx, x, layer, keep, tap, tap_scale):
+        n, channels, h, w = (int(s) for s in x.shape)
+        x, bias, _ = _conv_inputs(x, layer.bias, None)
+        shape = (n, layer.cout, h, w)
+        y = torch.empty(shape, dtype=torch.float32, device=x.device) if keep else None
+        if tap is not None:
+            _check_tap(tap, x, n * layer.cout * h * w)
+        pool = torch.empty((n, layer.cout, h // 2, w // 2), dtype=torch.float32, device=x.device)
+        _lib.call("svbrdf_conv3x3_pooled", _lib.ptr(x), n, channels, h, w, _lib.ptr(layer.split), layer.cout,
+                  _lib.ptr(bias), None, 0.0, ACT[layer.act], _lib.ptr(y), _lib.ptr(tap), float(tap_scale),
+                  _lib.ptr(pool), _lib.stream_handle(x.device))
+        return (pool, y) if keep else pool
+
+
 class Conv3x3(torch.nn.Module):
     """A 3x3 layer with frozen weights [Cout, Cin, 3, 3] and bias [Cout],
     followed by `act`: packed once in the forward and input-gradient layouts."""
@@ -554,3 +576,16 @@ class Conv3x3(torch.nn.Module):
         if torch.is_grad_enabled() and x.requires_grad:
             raise ValueError("tap is written outside autograd: not with an input that requires a gradient")
         return _FrozenConvFunction.apply(x, self, tap, tap_scale)
+
+    def pooled(self, x, keep=True, tap=None, tap_scale=1.0):
+        """(avgpool2(output), output): outside autograd in one kernel where the
+        shape allows it (svbrdf_conv3x3_split_pools), the output then written
+        only where `keep` (else None); tap as in forward."""
+        n, channels, h, w = x.shape
+        if (self.split is None or channels != self.cin or (torch.is_grad_enabled() and x.requires_grad)
+                or not _lib.query("svbrdf_conv3x3_split_pools", n, channels, h, w, self.cout)):
+            y = self(x, tap, tap_scale)
+            return avgpool2(y), y
+        if keep:
+            return _PooledConvFunction.apply(x, self, True, tap, tap_scale)
+        return _PooledConvFunction.apply(x, self, False, tap, tap_scale), None

@@ -36,6 +36,7 @@ struct ConvArgs {
     float *y;             // [N, Cout, H, W]
     float *tap;           // a second copy of y, times tap_scale, or null
     float tap_scale;
+    float *pool;          // the 2 x 2 averages of y [N, Cout, H / 2, W / 2], or null; y may then be null
     float *part;          // [slices][N, Cout, H, W] partial sums when K is split, else null
     int n, cin, cout, h, w_;
     int tw, th, tiles_x;  // pixel tile: th rows x tw columns

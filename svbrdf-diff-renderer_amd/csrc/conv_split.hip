@@ -302,20 +302,56 @@ __device__ __forceinline__ void store_rows(const ConvArgs &a, float *out, int co
     }
 }
 
+// The 2 x 2 averages of a tile of 32 columns: its two MFMA columns are two rows
+// of the image, its even and odd lanes two columns.  Even lanes write, in
+// avgpool2_kernel's order of operations.
 template <int ACT>
-__device__ __forceinline__ void store_outputs(const ConvArgs &a, size_t first, int com, const int (&oy)[2],
+__device__ __forceinline__ void store_pooled(const ConvArgs &a, int img, int com, const int (&oy)[2],
+                                             const int (&ox)[2], const v16f (&acc)[2][2]) {
+    const int half = ((threadIdx.x >> 5) & 1) * 4, hp = a.h / 2, wp = a.w_ / 2;
+    const bool whole = !(threadIdx.x & 1) && oy[1] < a.h && ox[0] + 1 < a.w_;
+    const size_t HP = (size_t)hp * wp;
+    float *out = a.pool + (size_t)img * a.cout * HP;
+    const unsigned off = ((unsigned)(oy[0] / 2 * wp + ox[0] / 2) + (unsigned)half * (unsigned)HP) * 4u;
+    float nz[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        if (a.noise && oy[j] < a.h && ox[j] < a.w_) nz[j] = a.noise_strength * a.noise[oy[j] * a.w_ + ox[j]];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = com + i * 32 + (r >> 2) * 8 + (r & 3);
+            const float b = a.bias && row + half < a.cout ? a.bias[row + half] : 0.0f;
+            float v[2], u[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                v[j] = acc[i][j][r] + nz[j];
+                v[j] = activate(v[j] + b, ACT);
+                u[j] = __shfl_xor(v[j], 1, 64);
+            }
+            if (!whole || row + half >= a.cout) continue;
+            *reinterpret_cast<float *>(reinterpret_cast<char *>(out + (size_t)row * HP) + off) =
+                (((v[0] + u[0]) + v[1]) + u[1]) / 4.0f;
+        }
+}
+
+template <int ACT>
+__device__ __forceinline__ void store_outputs(const ConvArgs &a, int img, int com, const int (&oy)[2],
                                               const int (&ox)[2], const v16f (&acc)[2][2]) {
-    store_rows<ACT>(a, a.y + first, com, oy, ox, acc);
+    const size_t first = (size_t)img * a.cout * a.h * a.w_;
+    if (a.y) store_rows<ACT>(a, a.y + first, com, oy, ox, acc);
     if (a.tap) store_rows<ACT, true>(a, a.tap + first, com, oy, ox, acc);
+    if (a.pool) store_pooled<ACT>(a, img, com, oy, ox, acc);
 }
 
 __device__ __forceinline__ void store_tile(const ConvArgs &a, int img, int slice, int com, const int (&oy)[2],
                                            const int (&ox)[2], const v16f (&acc)[2][2]) {
     const size_t image = (size_t)a.cout * a.h * a.w_;
     if (a.part) store_rows<kPartial>(a, a.part + ((size_t)slice * a.n + img) * image, com, oy, ox, acc);
-    else if (a.act == SVBRDF_ACT_RELU) store_outputs<SVBRDF_ACT_RELU>(a, img * image, com, oy, ox, acc);
-    else if (a.act == SVBRDF_ACT_LRELU) store_outputs<SVBRDF_ACT_LRELU>(a, img * image, com, oy, ox, acc);
-    else store_outputs<SVBRDF_ACT_NONE>(a, img * image, com, oy, ox, acc);
+    else if (a.act == SVBRDF_ACT_RELU) store_outputs<SVBRDF_ACT_RELU>(a, img, com, oy, ox, acc);
+    else if (a.act == SVBRDF_ACT_LRELU) store_outputs<SVBRDF_ACT_LRELU>(a, img, com, oy, ox, acc);
+    else store_outputs<SVBRDF_ACT_NONE>(a, img, com, oy, ox, acc);
 }
 
 // A wave's 64 x 64 tile again on the fp32 instruction, from the fp32 inputs:
@@ -1032,6 +1068,31 @@ int svbrdf_conv3x3_split(const float *x, int n, int cin, int height, int width, 
     a.x = x; a.bias = bias; a.noise = noise; a.noise_strength = noise_strength; a.act = activation;
     a.y = y; a.n = n; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
     return run_split(what, a, split, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+// Where a tile holds whole 2 x 2 windows and all of K: 32 columns (images wider
+// than 16), unsplit. The layer before VGG's first pooling (9 x 64 x 256^2) then
+// writes its scaled copy and 38 MB of averages instead of 151 MB that a pooling
+// kernel reads again: 309 + 44 us -> 296; the second one 211 + 15 -> 214.
+int svbrdf_conv3x3_split_pools(int n, int cin, int height, int width, int cout) {
+    if (!svbrdf_conv3x3_split_preferred(n, cin, height, width, cout) || height < 2) return 0;
+    const SplitPlan p = plan_split(n, cin, height, width, cout);
+    return p.slices == 1 && p.tw == 32;
+}
+
+int svbrdf_conv3x3_pooled(const float *x, int n, int cin, int height, int width, const void *split, int cout,
+                          const float *bias, const float *noise, float noise_strength, int activation, float *y,
+                          float *tap, float tap_scale, float *pool, void *stream) {
+    const char *what = "svbrdf_conv3x3_pooled";
+    if (!x || !split || !pool) return fail(SVBRDF_EINVAL, "%s: null pointer argument", what);
+    if (!svbrdf_conv3x3_split_pools(n, cin, height, width, cout))
+        return fail(SVBRDF_ESHAPE, "%s: n=%d cin=%d cout=%d height=%d width=%d (svbrdf_conv3x3_split_pools)", what, n,
+                    cin, cout, height, width);
+    ConvArgs a{};
+    a.x = x; a.bias = bias; a.noise = noise; a.noise_strength = noise_strength; a.act = activation;
+    a.y = y; a.tap = tap; a.tap_scale = tap_scale; a.pool = pool;
+    a.n = n; a.cin = cin; a.cout = cout; a.h = height; a.w_ = width;
+    return run_split(what, a, split, nullptr, 0, (hipStream_t)stream);
 }
 
 int svbrdf_conv3x3_tapped(const float *x, int n, int cin, int height, int width, const float *packed,

@@ -242,22 +242,29 @@ class VGGLoss(torch.nn.Module):
     def normalize(self, im):
         return (im - self.mean) / self.std
 
-    def _features(self, x, vector=None):
+    def _features(self, x, vector=None, keep=True):
         """The hooked layers' outputs; with `vector` also their weighted
-        concatenation, which the convolutions write beside their outputs."""
-        feats, at = [], 0
-        for step in self.plan:
+        concatenation, which the convolutions write beside their outputs.  A
+        hooked layer that only the pooling behind it and `vector` read is not
+        written itself unless `keep` (its entry is then None)."""
+        feats, at, pooled = [], 0, False
+        for step, behind in zip(self.plan, [*self.plan[1:], None]):
             if step == "P":
-                x = convnet.avgpool2(x)
+                x = x if pooled else convnet.avgpool2(x)
+                pooled = False
                 continue
-            if vector is not None and step in self.HOOKS and len(feats) < len(self.weights):
+            hook, tap, scale = step in self.HOOKS, None, 1.0
+            if vector is not None and hook and len(feats) < len(self.weights):
                 size = x.shape[0] * self.convs[step].cout * x.shape[2] * x.shape[3]
-                x = self.convs[step](x, vector[at:at + size], self.weights[len(feats)])
+                tap, scale = vector[at:at + size], self.weights[len(feats)]
                 at += size
+            pooled = vector is not None and behind == "P"
+            if pooled:
+                x, y = self.convs[step].pooled(x, hook and keep, tap, scale)
             else:
-                x = self.convs[step](x)
-            if step in self.HOOKS:
-                feats.append(x.flatten())
+                x = y = self.convs[step](x) if tap is None else self.convs[step](x, tap, scale)
+            if hook:
+                feats.append(None if y is None else y.flatten())
         return feats
 
     def _vector(self, x):
@@ -275,7 +282,7 @@ class VGGLoss(torch.nn.Module):
         if not self.weights or (torch.is_grad_enabled() and x.requires_grad):
             return torch.cat([f * w for f, w in zip(self._features(x), self.weights)])
         vector = self._vector(x)
-        self._features(x, vector)
+        self._features(x, vector, keep=False)
         return vector
 
     def load(self, im):
