@@ -488,12 +488,21 @@ __device__ __forceinline__ void store_one(const ConvArgs &a, float acc, int co, 
 // chunk of 8 input channels the block stages the 66 x 10 input tiles (with
 // the one-pixel halo, zero outside the image; times the gate, when there is
 // one) in LDS with coalesced loads, and every thread reads its 4 x 3 window
-// per channel from there.  The weights of one input channel and tap are the
-// same for every thread: scalar loads.
+// per channel from there, the next chunk's loads in flight beside the products.
+// The weights of one input channel and tap are the same for every thread: up to
+// four output channels through LDS, as broadcasts (scalar loads return out of
+// order, so each channel waits for all of its own); above that scalar loads
+// again, 72 LDS weights a channel cost more than that wait (512 -> 8 at 32^2 415
+// against 329 us).  Bound by the latency of a chunk's round on small images, by
+// its bytes on large ones.  64 -> 3 at 9 x 256^2 90 -> 65 us (with the gate 115 ->
+// 108), at 1 x 256^2 43 -> 26; 64 -> 8 at 4 x 333^2 110 -> 98, gated 145 -> 108.
 template <int CO, bool GATE>
 __global__ __launch_bounds__(kThreads) void conv3x3_direct_kernel(ConvArgs a) {
     constexpr int TX = 64, TY = 8, HX = TX + 2, HY = TY + 2, CC = 8;
+    constexpr bool LDSW = CO <= 4;
+    constexpr int WP = (9 * CO + 3) / 4 * 4, WPER = (CC * 9 * CO + kThreads - 1) / kThreads;
     __shared__ float tile[CC][HY * HX];
+    __shared__ __attribute__((aligned(16))) float wl[LDSW ? CC : 1][WP];   // the chunk's weights, [tap][co] per channel
     const int H = a.h, W = a.w_;
     const int bx0 = blockIdx.x * TX, by0 = blockIdx.y * TY;
     const int tx = threadIdx.x & 63, ty = (threadIdx.x >> 6) * 2;   // column, first of the two rows
@@ -506,30 +515,54 @@ __global__ __launch_bounds__(kThreads) void conv3x3_direct_kernel(ConvArgs a) {
 #pragma unroll
     for (int co = 0; co < CO; ++co) acc0[co] = acc1[co] = 0.0f;
     constexpr int NE = CC * HY * HX, PER = (NE + kThreads - 1) / kThreads;
-    for (int c0 = 0; c0 < a.cin; c0 += CC) {
-        // every load of the chunk first (branch-free: a clamped address and a
-        // select), then the LDS stores
-        float xv[PER], gv[PER];
-        bool ok[PER];
+    // This thread's elements of a chunk: byte offsets from the chunk's first
+    // plane (32 bits reach 8 planes of at most 2^28), past every plane for an
+    // element outside the image.
+    unsigned off[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int e = threadIdx.x + k * kThreads;
+        const int cc = e / (HY * HX), rem = e - cc * (HY * HX);
+        const int r = rem / HX, c = rem - r * HX;
+        const int yy = by0 - 1 + r, xx = bx0 - 1 + c;
+        const bool in = e < NE && yy >= 0 && yy < H && xx >= 0 && xx < W;
+        off[k] = in ? ((unsigned)cc * (unsigned)HW + (unsigned)(yy * W + xx)) * 4u : ~0u;
+    }
+    float xv[PER], gv[PER], wv[WPER];
+    const auto load = [&](int c0) {
+#pragma unroll
+        for (int k = 0; LDSW && k < WPER; ++k) {
+            const int e = min((int)threadIdx.x + k * kThreads, CC * 9 * CO - 1), cc = e / (9 * CO), q = e - cc * 9 * CO;
+            wv[k] = a.w[(size_t)(q / CO) * tap_stride + (size_t)min(c0 + cc, a.cin - 1) * CO + q % CO];
+        }
+        // branch-free: a clamped address and a select
+        const unsigned end = (unsigned)min(CC, a.cin - c0) * (unsigned)HW * 4u;
+        const char *xc = reinterpret_cast<const char *>(xi + (size_t)c0 * HW);
+        const char *gc = GATE ? reinterpret_cast<const char *>(gi + (size_t)c0 * HW) : nullptr;
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            const int e = threadIdx.x + k * kThreads;
-            const int cc = e / (HY * HX), rem = e - cc * (HY * HX);
-            const int r = rem / HX, c = rem - r * HX;
-            const int ci = c0 + cc, yy = by0 - 1 + r, xx = bx0 - 1 + c;
-            ok[k] = e < NE && ci < a.cin && yy >= 0 && yy < H && xx >= 0 && xx < W;
-            const size_t o = ok[k] ? (size_t)ci * HW + (size_t)yy * W + xx : 0;
-            xv[k] = xi[o];
-            if constexpr (GATE) gv[k] = gi[o];
+            const unsigned o = off[k] < end ? off[k] : 0u;
+            xv[k] = *reinterpret_cast<const float *>(xc + o);
+            if constexpr (GATE) gv[k] = *reinterpret_cast<const float *>(gc + o);
         }
+    };
+    load(0);
+    for (int c0 = 0; c0 < a.cin; c0 += CC) {
+        const unsigned end = (unsigned)min(CC, a.cin - c0) * (unsigned)HW * 4u;
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             const int e = threadIdx.x + k * kThreads;
             float v = xv[k];
             if constexpr (GATE) v = v * (gv[k] > 0.0f ? a.gate_pos : a.gate_neg);
-            if (e < NE) (&tile[0][0])[e] = ok[k] ? v : 0.0f;
+            if (e < NE) (&tile[0][0])[e] = off[k] < end ? v : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; LDSW && k < WPER; ++k) {
+            const int e = threadIdx.x + k * kThreads, cc = e / (9 * CO);
+            if (e < CC * 9 * CO) wl[cc][e - cc * 9 * CO] = wv[k];
         }
         __syncthreads();
+        if (c0 + CC < a.cin) load(c0 + CC);   // in flight beside this chunk's products
         const int nc = min(CC, a.cin - c0);
         for (int cc = 0; cc < nc; ++cc) {
             float v[4][3];
@@ -542,9 +575,9 @@ __global__ __launch_bounds__(kThreads) void conv3x3_direct_kernel(ConvArgs a) {
             for (int t = 0; t < 9; ++t) {
 #pragma unroll
                 for (int co = 0; co < CO; ++co) {
-                    const float wv = wc[t * tap_stride + co];
-                    acc0[co] += v[t / 3][t % 3] * wv;
-                    acc1[co] += v[t / 3 + 1][t % 3] * wv;
+                    const float w = LDSW ? wl[cc][t * CO + co] : wc[t * tap_stride + co];
+                    acc0[co] += v[t / 3][t % 3] * w;
+                    acc1[co] += v[t / 3 + 1][t % 3] * w;
                 }
             }
         }
