@@ -421,25 +421,30 @@ __global__ __launch_bounds__(kThreads) void conv3x3_mfma_kernel(ConvArgs a) {
     // and column n = lane % 32 of that 32 x 32 tile.  A K slice stores its raw
     // partial sums instead.
     float *yi = a.part ? a.part + ((size_t)slice * a.n + img) * a.cout * HW : a.y + (size_t)img * a.cout * HW;
-    float *ti = a.tap && !a.part ? a.tap + (size_t)img * a.cout * HW : nullptr;
+    const auto store = [&](auto &&put) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int nn = wn * (BN / 2) + j * 32 + (lane & 31);
-        const int ty = nn / a.tw, tx = nn - ty * a.tw;
-        const int yy = y0 + ty, xx = x0 + tx;
-        if (yy >= H || xx >= W) continue;
-        const size_t p = (size_t)yy * W + xx;
+        for (int j = 0; j < TN; ++j) {
+            const int nn = wn * (BN / 2) + j * 32 + (lane & 31);
+            const int ty = nn / a.tw, tx = nn - ty * a.tw;
+            const int yy = y0 + ty, xx = x0 + tx;
+            if (yy >= H || xx >= W) continue;
+            const size_t p = (size_t)yy * W + xx;
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
+            for (int i = 0; i < TM; ++i) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int co = co0 + wm * (BM / 2) + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                if (co >= a.cout) continue;
-                const float v = a.part ? acc[i][j][r] : finish(a, acc[i][j][r], co, p);
-                yi[(size_t)co * HW + p] = v;
-                if (ti) ti[(size_t)co * HW + p] = v * a.tap_scale;
+                for (int r = 0; r < 16; ++r) {
+                    const int co = co0 + wm * (BM / 2) + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                    if (co >= a.cout) continue;
+                    put(acc[i][j][r], co, p);
+                }
             }
         }
+    };
+    store([&](float v, int co, size_t p) { yi[(size_t)co * HW + p] = a.part ? v : finish(a, v, co, p); });
+    // a pass of its own: tested beside every store it took 1 % of a small layer
+    if (a.tap && !a.part) {
+        float *ti = a.tap + (size_t)img * a.cout * HW;
+        store([&](float v, int co, size_t p) { ti[(size_t)co * HW + p] = finish(a, v, co, p) * a.tap_scale; });
     }
 }
 
