@@ -444,8 +444,11 @@ int svbrdf_conv3x3_input_grad(const float *grad_y, const float *y, int activatio
 /* The same convolutions (same epilogues, gate, results to fp32 rounding) on
  * the bf16 matrix cores: every fp32 input and weight enters as the exact sum of
  * three bf16 values and a product as its six leading bf16 products, accumulated
- * in fp32; the error against 64 bits is below the fp32 matrix instruction's,
- * and infinities and NaN spread as in svbrdf_conv3x3.  The weights are laid out
+ * in fp32; the error against 64 bits is below the fp32 matrix instruction's.
+ * Values that are no such sum (infinities, NaN, above 3.39e38, small ones with
+ * bits below 2^-126) and sums below 2^-100 take the fp32 instruction, so they
+ * count and spread as in svbrdf_conv3x3; a call that consists of them takes
+ * four to five times as long as there.  The weights are laid out
  * once in the matrix core's order: a 16-byte aligned buffer of
  * svbrdf_conv3x3_split_weights_bytes(cin, cout) bytes (cin and cout exchanged
  * for the input gradient's), written by svbrdf_conv3x3_pack_split (arguments

@@ -8,8 +8,8 @@
 // leave, 8 significant bits apiece, 24 in all.  A product is then
 //   x w = hh' + (hm' + mh') + (hl' + mm' + lh') + O(2^-25 |x w|),
 // six bf16 products that the matrix core multiplies exactly and accumulates
-// in fp32, at 1,970 / 6 = 328 TFLOP/s.  bf16 has fp32's exponent, so there is
-// no scaling and no range to check.
+// in fp32, at 1,970 / 6 = 328 TFLOP/s.  bf16 has fp32's exponent, so nothing is
+// scaled; what lies at either end of the range is taken apart (below).
 //
 // Precision.  The hh' products and the five small ones have accumulators of
 // their own, so the sum is rounded at its own size once per 16 products (the
@@ -26,10 +26,15 @@
 // gradient through the 13 layers of the generator was 3.1e-5 off; it is
 // 1.0e-6, and 1.4e-6 on the fp32 instruction.
 //
-// Infinities and NaN, and finite values that round to infinity in bf16
-// (above 3.39e38), do not split; a wave whose sums come out non-finite
-// repeats its tile from the fp32 inputs on the fp32 instruction
-// (redo_fp32), so they spread exactly as in conv.hip.
+// Values that do not split: infinities and NaN, finite values that round to
+// infinity in bf16 (above 3.39e38), and small ones (2^-102) whose last term
+// would leave bf16's normal range (exact down to 2^-110, 8 bits short at
+// 2^-118, lost at 2^-133).  Such an operand puts a NaN among its tile's, and a
+// wave whose sums come out NaN, infinite or themselves below 2^-100 repeats
+// its tile from the fp32 values on the fp32 instruction (redo_fp32), so they
+// count and spread exactly as in conv.hip.  The check costs 0.2 to 0.3 % of a
+// convolution and 1 % of a modulated layer's pass; one such pixel in 9 x 64 ->
+// 64 at 256^2 nothing to be seen, all of them 1,750 us (fp32 kernel 390-450).
 //
 // Kernels
 //   split_factor_kernel   the demodulation factor of each output channel.
@@ -71,7 +76,10 @@ __device__ __forceinline__ float bf_hi(unsigned p) { return __uint_as_float(p & 
 
 // h + m + l of two finite values, as packed bf16 pairs.  No contraction: the
 // value is the rounded product that a caller passes, not the product itself.
-__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l) {
+// True where a last term leaves bf16's normal range, so that it may be off: the
+// rest is a subnormal number there (a compare per value; 0 and every value of
+// 2^-102 or more have none).
+__device__ __forceinline__ bool split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l) {
 #pragma clang fp contract(off)
     h = __builtin_bit_cast(unsigned, v2bf{(__bf16)a, (__bf16)b});
     a -= bf_lo(h);
@@ -80,6 +88,8 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsign
     a -= bf_lo(m);
     b -= bf_hi(m);
     l = __builtin_bit_cast(unsigned, v2bf{(__bf16)a, (__bf16)b});
+    constexpr int kSubnormal = 0x90;
+    return __builtin_amdgcn_classf(a, kSubnormal) | __builtin_amdgcn_classf(b, kSubnormal);
 }
 
 // ---------------------------------------------------------------------------
@@ -118,6 +128,14 @@ __global__ __launch_bounds__(kThreads) void split_factor_kernel(const float *__r
     __syncthreads();
     if (threadIdx.x == 0) factor[blockIdx.x] = rsqrtf(((red[0] + red[1]) + red[2]) + red[3] + 1e-8f);
 }
+
+// Non-zero values below 2^-100 do not split: (bits << 1) - 1 orders magnitudes
+// as unsigned numbers, with zero above all.
+constexpr unsigned kTiny = (27u << 24) - 1u;
+__device__ __forceinline__ unsigned rank_of(float v) { return (__float_as_uint(v) << 1) - 1u; }
+// A NaN in both halves of a packed pair.  As a weight's first term it marks a
+// value that does not split: its other two then hold the fp32 bits.
+constexpr unsigned kMark = 0x7fffu, kMarkPair = 0x7fff7fffu;
 
 enum PackForm {
     kNatural,      // [M, K, 3, 3]
@@ -202,24 +220,16 @@ __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float *__res
                 else v[i] = tile[k * PITCH + mm * 9 + (8 - t)] * scale * by_m[mm] * by_k[k];
                 v[i] = chunk & 1 ? -v[i] : v[i];
             }
-            split_pair(v[0], v[1], h[j / 2], md[j / 2], l[j / 2]);
+            const bool tiny = split_pair(v[0], v[1], h[j / 2], md[j / 2], l[j / 2]);
+            const bool huge = (h[j / 2] & 0x7f80u) == 0x7f80u || (h[j / 2] & 0x7f800000u) == 0x7f800000u;
+            if (tiny || huge) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                // a value whose rounding is infinite: infinities and NaN keep
-                // h alone; a finite one takes the largest bf16 and its rest,
-                // so that h + m + l is the value itself for redo_fp32
-                const unsigned sh = i * 16, keep = 0xffff0000u >> sh;
-                if (((h[j / 2] >> sh) & 0x7f80u) != 0x7f80u) continue;
-                md[j / 2] &= keep;
-                l[j / 2] &= keep;
-                if (fabsf(v[i]) <= FLT_MAX) {
-                    const unsigned top = (__float_as_uint(v[i]) >> 16);   // towards zero: finite
-                    const float rest = v[i] - __uint_as_float(top << 16);
-                    const unsigned mid = __float_as_uint(rest) >> 16;
-                    const unsigned low = __float_as_uint(rest - __uint_as_float(mid << 16)) >> 16;
-                    h[j / 2] = (h[j / 2] & keep) | (top << sh);
-                    md[j / 2] |= mid << sh;
-                    l[j / 2] |= low << sh;
+                for (int i = 0; i < 2; ++i) {
+                    const unsigned sh = i * 16, keep = 0xffff0000u >> sh, bits = __float_as_uint(v[i]);
+                    if (((h[j / 2] >> sh) & 0x7f80u) != 0x7f80u && rank_of(v[i]) >= kTiny) continue;
+                    h[j / 2] = (h[j / 2] & keep) | (kMark << sh);
+                    md[j / 2] = (md[j / 2] & keep) | (bits >> 16 << sh);
+                    l[j / 2] = (l[j / 2] & keep) | ((bits & 0xffffu) << sh);
                 }
             }
         }
@@ -260,11 +270,11 @@ __device__ __forceinline__ float split_weight(const uint4 *w, int groups, int k_
     const int chunk = k / kKC, kk = k - chunk_base(chunk, k_total);
     const size_t base = ((size_t)(chunk * 9 + t) * 3 * groups + m / 32) * 64 + (m & 31) + 32 * (kk >> 3);
     const size_t step = (size_t)groups * 64;
-    float v[3];
+    unsigned v[3];
 #pragma unroll
-    for (int s = 0; s < 3; ++s)
-        v[s] = __uint_as_float((unsigned)reinterpret_cast<const unsigned short *>(w + base + s * step)[kk & 7] << 16);
-    const float x = v[0] + (v[1] + v[2]);
+    for (int s = 0; s < 3; ++s) v[s] = reinterpret_cast<const unsigned short *>(w + base + s * step)[kk & 7];
+    const float x = v[0] == kMark ? __uint_as_float(v[1] << 16 | v[2])
+                                  : bf_lo(v[0]) + (bf_lo(v[1]) + bf_lo(v[2]));
     return chunk & 1 ? -x : x;
 }
 
@@ -456,6 +466,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv3x3_split_kernel(SplitArgs s)
     auto store_item = [&](int k, int buf) {
         uint4 t[3];
         unsigned *h = &t[0].x, *m = &t[1].x, *l = &t[2].x;
+        bool tiny = false;
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
             float v[2];
@@ -465,8 +476,9 @@ __global__ __launch_bounds__(kThreads, 2) void conv3x3_split_kernel(SplitArgs s)
                 if constexpr (GATE) v[i] = v[i] * (open[k] >> (j + i) & 1 ? a.gate_pos : a.gate_neg);
                 v[i] = in[k] ? v[i] : 0.0f;
             }
-            split_pair(v[0], v[1], h[j / 2], m[j / 2], l[j / 2]);
+            tiny |= split_pair(v[0], v[1], h[j / 2], m[j / 2], l[j / 2]);
         }
+        t[0].x = tiny ? kMarkPair : t[0].x;
 #pragma unroll
         for (int i = 0; i < 3; ++i) tile[buf][i][dst[k]] = t[i];
     };
@@ -573,6 +585,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv3x3_split_kernel(SplitArgs s)
     run_chunk(c_end - 1, std::true_type{});
 
     bool bad = false;
+    unsigned least = ~0u;   // a sum below 2^-100 has low products that leave fp32's range
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -582,8 +595,9 @@ __global__ __launch_bounds__(kThreads, 2) void conv3x3_split_kernel(SplitArgs s)
                 acc[i][j][r] += low[i][j][r];
                 acc[i][j][r] = c_end & 1 ? acc[i][j][r] : -acc[i][j][r];
                 bad |= !(fabsf(acc[i][j][r]) <= FLT_MAX);
+                least = min(least, rank_of(acc[i][j][r]));
             }
-    if (__any(bad)) redo_fp32(s, img, slice, com, oy, ox, acc);
+    if (__any(bad || least < kTiny)) redo_fp32(s, img, slice, com, oy, ox, acc);
     store_tile(a, img, slice, com, oy, ox, acc);
 }
 
@@ -728,8 +742,11 @@ __global__ __launch_bounds__(kWgThreads) void conv3x3_wgrad_split_kernel(WgradSp
     };
     auto split_octet = [&](const float (&v)[8], uint4 (&t)[3]) {
         unsigned *h = &t[0].x, *m = &t[1].x, *l = &t[2].x;
+        bool tiny = false;
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) split_pair(v[j], v[j + 1], h[j / 2], m[j / 2], l[j / 2]);
+        for (int j = 0; j < 8; j += 2) tiny |= split_pair(v[j], v[j + 1], h[j / 2], m[j / 2], l[j / 2]);
+        // the first two pixels: every tap's octet holds one of them
+        t[0].x = tiny ? kMarkPair : t[0].x;
     };
     auto store_input = [&](const float (&v)[8], int yy) {
         const int slot = (yy + 1) & 3;
@@ -741,7 +758,7 @@ __global__ __launch_bounds__(kWgThreads) void conv3x3_wgrad_split_kernel(WgradSp
         } else if (has_edge) {
             // the last pixel of the octet before, the first of the one after
             unsigned t[3];
-            split_pair(e_side ? v[0] : 0.0f, e_side ? 0.0f : v[0], t[0], t[1], t[2]);
+            if (split_pair(e_side ? v[0] : 0.0f, e_side ? 0.0f : v[0], t[0], t[1], t[2])) t[0] = kMarkPair;
 #pragma unroll
             for (int k = 0; k < 3; ++k)
                 reinterpret_cast<unsigned *>(&xs[slot][k][e_side ? 1 + kWgOctets : 0][e_ch])[e_side ? 0 : 3] = t[k];
@@ -843,6 +860,7 @@ __global__ __launch_bounds__(kWgThreads) void conv3x3_wgrad_split_kernel(WgradSp
     }
     const bool flip = c_end > c_begin && negative(c_end - 1);
     bool bad = false;
+    unsigned least = ~0u;
 #pragma unroll
     for (int t = 0; t < 3; ++t)
 #pragma unroll
@@ -850,9 +868,10 @@ __global__ __launch_bounds__(kWgThreads) void conv3x3_wgrad_split_kernel(WgradSp
             acc[t][r] += low[t][r];
             acc[t][r] = flip ? -acc[t][r] : acc[t][r];
             bad |= !(fabsf(acc[t][r]) <= FLT_MAX);
+            least = min(least, rank_of(acc[t][r]));
         }
     const int ci = ci0 + nh * 32 + (lane & 31);
-    if (__any(bad)) redo_wgrad_fp32(a, c_begin, c_end, co0 + mh * 32 + (lane & 31), ci, dy, acc);
+    if (__any(bad || least < kTiny)) redo_wgrad_fp32(a, c_begin, c_end, co0 + mh * 32 + (lane & 31), ci, dy, acc);
     // through LDS: a row of the output is 64 x 9 consecutive values, a lane's are 9 apart
     __syncthreads();
 #pragma unroll
