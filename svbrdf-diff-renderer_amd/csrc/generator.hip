@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cstdint>
 
 #include "conv_common.hpp"
@@ -334,9 +335,31 @@ __global__ __launch_bounds__(256) void modconv_small_kernel(SmallArgs a) {
     }
 }
 
+// One output from the weights times the demodulation factor, as packed weights
+// give it.  Where the factor is far from 1 the sums above, which it multiplies
+// afterwards, can overflow or leave the normal range while the output does not;
+// one thread's serial loop, for those alone.
+__device__ float modulated_sum(const SmallArgs &a, int co, int p, float factor) {
+    const int P = a.h * a.w_, y0 = p / a.w_, x0 = p - y0 * a.w_;
+    float acc = 0.0f;
+#pragma unroll 1
+    for (int c = 0; c < a.cin; ++c) {
+        const float s = a.style ? a.style[c] : 1.0f;
+        const float *w = a.w + ((size_t)co * a.cin + c) * 9, *xc = a.x + (size_t)c * P;
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const int y = y0 + t / 3 - 1, x = x0 + t % 3 - 1;
+            const bool in = y >= 0 && y < a.h && x >= 0 && x < a.w_;
+            const float v = xc[in ? y * a.w_ + x : 0];
+            acc += w[t] * a.scale * s * factor * (in ? v : 0.0f);
+        }
+    }
+    return acc;
+}
+
 // c: the epilogue's arguments; c.part and squares as written above.
-__global__ __launch_bounds__(256) void modconv_small_sum_kernel(ConvArgs c, const float *__restrict__ squares,
-                                                                int demodulate) {
+__global__ __launch_bounds__(256) void modconv_small_sum_kernel(ConvArgs c, SmallArgs a, int demodulate) {
+    const float *__restrict__ squares = a.squares;
     const int P = c.h * c.w_, total = c.cout * P, e = blockIdx.x * 256 + threadIdx.x;
     if (e >= total) return;
     const int co = e / P;
@@ -357,7 +380,11 @@ __global__ __launch_bounds__(256) void modconv_small_sum_kernel(ConvArgs c, cons
             }
         }
     }
-    if (demodulate) v *= rsqrtf(sq + 1e-8f);
+    if (demodulate) {
+        const float factor = rsqrtf(sq + 1e-8f), size = fabsf(v);
+        const bool kept = size == 0.0f || (size >= 0x1p-100f && size <= FLT_MAX);
+        v = kept ? v * factor : modulated_sum(a, co, e - co * P, factor);
+    }
     c.y[e] = finish(c, v, co, e - co * P);
 }
 
@@ -458,8 +485,8 @@ int svbrdf_modconv3x3_small(const float *x, int cin, int height, int width, cons
     ConvArgs c{};
     c.bias = bias; c.noise = noise; c.noise_strength = noise_strength; c.act = activation;
     c.y = y; c.part = a.part; c.cout = cout; c.h = height; c.w_ = width; c.slices = p.slices;
-    hipLaunchKernelGGL(modconv_small_sum_kernel, dim3((unsigned)((cout * P + 255) / 256)), dim3(256), 0, s, c,
-                       (const float *)a.squares, demodulate);
+    hipLaunchKernelGGL(modconv_small_sum_kernel, dim3((unsigned)((cout * P + 255) / 256)), dim3(256), 0, s, c, a,
+                       demodulate);
     return check_launch(what);
 }
 
