@@ -387,6 +387,8 @@ class StyleLayersFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, latent, weights, biases, layers):
         x = latent.detach().contiguous()
+        if x.data_ptr() % 16:   # a view at an odd offset: the kernel reads 16 bytes at a time
+            x = x.clone()
         table = StyleLayersFunction._table(weights, biases, layers)
         out = torch.empty(int(table["rows"].sum()), dtype=torch.float32, device=x.device)
         _lib.call("svbrdf_style_layers", table.ctypes.data, len(weights), _lib.ptr(x), int(x.shape[1]),

@@ -199,13 +199,14 @@ class StyleGAN2Generator(torch.nn.Module):
         """Every layer's style (the convolutions', then the toRGB layers'), [1,
         rows] each, from one launch; None each, for the layers to compute
         their own, where the latent is not one float32 W+ on the GPU or a
-        layer's weights are being trained."""
+        layer's weights are being trained or not 16-byte aligned."""
         layers = [*self.convs, *self.to_rgb]
         weights, biases = [c.affine.weight for c in layers], [c.affine.bias for c in layers]
         if (wp.dim() != 3 or wp.shape[0] != 1 or wp.shape[1] < self.num_layers or wp.shape[2] != 512
                 or wp.dtype != torch.float32 or not wp.is_cuda
                 or any(t.requires_grad or t.device != wp.device or not t.is_contiguous() or t.dtype != torch.float32
-                       for t in [*weights, *biases, *(c.weight for c in layers)])):
+                       for t in [*weights, *biases, *(c.weight for c in layers)])
+                or any(t.data_ptr() % 16 for t in weights)):
             return [None] * len(layers)
         # convolution i reads latent row i, the toRGB layer behind it row i + 1
         last = self.num_layers - 1
