@@ -29,6 +29,15 @@ from . import _lib
 ACT = {"none": _lib.ACT_NONE, "relu": _lib.ACT_RELU, "lrelu": _lib.ACT_LRELU}
 
 
+def plain(module, kind):
+    """Whether calling module is kind.forward and nothing else: no subclass or
+    replacement of it and no hooks.  What passes a module's call by asks first."""
+    return (type(module) is kind and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks)
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
 def _check(t, name):
     if t.device.type != "cuda" or t.dtype != torch.float32:
         raise ValueError(f"{name} must be a float32 CUDA tensor (there is no CPU path), got {t.dtype} on {t.device}")

@@ -184,23 +184,32 @@ class StyleGAN2Generator(torch.nn.Module):
         # of the per-layer gradients, not a zero-filled copy per layer
         ws = wp.unbind(1)
         styles = self._styles(wp)
+        fused = styles[0] is not None
         for i, conv in enumerate(self.convs):
             # conv + noise_strength * noise + bias, leaky ReLU x sqrt(2), in one kernel
+            known = {"style": styles[i]} if fused else {}
             x = conv(x, ws[min(wi, self.num_layers - 1)], bias=self.bias[i], noise=noises[i],
-                     noise_strength=self.noise_strength_values[i], act="lrelu", style=styles[i])
+                     noise_strength=self.noise_strength_values[i], act="lrelu", **known)
             wi += 1
             if i == 0 or i % 2 == 0:
                 # toRGB after each resolution's last convolution, skip-summed
-                k = (i + 1) // 2
-                rgb = self.to_rgb[k](x, ws[min(wi, self.num_layers - 1)], style=styles[len(self.convs) + k], skip=rgb)
+                k, w = (i + 1) // 2, ws[min(wi, self.num_layers - 1)]
+                if fused:
+                    rgb = self.to_rgb[k](x, w, style=styles[len(self.convs) + k], skip=rgb)
+                else:
+                    t = self.to_rgb[k](x, w)
+                    rgb = t if rgb is None else convnet.upsample2(rgb) + t
         return rgb
 
     def _styles(self, wp):
         """Every layer's style (the convolutions', then the toRGB layers'), [1,
-        rows] each, from one launch; None each, for the layers to compute
-        their own, where the latent is not one float32 W+ on the GPU or a
-        layer's weights are being trained or not 16-byte aligned."""
+        rows] each, from one launch; None each, for the layers to compute their own
+        and their output alone, where the latent is not one float32 W+ on the
+        GPU, a layer's weights are being trained or not 16-byte aligned, or a
+        layer or its affine is not the one built here or has hooks."""
         layers = [*self.convs, *self.to_rgb]
+        if not all(convnet.plain(c, _ModConv) and convnet.plain(c.affine, _Dense) for c in layers):
+            return [None] * len(layers)
         weights, biases = [c.affine.weight for c in layers], [c.affine.bias for c in layers]
         if (wp.dim() != 3 or wp.shape[0] != 1 or wp.shape[1] < self.num_layers or wp.shape[2] != 512
                 or wp.dtype != torch.float32 or not wp.is_cuda
@@ -279,8 +288,12 @@ class VGGLoss(torch.nn.Module):
                 size += n * self.convs[step].cout * h * w
         return torch.empty(size, dtype=torch.float32, device=x.device)
 
+    def _writes_vector(self):
+        """Whether the layers can write the feature vector themselves."""
+        return bool(self.weights) and all(convnet.plain(c, convnet.Conv3x3) for c in self.convs)
+
     def compute_feature_vector(self, x):
-        if not self.weights or (torch.is_grad_enabled() and x.requires_grad):
+        if (torch.is_grad_enabled() and x.requires_grad) or not self._writes_vector():
             return torch.cat([f * w for f, w in zip(self._features(x), self.weights)])
         vector = self._vector(x)
         self._features(x, vector, keep=False)
@@ -289,8 +302,13 @@ class VGGLoss(torch.nn.Module):
     def load(self, im):
         with torch.no_grad():
             im = self.normalize(im)
-            self.im_feature = self._vector(im)
-            self._targets = self._features(im, self.im_feature)
+            if self._writes_vector():
+                self.im_feature = self._vector(im)
+                self._targets = self._features(im, self.im_feature)
+                return
+            feats = self._features(im)
+            self.im_feature = torch.cat([f * w for f, w in zip(feats, self.weights)])
+            self._targets = feats
 
     def forward(self, x):
         # mean((w_l f_l - w_l t_l)^2) over the concatenated vector, taken per
