@@ -80,11 +80,16 @@ def _split_buffer(cin, cout, device):
                        device=device)
 
 
-def _split_packed(packed, out=None):
+def _version(t):
+    """Counts the writes to a tensor (None in inference mode, which has no count)."""
+    return None if t.is_inference() else t._version
+
+
+def _split_packed(packed):
     """Split weights of a convolution from its packed ones ([9, Cin, Cout])."""
     _, cin, cout = (int(s) for s in packed.shape)
     packed = packed.contiguous()
-    out = _split_buffer(cin, cout, packed.device) if out is None else out
+    out = _split_buffer(cin, cout, packed.device)
     _lib.call("svbrdf_conv3x3_split_packed", _lib.ptr(packed), cin, cout, _lib.ptr(out),
               _lib.stream_handle(packed.device))
     return out
@@ -569,15 +574,41 @@ class Conv3x3(torch.nn.Module):
         self.act = act
         self.packed = pack3x3(self.weight)
         self.packed_t = pack3x3(self.weight, transpose=True)
-        # the layout of the bf16 matrix cores beside them, for the sizes that take that path
-        self.split = self.split_t = None
-        if min(self.cin, self.cout) >= 32:
-            # one buffer for both; their sizes are multiples of 64 floats but for the factors' room
-            sizes = [int(_lib.query("svbrdf_conv3x3_split_weights_bytes", *c)) // 256 * 64 + 64
-                     for c in ((self.cin, self.cout), (self.cout, self.cin))]
-            both = torch.empty(sum(sizes), dtype=torch.float32, device=self.weight.device)
-            self.split = _split_packed(self.packed, both[:sizes[0]])
-            self.split_t = _split_packed(self.packed_t, both[sizes[0]:])
+        self._splits = {name: (t, _version(t), _split_packed(t))
+                        for name, t in (("packed", self.packed), ("packed_t", self.packed_t))
+                        if min(self.cin, self.cout) >= 32}
+
+    _splits = {}   # of a layer that was saved without any
+
+    def _split(self, name):
+        """The layout of the bf16 matrix cores of self.packed or self.packed_t,
+        for the sizes that take that path; None below 32 channels on either
+        side.  Kept with the tensor it was made from, and made again once that
+        one has been replaced or written to."""
+        if min(self.cin, self.cout) < 32:
+            return None
+        packed = getattr(self, name)
+        source, seen, split = self._splits.get(name, (None, None, None))
+        if source is packed and seen == _version(packed):
+            return split
+        _check(packed, name)
+        shape = (9, self.cin, self.cout) if name == "packed" else (9, self.cout, self.cin)
+        if tuple(packed.shape) != shape:
+            raise ValueError(f"{name} {tuple(packed.shape)} is not {shape}")
+        split = _split_packed(packed)
+        if not torch.cuda.is_current_stream_capturing():
+            # whole before another stream can find it
+            torch.cuda.current_stream(packed.device).synchronize()
+            self._splits = {**self._splits, name: (packed, _version(packed), split)}
+        return split
+
+    @property
+    def split(self):
+        return self._split("packed")
+
+    @property
+    def split_t(self):
+        return self._split("packed_t")
 
     def forward(self, x, tap=None, tap_scale=1.0):
         """The layer; tap: a flat tensor that also receives tap_scale times
