@@ -456,9 +456,12 @@ int svbrdf_conv3x3_input_grad(const float *grad_y, const float *y, int activatio
  * svbrdf_conv3x3_split_packed (cin, cout: of the convolution that reads it).
  * svbrdf_conv3x3_split_preferred: whether this path is the faster one for a
  * shape (more than 8 output channels, at least 32 input channels, 2 GFLOP); it
- * takes any shape of at least 16 input channels.  Workspace:
+ * takes any shape of at least 16 input channels.
+ * svbrdf_conv3x3_split_packed_preferred: whether it still is where a call of
+ * svbrdf_conv3x3_split_packed is paid each time.  Workspace:
  * svbrdf_conv3x3_split_workspace_bytes, as svbrdf_conv3x3_workspace_bytes. */
 int svbrdf_conv3x3_split_preferred(int n, int cin, int height, int width, int cout);
+int svbrdf_conv3x3_split_packed_preferred(int n, int cin, int height, int width, int cout);
 size_t svbrdf_conv3x3_split_weights_bytes(int cin, int cout);
 int svbrdf_conv3x3_pack_split(const float *weight, int cout, int cin, const float *style, float scale, int demodulate,
                               int transpose, void *split, void *stream);

@@ -97,6 +97,7 @@ SIGNATURES = {
     "svbrdf_conv3x3_input_grad": (ctypes.c_int, [_vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                                  ctypes.c_int, _vp, ctypes.c_int, _vp, _vp, ctypes.c_size_t, _vp]),
     "svbrdf_conv3x3_split_preferred": (ctypes.c_int, [ctypes.c_int] * 5),
+    "svbrdf_conv3x3_split_packed_preferred": (ctypes.c_int, [ctypes.c_int] * 5),
     "svbrdf_conv3x3_split_weights_bytes": (ctypes.c_size_t, [ctypes.c_int] * 2),
     "svbrdf_conv3x3_pack_split": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, _vp, ctypes.c_float, ctypes.c_int,
                                                  ctypes.c_int, _vp, _vp]),

@@ -69,10 +69,12 @@ def pack3x3(weight, style=None, scale=1.0, demodulate=False, transpose=False):
     return out
 
 
-def _takes_split(n, cin, h, w, cout):
+def _takes_split(n, cin, h, w, cout, from_packed=False):
     """Whether a shape runs on the bf16 matrix cores with split operands
-    (fp32 results; csrc/conv_split.hip)."""
-    return bool(_lib.query("svbrdf_conv3x3_split_preferred", n, cin, h, w, cout))
+    (fp32 results; csrc/conv_split.hip); from_packed: where this call has to
+    split packed weights first."""
+    rule = "svbrdf_conv3x3_split_packed_preferred" if from_packed else "svbrdf_conv3x3_split_preferred"
+    return bool(_lib.query(rule, n, cin, h, w, cout))
 
 
 def _split_buffer(cin, cout, device):
@@ -116,7 +118,7 @@ def conv3x3_packed(x, packed, cout, bias=None, noise=None, noise_strength=0.0, a
     n, cin, h, w = (int(s) for s in x.shape)
     if tuple(packed.shape) != (9, cin, cout):
         raise ValueError(f"packed weights {tuple(packed.shape)} do not match Cin={cin}, Cout={cout}")
-    split = _split_packed(packed) if _takes_split(n, cin, h, w, cout) else None
+    split = _split_packed(packed) if _takes_split(n, cin, h, w, cout, from_packed=True) else None
     return _conv3x3(x, packed, split, cin, cout, bias, noise, noise_strength, act)
 
 
@@ -181,7 +183,7 @@ def conv3x3_input_grad(grad_y, y, packed_t, cin, act):
         raise ValueError(f"y {tuple(y.shape)} and grad_y {tuple(g.shape)} differ")
     if tuple(packed_t.shape) != (9, cout, cin):
         raise ValueError(f"packed weights {tuple(packed_t.shape)} do not match Cout={cout}, Cin={cin}")
-    split_t = _split_packed(packed_t) if _takes_split(n, cout, h, w, cin) else None
+    split_t = _split_packed(packed_t) if _takes_split(n, cout, h, w, cin, from_packed=True) else None
     return _input_grad(g, y, packed_t, split_t, cin, act)
 
 

@@ -1082,6 +1082,7 @@ struct ConvPlan {
     int bm, bn, tw, th, tiles_x, tiles_y, co_tiles;
     int slices, cps;
     size_t part_floats;   // workspace floats (0 without a K split)
+    double us;            // the estimate below
 };
 
 // Estimated time (us) of a tiling with `slices` K slices.  Blocks are dealt
@@ -1121,7 +1122,6 @@ ConvPlan plan_conv(int n, int cin, int h, int w, int cout) {
     const int n_chunks = (cin + kKC - 1) / kKC;
     const size_t out_bytes = (size_t)n * cout * h * w * sizeof(float);
     const int max_slices = std::max(1, std::min({kMaxSlices, n_chunks / kMinChunksPerSlice, 65535 / n}));
-    double best_t = 0.0;
     // 128-channel tiles only where there are that many channels; fewer slices
     // win ties (less workspace)
     for (int bm = 128; bm >= 64; bm -= 64) {
@@ -1139,11 +1139,8 @@ ConvPlan plan_conv(int n, int cin, int h, int w, int cout) {
                 p.cps = (n_chunks + s - 1) / s;
                 p.slices = (n_chunks + p.cps - 1) / p.cps;   // no empty slice
                 if (p.slices != s) continue;
-                const double t = estimate_us(p, n, out_bytes);
-                if (best.bm == 0 || t < 0.98 * best_t) {
-                    best = p;
-                    best_t = t;
-                }
+                p.us = estimate_us(p, n, out_bytes);
+                if (best.bm == 0 || p.us < 0.98 * best.us) best = p;
             }
         }
     }
@@ -1221,6 +1218,8 @@ void launch_split_sum(const ConvArgs &a, hipStream_t s) {
     if (vec) hipLaunchKernelGGL(conv_split_sum_kernel<4>, grid, dim3(kThreads), 0, s, a);
     else hipLaunchKernelGGL(conv_split_sum_kernel<1>, grid, dim3(kThreads), 0, s, a);
 }
+
+double conv_us(int n, int cin, int h, int w, int cout) { return plan_conv(n, cin, h, w, cout).us; }
 
 int run_conv(const char *what, ConvArgs a, void *workspace, size_t workspace_bytes, hipStream_t s) {
     if (!conv_shape_ok(a.n, a.cin, a.h, a.w_, a.cout))

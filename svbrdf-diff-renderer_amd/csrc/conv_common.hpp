@@ -74,6 +74,10 @@ __attribute__((visibility("hidden"))) void launch_split_sum(const ConvArgs &a, h
 __attribute__((visibility("hidden"))) int run_conv(const char *what, ConvArgs a, void *workspace,
                                                    size_t workspace_bytes, hipStream_t s);
 
+// Estimated time (us, without its launch) of a convolution on the fp32
+// instruction of more than kDirectMaxCout output and 4 input channels (conv.hip).
+__attribute__((visibility("hidden"))) double conv_us(int n, int cin, int h, int w, int cout);
+
 // Fills the epilogue-independent arguments of an input-gradient call (conv.hip).
 __attribute__((visibility("hidden"))) ConvArgs input_grad_args(const float *grad_y, const float *y, int activation,
                                                                int n, int cout, int height, int width, int cin,

@@ -892,6 +892,7 @@ __global__ __launch_bounds__(kWgThreads) void conv3x3_wgrad_split_kernel(WgradSp
 struct SplitPlan {
     int wm, wn, tw, th, tiles_x, tiles_y, co_tiles, slices, cps;
     size_t part_floats;
+    double us;   // the estimate below
 };
 
 // Estimated time (us), fitted to a sweep of (block tile, slices) over the layer
@@ -914,7 +915,6 @@ SplitPlan plan_split(int n, int cin, int h, int w, int cout) {
     const int n_chunks = chunks_of(cin);
     const size_t out_bytes = (size_t)n * cout * h * w * sizeof(float);
     const int max_slices = std::max(1, std::min({kMaxSlices, n_chunks, 65535 / n}));
-    double best_t = 0.0;
     for (int wm = 2; wm >= 1; --wm) {
         SplitPlan p{};
         p.wm = wm;
@@ -930,11 +930,8 @@ SplitPlan plan_split(int n, int cin, int h, int w, int cout) {
             p.cps = (n_chunks + s - 1) / s;
             p.slices = (n_chunks + p.cps - 1) / p.cps;
             if (p.slices != s) continue;
-            const double t = split_estimate_us(p, n, out_bytes);
-            if (best.wm == 0 || t < 0.98 * best_t) {
-                best = p;
-                best_t = t;
-            }
+            p.us = split_estimate_us(p, n, out_bytes);
+            if (best.wm == 0 || p.us < 0.98 * best.us) best = p;
         }
     }
     best.part_floats = best.slices > 1 ? (size_t)best.slices * n * cout * h * w : 0;
@@ -1025,6 +1022,22 @@ extern "C" {
 int svbrdf_conv3x3_split_preferred(int n, int cin, int height, int width, int cout) {
     if (!conv_shape_ok(n, cin, height, width, cout)) return 0;
     return cout > kDirectMaxCout && cin >= 32 && 18.0 * n * cin * cout * height * width >= 2.0e9;
+}
+
+// Where each call also splits the packed weights it is given: 90 bytes for
+// each pair of channels, 12 us a million pairs and 18 above three million (past
+// the caches), at least 3.7, and 3 for the launch. Layers of many channels on few pixels are mostly that pass
+// (fp32 / split with it, us: 4096 -> 4096 at 4^2 197 / 487, 2048 -> 2048 at 8^2
+// 61 / 124, 9 x 512 -> 512 at 8^2 42 / 45; 512 -> 512 at 22^2 46 / 38). Over 275
+// shapes of 32 to 4096 channels between 2 and 12 GFLOP this line takes one that
+// is slower by more than 2 % (256 -> 512 at 32^2, 35 / 37) and leaves 14 that
+// would be faster by more than 3 %, none of at most 512 channels.
+int svbrdf_conv3x3_split_packed_preferred(int n, int cin, int height, int width, int cout) {
+    if (!svbrdf_conv3x3_split_preferred(n, cin, height, width, cout)) return 0;
+    const double weights = (double)cin * cout;
+    const double pass = 3.0 + std::max(3.7, weights * (weights < 3.0e6 ? 1.2e-5 : 1.8e-5));
+    constexpr double kLaunch = 4.0;   // in split_estimate_us, not in conv_us
+    return plan_split(n, cin, height, width, cout).us + pass < conv_us(n, cin, height, width, cout) + kLaunch;
 }
 
 size_t svbrdf_conv3x3_split_weights_bytes(int cin, int cout) {
