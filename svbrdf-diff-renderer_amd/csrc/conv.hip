@@ -857,32 +857,33 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 }
 
 // Sum of the weight-gradient slices: eight running sums over the slices
-// s = j mod 8 (eight loads in flight per trip), then combined in a fixed
-// order -- the same bits on every run, and for either VEC (4 consecutive values
-// per thread where the count is a multiple of 4 and the tensors are aligned:
-// 4 slices of 512 x 512 x 9 take 8.8 us, 11.3 one value per thread).
-template <int VEC>
+// s = j mod 8 (eight loads in flight per trip, also in the last one), then
+// combined in a fixed order -- the same bits on every run.  Bound by latency: a
+// thread a value, so that few values with many slices still spread over the
+// chip.  Four values a thread were no faster for many values (512 x 512 x 9 in 4
+// slices, with the gradient's kernel: 48.8 us, 47.6 one by one) and slower for
+// few (64 x 64 x 9 in 256 slices: 72.5 and 49.9).
 __global__ __launch_bounds__(kThreads) void wgrad_sum_kernel(const float *__restrict__ part, int slices, size_t total,
                                                              float *__restrict__ out) {
-    typedef float vec __attribute__((ext_vector_type(VEC)));
-    const size_t e = ((size_t)blockIdx.x * kThreads + threadIdx.x) * VEC;
+    const size_t e = (size_t)blockIdx.x * kThreads + threadIdx.x;
     if (e >= total) return;
-    vec v[8];
+    float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = 0.0f;
-    for (int s = 0; s < slices; s += 8) {
-        vec q[8];
+    int s = 0;
+    for (; s + 8 <= slices; s += 8) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            // past the last slice: its own values again, not added
-            const int k = s + j < slices ? s + j : slices - 1;
-            q[j] = *reinterpret_cast<const vec *>(part + (size_t)k * total + e);
-        }
+        for (int j = 0; j < 8; ++j) v[j] += part[(size_t)(s + j) * total + e];
+    }
+    if (s < slices) {
+        float q[8];   // past the last slice: its own value again, not added
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = part[(size_t)min(s + j, slices - 1) * total + e];
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             if (s + j < slices) v[j] += q[j];
     }
-    *reinterpret_cast<vec *>(out + e) = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    out[e] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
 }
 
 // ---------------------------------------------------------------------------
@@ -1425,13 +1426,8 @@ int svbrdf_conv3x3_wgrad(const float *x, const float *grad_z, int n, int cin, in
     }
     if (slices > 1) {
         const size_t total = (size_t)9 * cin * cout;
-        const bool vec = total % 4 == 0 && (((uintptr_t)workspace | (uintptr_t)grad_w) & 15u) == 0;
-        const size_t threads = vec ? total / 4 : total;
-        const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
-        if (vec) hipLaunchKernelGGL(wgrad_sum_kernel<4>, grid, dim3(kThreads), 0, s, (const float *)workspace, slices,
-                                    total, grad_w);
-        else hipLaunchKernelGGL(wgrad_sum_kernel<1>, grid, dim3(kThreads), 0, s, (const float *)workspace, slices, total,
-                                grad_w);
+        const dim3 grid((unsigned)((total + kThreads - 1) / kThreads));
+        hipLaunchKernelGGL(wgrad_sum_kernel, grid, dim3(kThreads), 0, s, (const float *)workspace, slices, total, grad_w);
     }
     return check_launch(what);
 }
