@@ -25,6 +25,9 @@ from . import _lib
 
 LOSSES = {"l2": _lib.LOSS_L2, "log_l2": _lib.LOSS_LOG_L2, "logl2": _lib.LOSS_LOG_L2}
 
+# FusedStep.run: when a long run is worth a graph (sides in pixels, iterations)
+RECORD_RES, RECORD_AFTER, RECORD_STEPS = 512, 4000, 50
+
 # layout of svbrdf_step_state (include/svbrdf_hip.h)
 _STATE_DTYPE = np.dtype([("beta1_pow", "<f8"), ("beta2_pow", "<f8"),
                          ("inv_bias_correction1", "<f8"), ("inv_bias_correction2_sqrt", "<f4"),
@@ -169,16 +172,20 @@ class FusedStep:
         self.steps_launched = 0
         self.graph = None
         self.graph_steps = 0
+        self._record = None   # (key, graph, steps launched before it) of a long run
 
-    def _launch(self, stream, steps=1):
+    def _arguments(self):
+        """What svbrdf_fused_steps takes between the count and the stream."""
         r = self.renderer
         hist = self.history if self.history.numel() else None
-        _lib.call("svbrdf_fused_steps", steps, _lib.ptr(self.textures), _lib.ptr(self.exp_avg), _lib.ptr(self.exp_avg_sq),
-                  _lib.ptr(self.targets), self.res, self.texture_stride, self.plane_stride, self.n_views, r.size,
-                  _lib.ptr(r.camera_pos), _lib.ptr(r.light_pos), _lib.ptr(self.light_pow), self.mode,
-                  int(self.optim_light), self.lr, self.beta1, self.beta2, self.eps, _lib.ptr(self.state),
-                  _lib.ptr(hist), self.history.numel(), _lib.ptr(self.workspace), self.workspace.numel() * 4,
-                  stream)
+        return (_lib.ptr(self.textures), _lib.ptr(self.exp_avg), _lib.ptr(self.exp_avg_sq),
+                _lib.ptr(self.targets), self.res, self.texture_stride, self.plane_stride, self.n_views, r.size,
+                _lib.ptr(r.camera_pos), _lib.ptr(r.light_pos), _lib.ptr(self.light_pow), self.mode,
+                int(self.optim_light), self.lr, self.beta1, self.beta2, self.eps, _lib.ptr(self.state),
+                _lib.ptr(hist), self.history.numel(), _lib.ptr(self.workspace), self.workspace.numel() * 4)
+
+    def _launch(self, stream, steps=1):
+        _lib.call("svbrdf_fused_steps", steps, *self._arguments(), stream)
 
     def step(self):
         """Launch one fused iteration on the current stream (asynchronous)."""
@@ -196,10 +203,12 @@ class FusedStep:
         """n iterations, launched by the library's own loop `graph_steps` at a
         time (an interrupt is seen between two such calls); graph_steps=0
         launches them one by one from here.  The loop's launches stay ahead of
-        the GPU: per iteration it takes what a replayed graph of 100 takes (at
-        512^2 x 9 17.4 us each, at 256^2 8.5 and 8.3) and saves its recording
-        (0.3 ms for 10 iterations, 0.9 ms for 100) and the ~10-25 us by which
-        the GPU waits for a graph launch."""
+        the GPU and save a graph's recording (0.3 ms for 10 iterations, 0.9 ms
+        for 100); short steps stand 0.25 us closer in a replayed graph (256^2 x
+        9 8.21 us each, 8.47 in the loop; 64^2 7.46 and 7.72; none at 1024^2).
+        So at up to RECORD_RES pixels a side, pieces of graph_steps iterations
+        (RECORD_STEPS or more) are replayed once this object has launched
+        RECORD_AFTER, by when that has cost what the recording does."""
         if n <= 0:
             return
         if not graph_steps:
@@ -210,17 +219,35 @@ class FusedStep:
         per = max(1, int(graph_steps))
         for first in range(0, int(n), per):
             steps = min(per, int(n) - first)
-            self._launch(stream, steps)
+            graph = self._recorded(per) if steps == per >= RECORD_STEPS else None
+            if graph is not None:
+                graph.replay()
+            else:
+                self._launch(stream, steps)
             self.steps_launched += steps
 
-    def _capture_graph(self, steps):
+    def _recorded(self, steps):
+        """The graph of `steps` iterations of a long run, None while it has not
+        paid off or where the caller is recording.  It holds the launches of
+        _arguments() as they are now, and is dropped when one differs."""
+        if (self.res > RECORD_RES or self.steps_launched < RECORD_AFTER
+                or torch.cuda.is_current_stream_capturing()):
+            return None
+        key = (steps, *(getattr(a, "value", a) for a in self._arguments()))
+        if self._record is None or self._record[0] != key:
+            if self._record is not None and self.steps_launched < self._record[2] + RECORD_AFTER:
+                return None   # arguments that keep changing are not worth recording
+            self._record = (key, self._capture_graph(steps, "thread_local"), self.steps_launched)
+        return self._record[1]
+
+    def _capture_graph(self, steps, error_mode="global"):
         if steps < 1:
             raise ValueError("steps must be >= 1")
         g = torch.cuda.CUDAGraph()
         s = torch.cuda.Stream(device=self.textures.device)
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            g.capture_begin()
+            g.capture_begin(capture_error_mode=error_mode)
             self._launch(ctypes.c_void_p(s.cuda_stream), steps)
             g.capture_end()
         torch.cuda.current_stream().wait_stream(s)
