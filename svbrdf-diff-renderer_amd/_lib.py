@@ -163,7 +163,11 @@ def load():
         raise ImportError(f"{LIB_PATH} implements ABI {version}, these bindings need {ABI_VERSION}: rebuild it "
                           "with `python __graft_entry__.py build`")
     for name, (res, args) in SIGNATURES.items():
-        fn = getattr(lib, name)
+        fn = getattr(lib, name, None)
+        if fn is None:
+            # entry points are added within a version
+            raise ImportError(f"{LIB_PATH} is older than these bindings, it has no {name}: rebuild it with "
+                              "`python __graft_entry__.py build`")
         fn.restype = res
         fn.argtypes = args
     _lib = lib
