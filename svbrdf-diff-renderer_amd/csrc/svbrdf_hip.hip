@@ -871,12 +871,10 @@ __device__ __forceinline__ float4 *partial_buffer(void *ws, unsigned nb, unsigne
     return reinterpret_cast<float4 *>(static_cast<char *>(ws) + kCounterBytes + parity * stride);
 }
 
-// Fixed-order sum of n float4 partials (member .x, and .y .z .w when NQ == 4)
-// by one block of kBlock threads: thread i adds i, i + kBlock, ... in double,
-// then the wave and the block combine in index order.  Every reader of a
-// step's partials (the next step's block 0, the flush, the light finalize)
-// uses this routine, so they agree to the bit.  Result valid in thread 0.
-// wave_sums leaves the waves' sums in LDS, behind a barrier.
+// Fixed-order sums of n float4 partials (member .x, and .y .z .w when NQ == 4)
+// by one block: thread i adds i, i + BLOCK, ... in double, then the wave
+// combines.  Leaves the waves' sums in LDS, behind a barrier, for the caller to
+// add in index order.
 template <int NQ, int BLOCK>
 __device__ void wave_sums(const float4 *__restrict__ parts, unsigned n, double (*lds)[BLOCK / 64]) {
     double acc[NQ];
@@ -907,17 +905,17 @@ __device__ void wave_sums(const float4 *__restrict__ parts, unsigned n, double (
     __syncthreads();
 }
 
-template <int NQ, int BLOCK = kBlock>
-__device__ void reduce_partials(const float4 *__restrict__ parts, unsigned n, double (&tot)[NQ],
-                                double (*lds)[BLOCK / 64]) {
-    wave_sums<NQ, BLOCK>(parts, n, lds);
-#pragma unroll
-    for (int c = 0; c < NQ; ++c) {
-        tot[c] = 0.0;
-        if (threadIdx.x == 0)
-            for (int w = 0; w < BLOCK / 64; ++w) tot[c] += lds[c][w];
-    }
+// The loss's sum by a block of kBlock threads.  Both readers of a step's pending
+// loss (the next step's block 0 and the flush) use this routine, so they agree
+// to the bit; a light-optimising step has none pending, its finalize sums all
+// four in an order of its own.  Result valid in thread 0.
+__device__ double reduce_partials(const float4 *__restrict__ parts, unsigned n, double (*lds)[kBlock / 64]) {
+    wave_sums<1, kBlock>(parts, n, lds);
+    double total = 0.0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < kBlock / 64; ++w) total += lds[0][w];
     __syncthreads();
+    return total;
 }
 
 // Records the loss of step t (1-based) from its partials: state->loss and
@@ -966,9 +964,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SVBRDF_F
     const unsigned t = (unsigned)step_f;
     if (blockIdx.x == 0 && t >= 1 && st->pending_step == t) {
         __shared__ double ldsd[1][kBlock / 64];
-        double tot[1];
-        reduce_partials<1>(partial_buffer(ws, gridDim.x, (t - 1) & 1u), gridDim.x, tot, ldsd);
-        if (threadIdx.x == 0) record_loss(st, t, tot[0], count, loss_history, history_len);
+        const double total = reduce_partials(partial_buffer(ws, gridDim.x, (t - 1) & 1u), gridDim.x, ldsd);
+        if (threadIdx.x == 0) record_loss(st, t, total, count, loss_history, history_len);
     }
     const float P[3] = {lpow[0], lpow[1], lpow[2]};
     Pix px[NPIX];
@@ -1003,7 +1000,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SVBRDF_F
 }
 
 // One block, after a light-optimising step: reduces that step's partials in
-// the fixed order of reduce_partials, records the loss, takes the light-power
+// a fixed order (wave_sums at this block's size), records the loss, takes the light-power
 // Adam step (one param group with the maps, src/svbrdf.py:50) and advances
 // the state.  The next step needs the new light power in every block, so this
 // sits between two step launches and its latency counts.  At most
@@ -1061,10 +1058,10 @@ __global__ __launch_bounds__(kBlock) void flush_step_kernel(const void *ws, unsi
     __shared__ double lds[1][kBlock / 64];
     const unsigned t = (unsigned)st->step;
     if (t == 0 || st->pending_step != t) return;
-    double tot[1];
-    reduce_partials<1>(partial_buffer(const_cast<void *>(ws), n_partials, (t - 1) & 1u), n_partials, tot, lds);
+    const double total = reduce_partials(partial_buffer(const_cast<void *>(ws), n_partials, (t - 1) & 1u), n_partials,
+                                         lds);
     if (threadIdx.x != 0) return;
-    record_loss(st, t, tot[0], count, loss_history, history_len);
+    record_loss(st, t, total, count, loss_history, history_len);
     st->pending_step = 0u;
 }
 
