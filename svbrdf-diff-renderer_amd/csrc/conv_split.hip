@@ -252,10 +252,11 @@ __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float *__res
 // issued before this chunk's 9 x 24 MFMAs and split into the other LDS buffer
 // beside the last taps' MFMAs, so a block has one short barrier per chunk.
 //
-// Bound by the matrix cores, and those by power: 63 % busy at 1.94 GHz (peak
-// 2.4), where all-register MFMAs reach 1.88.  9 x 64 -> 64 at 256^2: 224 us =
-// 194 TFLOP/s of fp32 products (fp32 instruction 387 us), 256 -> 128 at 256^2:
-// 170 us, 227 TFLOP/s (333 us).  Splitting after the MFMAs instead of beside
+// Bound by the matrix cores, and those by power: 55 to 65 % busy at 1.96 to 2.05
+// GHz (peak 2.4), where all-register MFMAs reach 1.88.  9 x 64 -> 64 at 256^2
+// with inputs behind a ReLU: 230 us = 189 TFLOP/s of fp32 products (fp32
+// instruction 387 us), 256 -> 128 at 256^2: 172 us, 224 TFLOP/s (333 us); inputs
+// without zeros draw more power, 265-300 us for the first.  Splitting after the MFMAs instead of beside
 // them: 249 and 189 us; weights loaded where they are used: 310 and 234 us.
 // Three waves per SIMD (168 registers) gain nothing: 227 and 179 us.
 constexpr int halo_pixels(int wn) { return wn == 4 ? 340 : 204; }   // largest (th + 2)(tw + 2), see plan
@@ -616,7 +617,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv3x3_split_kernel(SplitArgs s)
 // change sign every second chunk, for the reason given above.
 // The sums leave through LDS: a lane's are 9 floats apart in the output.
 //
-// Matrix cores 41 % busy at 2.1 GHz; what is left is the operand reads behind
+// Matrix cores 43 to 46 % busy at 2.2 GHz; what is left is the operand reads behind
 // each chunk's barrier.  512 x 512 at 64^2: 122 us with the sum of 4 slices (159
 // TFLOP/s; the fp32 kernel 223), 256 -> 128 at 256^2 222 (408).  Re-reading all
 // three input rows for every chunk took 155 and 265, stores straight from the
